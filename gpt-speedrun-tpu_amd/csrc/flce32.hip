@@ -2,136 +2,420 @@
 // rig/kernels/linear_cross_entropy.py:38-41): the same algorithm as the bf16
 // kernels of flce.hip -- tiled logits with a per-tile (max, sum exp) in the
 // forward, the logits recomputed one vocabulary chunk at a time in the
-// backward -- with every product and sum in float32, as the reference's
+// backward -- with float32 operands, products and sums, as the reference's
 // einsums with compute_dtype float32 (`_tile_logits`, :92-112; the backward,
 // :220-302).  The [n, vocab] logits never exist; the backward's working set is
 // one float32 [n, chunk] logit gradient, the reference's own [n,
-// vocab_tile_size] bound.
+// vocab_tile_size] bound, plus partial sums of at most the same size each for
+// the two gradient products (below).
 //
-// Everything runs on one float32 GEMM tile kernel (64 x 64 outputs per
-// 256-thread workgroup, k in steps of 16 through LDS, 4 x 4 outputs per
-// thread, the vector ALU's fused multiply-add) with four epilogues.  The
-// bf16 path carries the training step; this one serves the API's float32
-// mode and its tests, so it favours plain code over peak rate.
-#include "common.h"
+// Float32 products on the bf16 matrix cores: every float32 operand element is
+// split exactly into three bf16 pieces (x = hi + mid + lo, 8 significant bits
+// each, by truncation), and a product keeps the six terms of weight 2^-16 and
+// above (lo*hi, hi*lo, mid*mid, mid*hi, hi*mid, hi*hi, added smallest first in
+// the MFMA's float32 accumulator).  What is dropped is below 2^-22 of a
+// product, less than the rounding of a float32 sum of a few products.
+// Relative error of dh and dW against 64 bits at 2048 tokens, d 512, V 50304:
+// 2.8e-7, against 8.1e-7 for one float32 multiply-add chain per output on the
+// vector ALU (fewer roundings of the running sum); at every size tried (1..2048
+// tokens, d 1..768, V 1..50304) no larger than that chain's.
+// A bf16 MFMA has 16 times the float32 MFMA's rate, so six of them are 2.7
+// times cheaper than one float32 MFMA and 5 times cheaper than the vector
+// ALU's multiply-adds.
+//
+// Tile kernel: 128 x 128 outputs per 256-thread workgroup, four waves of 64 x
+// 64 (2 x 2 blocks of v_mfma_f32_32x32x16_bf16), k in stages of 16.  A stage's
+// float32 elements go global -> registers one stage ahead, are split there and
+// written as three bf16 planes per operand into a double-buffered LDS stage
+// (24 KB): splitting on the way costs 5.5 vector operations per element, far
+// below the 24 MFMAs per wave and stage, and needs neither a pre-pass over the
+// weight nor a buffer for its planes.  ~50 KB of LDS and under 170 registers
+// let three workgroups share a CU, so one's loads, splits and epilogue run
+// under another's MFMAs.
+// Measured at 2048 tokens, d 512, V 50304, chunk 2048, against 64 x 64 vector-
+// ALU tiles: logits 592 us (178 TFLOP/s, 1.07 PFLOP/s of MFMA) against 1430,
+// forward + backward 2.83 ms against 23.0.  What bounds it now: the chunk's
+// launches (37 us logit gradient, 55 us the two products, 25 chunks) hold one or
+// two workgroups per CU at this size, so a stage's serial parts (fragment reads,
+// 24 MFMAs, split, barrier) overlap only partly.
+#include "gemm_core.h"
 
 #include <math.h>
 
 namespace {
 
-constexpr int kT = 64;   // tile edge
-constexpr int kK = 16;   // k per LDS stage
+constexpr int kT = 128;      // tile edge
+constexpr int kK = 16;       // k per LDS stage
+constexpr int kThreads = 256;
+constexpr int kPlane = kT * kK;          // bf16 elements of one plane of one operand
+constexpr int kStage = 6 * kPlane;       // A's three planes, then B's
+constexpr int kChunkRows = 64;           // granularity of the vocabulary chunk
 
-// Element (r, c) at p[r * rs + c * cs]; one of the strides is 1.
+using gemm::lds_t;
+using gemm::lds_x8;
+
+__shared__ __attribute__((aligned(1024))) bf16 s32_stage0[kStage];
+__shared__ __attribute__((aligned(1024))) bf16 s32_stage1[kStage];
+
+// Operand X(mn, k): element (mn, k) at p[mn * ld + k] (K-major) or
+// p[k * ld + mn] (MN-major); extents: mn < mn_end, k < k_end.
 struct Mat {
   const float* p;
-  int64_t rs, cs;
-};
-
-enum { kStats = 0, kGrad = 1, kStore = 2, kAccum = 3 };
-
-struct Epi32 {
-  float* out;         // kGrad: G [M][ld]; kStore / kAccum: C [M][ld]
   int64_t ld;
-  float2* partial;    // kStats: [column tile][M] = (max, sum exp(logit - max)), natural units
-  int col0;           // vocabulary row of output column 0 (masks, targets)
-  int sem_v;          // vocabulary rows >= sem_v are not classes
-  const int32_t* targets;
-  const float* lse;
-  const float* cot;   // per-row cotangent (nullable: cot_scale for every row)
-  float cot_scale;
 };
 
-template <int kEpi>
-__global__ void __launch_bounds__(256) gemm32_kernel(Mat A, Mat B, int M, int N, int K, Epi32 e) {
-  __shared__ float As[kK][kT + 4], Bs[kK][kT + 4];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int m0 = blockIdx.x * kT, n0 = blockIdx.y * kT;
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-  const bool a_k_inner = A.cs == 1, b_k_inner = B.rs == 1;
-  for (int k0 = 0; k0 < K; k0 += kK) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int idx = tid + 256 * r;
-      // Consecutive threads walk the unit-stride dimension.
-      const int mm = a_k_inner ? idx >> 4 : idx & 63, ka = a_k_inner ? idx & 15 : idx >> 6;
-      const int nn = b_k_inner ? idx >> 4 : idx & 63, kb = b_k_inner ? idx & 15 : idx >> 6;
-      const int m = m0 + mm, n = n0 + nn, k1 = k0 + ka, k2 = k0 + kb;
-      As[ka][mm] = (m < M && k1 < K) ? A.p[m * A.rs + k1 * A.cs] : 0.f;
-      Bs[kb][nn] = (n < N && k2 < K) ? B.p[k2 * B.rs + n * B.cs] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < kK; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[i] = As[kk][4 * ty + i];
-        b[i] = Bs[kk][4 * tx + i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
+// Where the 16-byte half `c` (8 values) of an operand plane's row sits.
+// K-major plane: 128 rows (mn) of 16 k, 32 bytes each; the half is swapped in
+// every other group of 8 rows, so the 16 rows a quarter-wave reads at one half
+// cover all 64 banks.
+__device__ __forceinline__ int kpos(int row, int c) { return row * 16 + 8 * (c ^ ((row >> 3) & 1)); }
+// MN-major plane: 8 blocks of 16 k-rows x 16 mn, 32 bytes per k-row.  Row k of
+// block b sits at k ^ f(b), f(b) = (b & 1) << 2 | (b >> 1): the 8 blocks one
+// k-row spans (a write) then cover all banks, and so do the two neighbouring
+// blocks of a transposed read.
+__device__ __forceinline__ int mpos(int b, int k) { return b * 256 + (k ^ (((b & 1) << 2) | ((b >> 1) & 3))) * 16; }
 
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + 4 * ty + i;
-    if constexpr (kEpi == kStats) {
-      // Row statistics over the tile's 64 columns: the 16 threads of a row
-      // group are lanes 16 q .. 16 q + 15 of one wave.
-      float y[4], mx = -INFINITY;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int v = e.col0 + n0 + 4 * tx + j;
-        y[j] = (n0 + 4 * tx + j < N && v < e.sem_v) ? acc[i][j] : -INFINITY;
-        mx = fmaxf(mx, y[j]);
-      }
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-      float s = 0.f;
-      if (mx != -INFINITY) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s += expf(y[j] - mx);
-      }
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o);
-      if (tx == 0 && m < M) e.partial[(size_t)blockIdx.y * M + m] = make_float2(mx, s);
+// One thread's 8 consecutive elements of a stage: K-major, row tid / 2 and k
+// 8 (tid % 2) ..; MN-major, k-row tid / 16 and mn 8 (tid % 16) ... kVec: 16-byte
+// loads (base, ld and the contiguous extent multiples of 4 elements).
+template <bool KMAJOR, bool kVec>
+struct Loader {
+  const float* p;    // this thread's first element at the tile's first stage
+  const float* safe; // a readable address for masked-out loads
+  int64_t step;      // elements per stage
+  int inner;         // contiguous elements left from this thread's first one (K-major: shrinks by stage)
+  int outer;         // K-major: row inside the extent (> 0); MN-major: k-rows left
+  f32x4 lo, hi;
+
+  __device__ __forceinline__ void init(Mat m, int mn0, int k0, int mn_end, int k_end, int tid) {
+    safe = m.p;
+    if (KMAJOR) {
+      const int row = mn0 + (tid >> 1), k = k0 + 8 * (tid & 1);
+      p = m.p + (int64_t)row * m.ld + k;
+      inner = k_end - k;
+      outer = mn_end - row;
+      step = kK;
     } else {
-      if (m >= M) continue;
-      float ct = 0.f, l = 0.f;
-      int t = -1;
-      if constexpr (kEpi == kGrad) {
-        t = e.targets[m];
-        const bool valid = t >= 0 && t < e.sem_v;
-        ct = valid ? (e.cot ? e.cot[m] : e.cot_scale) : 0.f;
-        l = e.lse[m];
-      }
+      const int k = k0 + (tid >> 4), mn = mn0 + 8 * (tid & 15);
+      p = m.p + (int64_t)k * m.ld + mn;
+      inner = mn_end - mn;
+      outer = k_end - k;
+      step = (int64_t)kK * m.ld;
+    }
+  }
+  // Elements past an extent come from `safe` and are replaced by zeros when split.
+  __device__ __forceinline__ void load(int kt) {
+    const float* q = p + kt * step;
+    const int in = KMAJOR ? inner - kK * kt : inner;
+    const bool ok = KMAJOR ? outer > 0 : outer > kK * kt;
+    if constexpr (kVec) {
+      lo = *reinterpret_cast<const f32x4*>(ok && in > 0 ? q : safe);
+      hi = *reinterpret_cast<const f32x4*>(ok && in > 4 ? q + 4 : safe);
+    } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int n = n0 + 4 * tx + j;
-        if (n >= N) continue;
-        float* dst = e.out + (int64_t)m * e.ld + n;
-        if constexpr (kEpi == kGrad) {
-          const int v = e.col0 + n;
-          // (exp(logit - lse) - [v == t]) * ct, zero for non-class rows
-          // (linear_cross_entropy.py:255-266).
-          *dst = v < e.sem_v ? (expf(acc[i][j] - l) - (v == t ? 1.f : 0.f)) * ct : 0.f;
-        } else if constexpr (kEpi == kStore) {
-          *dst = acc[i][j];
-        } else {
-          *dst += acc[i][j];
-        }
+        lo[j] = *(ok && in > j ? q + j : safe);
+        hi[j] = *(ok && in > 4 + j ? q + 4 + j : safe);
       }
     }
   }
+  // Split the loaded stage kt and write its planes (plane q at dst + q * kPlane).
+  __device__ __forceinline__ void store(lds_t* dst, int kt, int tid) const {
+    const int in = KMAJOR ? inner - kK * kt : inner;
+    const bool ok = KMAJOR ? outer > 0 : outer > kK * kt;
+    uint32_t w[3][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t piece[3][2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int i = 2 * j + u;
+        const float raw = i < 4 ? lo[i] : hi[i - 4];
+        const float x = ok && in > (kVec ? i & 4 : i) ? raw : 0.f;
+        const uint32_t b0 = __builtin_bit_cast(uint32_t, x);
+        const float r1 = x - __builtin_bit_cast(float, b0 & 0xFFFF0000u);   // exact
+        const uint32_t b1 = __builtin_bit_cast(uint32_t, r1);
+        const float r2 = r1 - __builtin_bit_cast(float, b1 & 0xFFFF0000u);  // exact, 8 bits
+        piece[0][u] = b0;
+        piece[1][u] = b1;
+        piece[2][u] = __builtin_bit_cast(uint32_t, r2);
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q)  // the upper halves of the two words
+        w[q][j] = __builtin_amdgcn_perm(piece[q][1], piece[q][0], 0x07060302u);
+    }
+    const int pos = KMAJOR ? kpos(tid >> 1, tid & 1) : mpos((tid & 15) >> 1, tid >> 4) + 8 * (tid & 1);
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      *(lds_x8*)(dst + q * kPlane + pos) = __builtin_bit_cast(bf16x8, u32x4{w[q][0], w[q][1], w[q][2], w[q][3]});
+  }
+};
+
+// MFMA operand (8 k of this lane's half) of rows / columns r0 + lane % 32 of a plane.
+template <bool KMAJOR>
+__device__ __forceinline__ bf16x8 frag32(const lds_t* plane, int r0, int lane) {
+  if (KMAJOR) return *(const lds_x8*)(plane + kpos(r0 + (lane & 31), lane >> 5));
+  // Transposed read: lane 4j + q of a 16-lane group supplies row k0 + j,
+  // columns 4q .. +3 of its block and receives rows k0 .. k0 + 3 of one column.
+  const int c = lane & 15, b = (r0 >> 4) + ((lane >> 4) & 1), k = 8 * (lane >> 5) + (c >> 2);
+  const bf16x4 lo = gemm::read_tr(plane + mpos(b, k) + 4 * (c & 3));
+  const bf16x4 hi = gemm::read_tr(plane + mpos(b, k + 4) + 4 * (c & 3));
+  return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+
+template <bool AK, bool BKM>
+__device__ __forceinline__ void mma_stage32(f32x16 (&acc)[2][2], const lds_t* st, int wm0, int wn0, int lane) {
+  bf16x8 a[2][3], b[2][3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      a[i][q] = frag32<AK>(st + q * kPlane, wm0 + 32 * i, lane);
+      b[i][q] = frag32<BKM>(st + (3 + q) * kPlane, wn0 + 32 * i, lane);
+    }
+  // Smallest terms first; the four accumulators alternate, so no MFMA waits
+  // for the one before it.
+  constexpr int kTerm[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+  for (int t = 0; t < 6; ++t)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(a[i][kTerm[t][0]], b[j][kTerm[t][1]], acc[i][j]);
+}
+
+// acc[i][j][r] = C[m0 + wm0 + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4][n0 + wn0 + 32 j + lane % 32],
+// wm0 = 64 (wave % 2), wn0 = 64 (wave / 2), over k in [k0, k_end).  Ends on a barrier:
+// the stage arrays may be reused.
+template <bool AK, bool BKM, bool kVec>
+__device__ __forceinline__ void tile32(f32x16 (&acc)[2][2], Mat A, Mat B, int m_end, int n_end, int k0, int k_end,
+                                       int m0, int n0) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm0 = 64 * (wave & 1), wn0 = 64 * (wave >> 1);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+  lds_t* const st0 = gemm::lds_cast(s32_stage0);
+  lds_t* const st1 = gemm::lds_cast(s32_stage1);
+  Loader<AK, kVec> la;
+  Loader<BKM, kVec> lb;
+  la.init(A, m0, k0, m_end, k_end, tid);
+  lb.init(B, n0, k0, n_end, k_end, tid);
+  const int nk = (k_end - k0 + kK - 1) / kK;
+  la.load(0);
+  lb.load(0);
+  la.store(st0, 0, tid);
+  lb.store(st0 + 3 * kPlane, 0, tid);
+  la.load(1);
+  lb.load(1);
+  __syncthreads();
+  // Stage kt + 1 (already in registers) is written into the other buffer, whose
+  // readers passed the last barrier, while stage kt is multiplied.
+  auto step = [&](const lds_t* cur, lds_t* nxt, int kt) __attribute__((always_inline)) {
+    mma_stage32<AK, BKM>(acc, cur, wm0, wn0, lane);
+    la.store(nxt, kt + 1, tid);
+    lb.store(nxt + 3 * kPlane, kt + 1, tid);
+    la.load(kt + 2);
+    lb.load(kt + 2);
+    GPTRIG_WAIT_LGKM0();  // this wave's LDS writes (the global loads stay in flight)
+    wg_barrier();
+  };
+  for (int kt = 0; kt < nk; kt += 2) {
+    step(st0, st1, kt);
+    if (kt + 1 < nk) step(st1, st0, kt + 1);
+  }
+}
+
+// Bytes of the rows of a tile that exist (at most kT of `ld` floats), and a
+// lane offset past any of them even with a row's offset added: such accesses
+// read zeros or are dropped.
+constexpr uint32_t kOff32Drop = 0x80000000u;
+__device__ __forceinline__ uint32_t row_bytes32(int rows, int ld) {
+  return 4u * (uint32_t)((rows < kT ? rows : kT) * ld);
+}
+
+// Workgroup -> (row tile, column tile) with the column tile fastest inside one
+// XCD's contiguous share, so the workgroups that run together on an XCD share
+// rows of A.
+__device__ __forceinline__ void tile_of(int pid, int total, int col_tiles, int& tr, int& tc) {
+  const int id = gemm::xcd_swizzle(pid, total);
+  tr = id / col_tiles;
+  tc = id % col_tiles;
+}
+
+// Logits of 128 vocabulary rows x 128 tokens (rows = vocabulary) and their
+// per-token (max, sum exp(logit - max)) over the tile's classes.
+template <bool kVec>
+__global__ void __launch_bounds__(kThreads, 3)
+    stats32_kernel(const float* __restrict__ w, const float* __restrict__ h, int V, int N, int D, int sem_v,
+                   float2* __restrict__ partial) {
+  __shared__ float2 half_s[kT];
+  const int tok_tiles = (N + kT - 1) / kT;
+  int tv, tn;
+  tile_of(blockIdx.x, gridDim.x, tok_tiles, tv, tn);
+  f32x16 acc[2][2];
+  tile32<true, true, kVec>(acc, Mat{w, D}, Mat{h, D}, V, N, 0, D, tv * kT, tn * kT);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
+  const int wm0 = 64 * (wave & 1), wn0 = 64 * (wave >> 1);
+  const int left = sem_v - (tv * kT + wm0 + 4 * hl);  // classes from this lane's first row on
+  float mx[2], sum[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    mx[j] = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx[j] = fmaxf(mx[j], 32 * i + 8 * (r >> 2) + (r & 3) < left ? acc[i][j][r] : -INFINITY);
+    mx[j] = fmaxf(mx[j], __shfl_xor(mx[j], 32));
+    sum[j] = 0.f;
+    // (max ignores NaN logits; the sum must not, also when nothing else is there.)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float x = acc[i][j][r];
+        if (32 * i + 8 * (r >> 2) + (r & 3) < left) sum[j] += mx[j] == -INFINITY && x == x ? 0.f : expf(x - mx[j]);
+      }
+    sum[j] += __shfl_xor(sum[j], 32);
+  }
+  // The two 64-row halves of a token, merged through LDS.
+  if ((wave & 1) && hl == 0) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) half_s[wn0 + 32 * j + lane] = make_float2(mx[j], sum[j]);
+  }
+  __syncthreads();
+  if (!(wave & 1) && hl == 0) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int n = tn * kT + wn0 + 32 * j + lane;
+      const float2 o = half_s[wn0 + 32 * j + lane];
+      const float m = fmaxf(mx[j], o.x);
+      // (A half without classes, or with -inf logits only, adds its sum as it is: 0, or NaN.)
+      const float s = (mx[j] == -INFINITY ? sum[j] : sum[j] * expf(mx[j] - m)) +
+                      (o.x == -INFINITY ? o.y : o.y * expf(o.x - m));
+      if (n < N) partial[(size_t)tv * N + n] = make_float2(m, s);
+    }
+  }
+}
+
+// G^T of one vocabulary chunk: gt[v][n] = (exp(logit - lse) - [v == target]) ct,
+// zero for rows that are no classes (linear_cross_entropy.py:255-266) and for
+// the padding columns N .. ld - 1.
+template <bool kVec>
+__global__ void __launch_bounds__(kThreads, 3)
+    grad32_kernel(const float* __restrict__ w, const float* __restrict__ h, int C, int N, int D, int v0, int sem_v,
+                  const int32_t* __restrict__ targets, const float* __restrict__ lse, const float* __restrict__ cot,
+                  float cot_scale, float* __restrict__ gt, int ld) {
+  const int tok_tiles = (N + kT - 1) / kT;
+  int tv, tn;
+  tile_of(blockIdx.x, gridDim.x, tok_tiles, tv, tn);
+  f32x16 acc[2][2];
+  tile32<true, true, kVec>(acc, Mat{w, D}, Mat{h, D}, C, N, 0, D, tv * kT, tn * kT);
+  // Branch-free, through a buffer resource over the tile's rows: stores past
+  // the chunk or the row are dropped.  (With a branch per element the 64
+  // elements of a lane ran one after the other: 44 against 37 us per chunk of
+  // 2048 rows x 2048 tokens, and 71 against 55 us for the two products below.)
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
+  const int wm0 = 64 * (wave & 1), wn0 = 64 * (wave >> 1);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(gt + (int64_t)tv * kT * ld, row_bytes32(C - tv * kT, ld));
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int n = tn * kT + wn0 + 32 * j + (lane & 31);
+    const bool in = n < N;
+    const int t = in ? targets[n] : -1;
+    const float ct = t >= 0 && t < sem_v ? (cot ? cot[n] : cot_scale) : 0.f;
+    const float l = in ? lse[n] : 0.f;
+    const int row0 = wm0 + 4 * hl;             // this lane's first row of the tile
+    const int left = sem_v - v0 - tv * kT - row0;  // classes from there on
+    const int hit = t - v0 - tv * kT - row0;       // the target's row from there
+    const uint32_t off = n < ld ? 4u * (uint32_t)(row0 * ld + n) : kOff32Drop;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int dr = 32 * i + 8 * (r >> 2) + (r & 3);
+        const float g = (expf(acc[i][j][r] - l) - (dr == hit ? 1.f : 0.f)) * ct;
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, in && dr < left ? g : 0.f), rs,
+                                              off + 4u * (uint32_t)(dr * ld), 0, 0);
+      }
+  }
+}
+
+// The two gradient products of one chunk in one launch: workgroups [0, n_dw)
+// compute dW[chunk] = G^T h (k = tokens), the others dh = G W[chunk] (k = the
+// chunk's rows).  Neither product has enough 128 x 128 tiles for 256 CUs at a
+// few thousand tokens, so each k range is cut into slices and every slice
+// writes a plain partial sum of its own: no atomics, so the results do not
+// depend on the order of the workgroups.  dh's slices accumulate over the
+// chunks in place; sum32_kernel adds the slices.
+struct Out32 {
+  float* p;        // [slices][rows][D]
+  int slices;
+  int64_t stride;  // elements between slices
+  bool add;        // += (the slice holds earlier sums) instead of =
+};
+
+template <bool kVec>
+__global__ void __launch_bounds__(kThreads, 3)
+    grads32_kernel(const float* __restrict__ gt, int ld, const float* __restrict__ w, const float* __restrict__ h, int C,
+                   int N, int D, Out32 dw, Out32 dh, int n_dw) {
+  const int col_tiles = (D + kT - 1) / kT;
+  f32x16 acc[2][2];
+  const bool is_dw = (int)blockIdx.x < n_dw;  // uniform
+  const Out32 o = is_dw ? dw : dh;
+  const int pid = is_dw ? blockIdx.x : blockIdx.x - n_dw;
+  const int rows = is_dw ? C : N, depth = is_dw ? N : C;
+  const int tiles = ((rows + kT - 1) / kT) * col_tiles;
+  const int slice = pid / tiles, id = pid % tiles;
+  const int tr = id / col_tiles, tc = id % col_tiles;
+  const int per = ((depth + o.slices - 1) / o.slices + kK - 1) / kK * kK;
+  const int k0 = slice * per, k1 = min(depth, k0 + per);  // (an empty slice writes zeros)
+  if (is_dw)
+    tile32<true, false, kVec>(acc, Mat{gt, ld}, Mat{h, D}, C, D, k0, k1, tr * kT, tc * kT);
+  else
+    tile32<false, false, kVec>(acc, Mat{gt, ld}, Mat{w, D}, ld, D, k0, k1, tr * kT, tc * kT);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
+  const int wm0 = 64 * (wave & 1), wn0 = 64 * (wave >> 1);
+  const __amdgpu_buffer_rsrc_t rs =
+      make_rsrc(o.p + slice * o.stride + (int64_t)tr * kT * D, row_bytes32(rows - tr * kT, D));
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int c = tc * kT + wn0 + 32 * j + (lane & 31);
+    const uint32_t off = c < D ? 4u * (uint32_t)((wm0 + 4 * hl) * D + c) : kOff32Drop;
+    // All loads of earlier sums first, then the stores.
+    if (o.add) {  // uniform
+      float old[2][16];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          old[i][r] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(rs, off + 4u * (uint32_t)((32 * i + 8 * (r >> 2) + (r & 3)) * D), 0, 0));
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] += old[i][r];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float x = acc[i][j][r];  // (a bit cast straight from a vector element reads element 0 of its quad)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), rs,
+                                              off + 4u * (uint32_t)((32 * i + 8 * (r >> 2) + (r & 3)) * D), 0, 0);
+      }
+  }
+}
+
+// out (+)= the sum of `slices` arrays of n elements.
+__global__ void __launch_bounds__(256) sum32_kernel(const float* __restrict__ parts, int slices, int64_t n,
+                                                    float* __restrict__ out, int add) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  float s = parts[i];
+  for (int k = 1; k < slices; ++k) s += parts[k * n + i];
+  out[i] = add ? out[i] + s : s;
 }
 
 // Target logit h[n] . W[t[n]] in float32 (0 for an invalid target): one wave per token.
@@ -149,39 +433,92 @@ __global__ void __launch_bounds__(256) target32_kernel(const float* __restrict__
   if (lane == 0) tlogit[n] = acc;
 }
 
-// lse = max + log(sum) over the column tiles' partials; loss = lse - target
-// logit, +inf for an invalid target.  One thread per token.
-__global__ void combine32_kernel(const float2* __restrict__ partial, int ntiles, int N, int sem_v,
-                                 const int32_t* __restrict__ targets, const float* __restrict__ tlogit,
-                                 float* __restrict__ lse, float* __restrict__ losses) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float m = -INFINITY;
-  for (int t = 0; t < ntiles; ++t) m = fmaxf(m, partial[(size_t)t * N + n].x);
-  float s = 0.f;
-  for (int t = 0; t < ntiles; ++t) {
-    const float2 p = partial[(size_t)t * N + n];
-    if (p.x != -INFINITY) s += p.y * expf(p.x - m);
+// lse = max + log(sum) over the vocabulary tiles' partials; loss = lse - target
+// logit, +inf for an invalid target.  64 tokens per workgroup, each of its 16
+// waves folding every 16th tile: one thread per token ran 365 us at 2048
+// tokens and V 50304 (8 workgroups, one dependent pass after the other), this
+// form 13 us.
+constexpr int kCombineWaves = 16;
+__global__ void __launch_bounds__(64 * kCombineWaves)
+    combine32_kernel(const float2* __restrict__ partial, int ntiles, int N, int sem_v,
+                     const int32_t* __restrict__ targets, const float* __restrict__ tlogit, float* __restrict__ lse,
+                     float* __restrict__ losses) {
+  __shared__ float m_s[kCombineWaves][64], s_s[kCombineWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = blockIdx.x * 64 + lane;
+  float m = -INFINITY, s = 0.f;
+  if (n < N) {
+    for (int t = wave; t < ntiles; t += kCombineWaves) m = fmaxf(m, partial[(size_t)t * N + n].x);
+    for (int t = wave; t < ntiles; t += kCombineWaves) {
+      const float2 p = partial[(size_t)t * N + n];
+      s += p.x == -INFINITY ? p.y : p.y * expf(p.x - m);  // (p.y is 0, or NaN, without a maximum)
+    }
   }
-  const float l = m + logf(s);
+  m_s[wave][lane] = m;
+  s_s[wave][lane] = s;
+  __syncthreads();
+  if (wave || n >= N) return;
+  float mt = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < kCombineWaves; ++k) mt = fmaxf(mt, m_s[k][lane]);
+  float st = 0.f;
+#pragma unroll
+  for (int k = 0; k < kCombineWaves; ++k)
+    st += m_s[k][lane] == -INFINITY ? s_s[k][lane] : s_s[k][lane] * expf(m_s[k][lane] - mt);
+  const float l = mt + logf(st);
   lse[n] = l;
   const int t = targets[n];
   losses[n] = (t >= 0 && t < sem_v) ? l - tlogit[n] : INFINITY;
 }
 
-__global__ void zero32_kernel(float* __restrict__ x, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = 0.f;
-}
-
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 int chunk32(int vocab, int vocab_chunk) {
-  const int c = vocab_chunk <= 0 ? 2048 : (vocab_chunk + kT - 1) / kT * kT;
-  return c < vocab ? c : (vocab + kT - 1) / kT * kT;
+  const int64_t c = vocab_chunk <= 0 ? 2048 : ((int64_t)vocab_chunk + kChunkRows - 1) / kChunkRows * kChunkRows;
+  return (int)(c < vocab ? c : ((int64_t)vocab + kChunkRows - 1) / kChunkRows * kChunkRows);
 }
 
-dim3 grid_of(int M, int N) { return dim3((unsigned)((M + kT - 1) / kT), (unsigned)((N + kT - 1) / kT)); }
+// Columns of the G^T rows: n rounded up to whole 16-byte groups.
+int64_t gt_ld(int n) { return ((int64_t)n + 3) & ~(int64_t)3; }
+
+int64_t tiles32(int64_t rows, int64_t cols) { return ((rows + kT - 1) / kT) * ((cols + kT - 1) / kT); }
+
+// Slices of a gradient product of rows x d outputs over `depth`: enough
+// workgroups for one per CU (256 are assumed; a fixed number keeps the
+// workspace query independent of the device), slices at least 8 stages deep,
+// and all partial sums together no larger than the [n, chunk] gradient.
+int slices32(int64_t rows, int d, int depth, int64_t budget) {
+  const int64_t tiles = tiles32(rows, d);
+  int64_t s = (256 + tiles / 2) / tiles;
+  const int64_t deep = depth / (8 * kK), fit = budget / (rows * d);
+  if (s > deep) s = deep;
+  if (s > fit) s = fit;
+  return s < 1 ? 1 : (int)s;
+}
+
+struct Plan32 {
+  int chunk, dh_slices, dw_slices;
+  int64_t ld;
+  size_t gt_bytes, dh_bytes, dw_bytes;  // workspace: G^T, dh partials, dW partials (0: written in place)
+};
+
+Plan32 plan32(int n, int d, int vocab, int vocab_chunk) {
+  Plan32 p;
+  p.chunk = chunk32(vocab, vocab_chunk);
+  p.ld = gt_ld(n);
+  const int64_t gt = (int64_t)p.chunk * p.ld;
+  p.dh_slices = slices32(n, d, p.chunk, gt);
+  p.dw_slices = slices32(p.chunk, d, n, gt);
+  p.gt_bytes = align256((size_t)gt * sizeof(float));
+  p.dh_bytes = p.dh_slices > 1 ? align256((size_t)p.dh_slices * n * d * sizeof(float)) : 0;
+  p.dw_bytes = p.dw_slices > 1 ? align256((size_t)p.dw_slices * p.chunk * d * sizeof(float)) : 0;
+  return p;
+}
+
+// 16-byte loads of rows of d floats.
+bool vec32(const float* a, const float* b, int d) {
+  return d % 4 == 0 && (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
+}
 
 }  // namespace
 
@@ -206,24 +543,23 @@ int gptrig_flce32_fwd(const float* hidden, const float* weight, const int32_t* t
   const int ntiles = (vocab + kT - 1) / kT;
   float2* partial = (float2*)workspace;
   float* tlogit = (float*)((char*)workspace + align256((size_t)ntiles * n * sizeof(float2)));
-  Epi32 e{};
-  e.partial = partial;
-  e.sem_v = semantic_vocab;
-  // logits[token][v] = sum_d h[token][d] W[v][d]
-  gemm32_kernel<kStats><<<grid_of(n, vocab), 256, 0, s>>>(Mat{hidden, d, 1}, Mat{weight, 1, d}, n, vocab, d, e);
+  // logits[v][token] = sum_d W[v][d] h[token][d]
+  const unsigned grid = (unsigned)tiles32(vocab, n);
+  (vec32(hidden, weight, d) ? stats32_kernel<true> : stats32_kernel<false>)<<<grid, kThreads, 0, s>>>(
+      weight, hidden, vocab, n, d, semantic_vocab, partial);
   GPTRIG_CHECK_LAUNCH();
   target32_kernel<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(hidden, weight, targets, n, d, semantic_vocab, tlogit);
   GPTRIG_CHECK_LAUNCH();
-  combine32_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(partial, ntiles, n, semantic_vocab, targets, tlogit,
-                                                                lse, losses);
+  combine32_kernel<<<(unsigned)((n + 63) / 64), 64 * kCombineWaves, 0, s>>>(partial, ntiles, n, semantic_vocab,
+                                                                             targets, tlogit, lse, losses);
   GPTRIG_CHECK_LAUNCH();
   return GPTRIG_OK;
 }
 
 size_t gptrig_flce32_bwd_workspace_bytes(int n, int d, int vocab, int vocab_chunk) {
-  (void)d;
-  if (n <= 0 || vocab <= 0) return 0;
-  return align256((size_t)n * chunk32(vocab, vocab_chunk) * sizeof(float));
+  if (n <= 0 || d <= 0 || vocab <= 0) return 0;
+  const Plan32 p = plan32(n, d, vocab, vocab_chunk);
+  return p.gt_bytes + p.dh_bytes + p.dw_bytes;
 }
 
 int gptrig_flce32_bwd(const float* hidden, const float* weight, const int32_t* targets, const float* lse,
@@ -236,39 +572,36 @@ int gptrig_flce32_bwd(const float* hidden, const float* weight, const int32_t* t
   if (workspace_bytes < gptrig_flce32_bwd_workspace_bytes(n, d, vocab, vocab_chunk)) return GPTRIG_E_WORKSPACE;
   if ((int64_t)n * d >= (1ll << 31) || (int64_t)vocab * d >= (1ll << 31)) return GPTRIG_E_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-  const int C = chunk32(vocab, vocab_chunk);
+  const Plan32 p = plan32(n, d, vocab, vocab_chunk);
   float* G = (float*)workspace;
-  zero32_kernel<<<(unsigned)(((int64_t)n * d + 255) / 256), 256, 0, s>>>(dhidden, (int64_t)n * d);
-  GPTRIG_CHECK_LAUNCH();
-  for (int v0 = 0; v0 < vocab; v0 += C) {
-    const int c = vocab - v0 < C ? vocab - v0 : C;
+  float* dh_parts = (float*)((char*)workspace + p.gt_bytes);
+  float* dw_parts = (float*)((char*)workspace + p.gt_bytes + p.dh_bytes);
+  const int64_t nd = (int64_t)n * d;
+  const bool vec = vec32(hidden, weight, d) && ((uintptr_t)workspace & 15) == 0;
+  for (int v0 = 0; v0 < vocab; v0 += p.chunk) {
+    const int c = vocab - v0 < p.chunk ? vocab - v0 : p.chunk;
     const float* Wc = weight + (int64_t)v0 * d;
-    Epi32 g{};
-    g.out = G;
-    g.ld = c;
-    g.col0 = v0;
-    g.sem_v = semantic_vocab;
-    g.targets = targets;
-    g.lse = lse;
-    g.cot = cotangent;
-    g.cot_scale = cotangent_scale;
-    // G[token][v] = (exp(logit - lse) - onehot) * ct for the chunk's rows.
-    gemm32_kernel<kGrad><<<grid_of(n, c), 256, 0, s>>>(Mat{hidden, d, 1}, Mat{Wc, 1, d}, n, c, d, g);
+    float* dWc = dweight + (int64_t)v0 * d;
+    const int64_t cd = (int64_t)c * d;
+    (vec ? grad32_kernel<true> : grad32_kernel<false>)<<<(unsigned)tiles32(c, n), kThreads, 0, s>>>(
+        Wc, hidden, c, n, d, v0, semantic_vocab, targets, lse, cotangent, cotangent_scale, G, (int)p.ld);
     GPTRIG_CHECK_LAUNCH();
-    // dh += G W[chunk]  (the reference's grad_hidden carry, :247)
-    Epi32 a{};
-    a.out = dhidden;
-    a.ld = d;
-    gemm32_kernel<kAccum><<<grid_of(n, d), 256, 0, s>>>(Mat{G, c, 1}, Mat{Wc, d, 1}, n, d, c, a);
+    // dW[chunk] (+)= G^T h (the dynamic_update_slice of :279-283) and
+    // dh += G W[chunk] (the reference's grad_hidden carry, :247).
+    const Out32 dw{p.dw_bytes ? dw_parts : dWc, p.dw_slices, cd, !p.dw_bytes && accumulate_dweight != 0};
+    const Out32 dh{p.dh_bytes ? dh_parts : dhidden, p.dh_slices, nd, v0 > 0};
+    const int64_t n_dw = tiles32(c, d) * p.dw_slices, n_dh = tiles32(n, d) * p.dh_slices;
+    (vec ? grads32_kernel<true> : grads32_kernel<false>)<<<(unsigned)(n_dw + n_dh), kThreads, 0, s>>>(
+        G, (int)p.ld, Wc, hidden, c, n, d, dw, dh, (int)n_dw);
     GPTRIG_CHECK_LAUNCH();
-    // dW[chunk] (+)= G^T h  (the dynamic_update_slice of :279-283)
-    Epi32 w{};
-    w.out = dweight + (int64_t)v0 * d;
-    w.ld = d;
-    if (accumulate_dweight)
-      gemm32_kernel<kAccum><<<grid_of(c, d), 256, 0, s>>>(Mat{G, 1, c}, Mat{hidden, d, 1}, c, d, n, w);
-    else
-      gemm32_kernel<kStore><<<grid_of(c, d), 256, 0, s>>>(Mat{G, 1, c}, Mat{hidden, d, 1}, c, d, n, w);
+    if (p.dw_bytes) {
+      sum32_kernel<<<(unsigned)((cd + 255) / 256), 256, 0, s>>>(dw_parts, p.dw_slices, cd, dWc,
+                                                                accumulate_dweight != 0);
+      GPTRIG_CHECK_LAUNCH();
+    }
+  }
+  if (p.dh_bytes) {
+    sum32_kernel<<<(unsigned)((nd + 255) / 256), 256, 0, s>>>(dh_parts, p.dh_slices, nd, dhidden, 0);
     GPTRIG_CHECK_LAUNCH();
   }
   return GPTRIG_OK;

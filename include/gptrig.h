@@ -131,8 +131,12 @@ int gptrig_flce_bwd(const void* hidden, const void* weight, const int32_t* targe
  * product and sum in float32 (lse and losses as gptrig_flce_fwd); the
  * backward recomputes the logits per chunk of vocab_chunk rows (0: 2048,
  * rounded up to 64) with a float32 [n, chunk] logit-gradient workspace, the
- * reference's [n, vocab_tile_size] bound, and writes dhidden f32 [n, d] and
- * dweight f32 [vocab, d] (+= with accumulate_dweight).  Any n, d. */
+ * reference's [n, vocab_tile_size] bound, plus partial sums of the two gradient
+ * products, each at most as large, and writes dhidden f32 [n, d] and
+ * dweight f32 [vocab, d] (+= with accumulate_dweight).  Any n, d.  Results do
+ * not depend on the order of the workgroups (no atomics).  The products run on
+ * the bf16 matrix cores from exact three-way splits of the float32 operands,
+ * so an infinite operand gives NaN where a float32 product may give an infinity. */
 size_t gptrig_flce32_fwd_workspace_bytes(int n, int d, int vocab);
 int gptrig_flce32_fwd(const float* hidden, const float* weight, const int32_t* targets, float* losses, float* lse,
                       void* workspace, size_t workspace_bytes, int n, int d, int vocab, int semantic_vocab,

@@ -339,3 +339,101 @@ def test_float32_compute_matches_float64_dense(n, d, V, sv, tile):
         print(f"  grad max-abs {err:.3e} of {scale:.3e}", flush=True)
         assert err <= 1e-5 * scale
     assert (wg.grad[sv:] == 0).all()
+
+
+@pytest.mark.parametrize("n,d,V,sv,tile,offset", [
+    (1, 1, 1, 1, 1, 0),            # one element everywhere
+    (127, 16, 129, 128, 64, 0),    # one row short of / past the 128 tile, one k stage, a 64-row chunk
+    (128, 132, 256, 256, 128, 0),  # whole tiles, k = 8 stages and 4 columns
+    (129, 37, 385, 300, 200, 0),   # odd width (element loads), ragged chunks
+    (514, 64, 1100, 1100, 2048, 1),  # 16-byte loads ruled out by the base address; sliced partial sums
+    (1280, 128, 2048, 2000, 1024, 0),  # several slices of both products, two chunks
+])
+def test_float32_split_products_at_tile_edges(n, d, V, sv, tile, offset):
+    """The split-operand float32 tiles against float64 where they can go
+    wrong: tile, stage, slice and chunk edges, widths and bases without
+    16-byte loads, accumulation into dweight, and the same bits twice.
+
+    Bound: a product drops less than 2^-22 of itself and the operands are
+    split exactly; a sum over k is rounded once per MFMA (16 products), so an
+    output is within (2^-22 + ceil(k/16) 6 2^-24) of the sum of its products'
+    magnitudes, k the contraction's length; G adds the error of its logits."""
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    g = torch.Generator().manual_seed(n)
+    flat = torch.randn(n * d + V * d + 1, generator=g).to(DEV)
+    h = flat[offset:offset + n * d].view(n, d)
+    w = flat[offset + n * d:offset + n * d + V * d].mul_(0.3).view(V, d)
+    t = torch.randint(0, sv, (n,), generator=g, dtype=torch.int32).to(DEV)
+    if n > 5:
+        t[3] = -1
+        t[5] = sv
+    ct = torch.rand(n, generator=g).to(DEV)
+    print(f"flce float32 tiles n={n} d={d} V={V} sv={sv} tile={tile} base%16={h.data_ptr() % 16}", flush=True)
+    runs = []
+    for _ in range(2):
+        losses, lse = lce.flce32_forward(h, w, t, sv)
+        runs.append((losses, *lce.flce32_backward(h, w, t, lse, ct, 0.0, sv, tile)))
+    assert all(torch.equal(a, b) for a, b in zip(*runs))
+    losses, dh, dw = (x.cpu().double() for x in runs[0])
+    h64, w64, t64 = h.cpu().double(), w.cpu().double(), t.cpu().long()
+    valid = (t64 >= 0) & (t64 < sv)
+    logits = h64 @ w64[:sv].t()
+    lse64 = torch.logsumexp(logits, -1)
+    safe = t64.clamp(0, sv - 1)[:, None]
+    want = torch.where(valid, lse64 - logits.gather(1, safe)[:, 0], torch.inf)
+    c64 = torch.where(valid, ct.cpu().double(), 0.0)[:, None]
+    grad = torch.zeros((n, V), dtype=torch.float64)
+    grad[:, :sv] = torch.exp(logits - lse64[:, None]) * c64
+    grad.scatter_add_(1, safe, -c64)
+    eps = lambda k: 2.0 ** -22 + -(-k // 16) * 6 * 2.0 ** -24  # noqa: E731
+    # A logit's absolute error; the probabilities (and lse) carry it relatively.
+    mags = (h64.abs() @ w64.abs().t()).max()
+    dl = float(mags) * eps(d) + 4 * 2.0 ** -24 * float(lse64.abs().max() + 1)
+    assert torch.equal(torch.isfinite(losses), valid)
+    err = (losses - want)[valid].abs().max()
+    print(f"  loss {float(err):.2e} of {2 * dl:.2e}", flush=True)
+    assert err <= 2 * dl
+    for name, got, ref, big, k in (("dh", dh, grad @ w64, grad.abs() @ w64.abs(), V),
+                                   ("dw", dw, grad.t() @ h64, grad.abs().t() @ h64.abs(), n)):
+        # (2 dl: the logit's and lse's error; onehot entries keep their own magnitude.)
+        p = torch.zeros_like(grad)
+        p[:, :sv] = torch.exp(logits - lse64[:, None]) * c64
+        noise = p @ w64.abs() if name == "dh" else p.t() @ h64.abs()
+        bound = big * eps(k) + noise * (2 * dl + 2.0 ** -22) + 1e-12
+        excess = float(((got - ref).abs() / bound).max())
+        print(f"  {name} error / bound {excess:.3f}", flush=True)
+        assert excess <= 1
+    assert (dw[sv:] == 0).all()
+    from gptrig import _lib
+
+    base = torch.randn((V, d), generator=g).to(DEV)
+    total = base.clone()
+    dh2 = torch.empty_like(h)
+    ws = _lib.workspace(_lib.query("gptrig_flce32_bwd_workspace_bytes", n, d, V, tile), DEV)
+    _lib.call("gptrig_flce32_bwd", h.data_ptr(), w.data_ptr(), t.data_ptr(), lse.data_ptr(), ct.data_ptr(), 0.0,
+              dh2.data_ptr(), total.data_ptr(), 1, ws.data_ptr(), ws.numel(), n, d, V, sv, tile, _lib.stream())
+    assert torch.equal(dh2, runs[0][1])
+    # accumulate_dweight adds to what is there (one more rounding).
+    torch.testing.assert_close(total, base + runs[0][2], rtol=0, atol=float(base.abs().max()) * 2.0 ** -22)
+
+
+def test_float32_nan_rows_stay_in_their_rows():
+    """A NaN hidden row gives a NaN loss and hidden gradient for its token
+    alone; the other tokens' losses and hidden gradients are untouched."""
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    g = torch.Generator().manual_seed(5)
+    h = torch.randn((200, 48), generator=g).to(DEV)
+    w = torch.randn((300, 48), generator=g).to(DEV)
+    t = torch.randint(0, 300, (200,), generator=g, dtype=torch.int32).to(DEV)
+    ct = torch.ones(200, device=DEV)
+    print("flce float32 NaN row", flush=True)
+    l0, s0 = lce.flce32_forward(h, w, t, 300)
+    dh0, _ = lce.flce32_backward(h, w, t, s0, ct, 0.0, 300, 128)
+    h[7, 5] = float("nan")
+    l1, s1 = lce.flce32_forward(h, w, t, 300)
+    dh1, _ = lce.flce32_backward(h, w, t, s1, ct, 0.0, 300, 128)
+    rest = torch.arange(200, device=DEV) != 7
+    assert torch.isnan(l1[7]) and torch.isnan(dh1[7]).all()
+    assert torch.equal(l0[rest], l1[rest]) and torch.equal(dh0[rest], dh1[rest])
