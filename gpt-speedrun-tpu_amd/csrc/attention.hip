@@ -121,6 +121,102 @@ __global__ void attn_dq_convert_kernel(const float* __restrict__ dq_acc, MutView
 }
 
 // ============================================================================
+// Skipping what document masking hides
+// ============================================================================
+// With segment ids a workgroup owns a block of positions (128 queries in the
+// forward, the keys in the backward) and walks 64-position blocks of the other
+// side.  A block none of whose ids lies between the lowest and the highest id
+// of the owned block holds no visible pair, whatever the order of the ids, so
+// it is neither loaded nor computed.  A block whose ids all equal the owned
+// block's single id needs no per-element id compare.
+// The blocks are tested 64 at a time: each wave reads its share of the ids
+// (one coalesced load, a compare and a ballot per block) and the bits are
+// exchanged through LDS.  That is 32 KB of ids per workgroup at 8192 positions
+// against the 16 KB of K and V that every block not skipped costs.
+// Measured at B2 H12 S8192 D64, documents of 1..3000 tokens: forward + backward
+// 1513 -> 595 us (backward kernel 994 -> 396, forward 554 -> 232); what is left
+// above the visible share of the work (about a quarter) is the uneven lengths
+// of the workgroups.  Where nothing can be skipped (one document) the test costs
+// about 2 us per workgroup and saves the compares: B16 H12 S1024 D64 forward
+// 93 -> 60, backward 192 -> 184 us; B8 H6 S1024 D128 forward 75 -> 39, backward
+// 122 -> 128 us.
+template <int kWaves>
+struct SegScan {
+  static constexpr int kPer = 64 / kWaves;  // blocks a wave tests
+  using Piece = std::conditional_t<kPer == 8, uint8_t, uint16_t>;
+  const int32_t* ids;  // this sequence's ids
+  uint64_t* sh;        // LDS: the need and the same bits of 64 blocks (kept here: registers are short)
+  int S, lo, hi;       // the owned block's id range
+  int group;           // the 64 blocks that the bits describe
+
+  // Id range of the owned positions p0 .. p0 + 64 kOwn - 1 (those below S).
+  template <int kOwn>
+  __device__ __forceinline__ void init(const int32_t* seq_ids, uint64_t* lds, int seq, int p0, int lane) {
+    ids = seq_ids;
+    sh = lds;
+    S = seq;
+    group = -1;
+    int a = ids[min(p0 + lane, S - 1)], z = a;
+#pragma unroll
+    for (int j = 1; j < kOwn; ++j) {
+      const int x = ids[min(p0 + 64 * j + lane, S - 1)];
+      a = min(a, x);
+      z = max(z, x);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      a = min(a, __shfl_xor(a, o));
+      z = max(z, __shfl_xor(z, o));
+    }
+    lo = __builtin_amdgcn_readfirstlane(a);
+    hi = __builtin_amdgcn_readfirstlane(z);
+  }
+
+  // (Every wave calls this the same number of times: it holds two barriers.)
+  __device__ __forceinline__ void load(int g, int wave, int lane) {
+    group = g;
+    uint32_t n = 0, f = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int p = (64 * g + kPer * wave + j) * 64 + lane;
+      const int id = ids[min(p, S - 1)];
+      const bool in = id >= lo && id <= hi;
+      n |= __ballot(in && p < S) != 0 ? 1u << j : 0u;
+      f |= __ballot(in || p >= S) == ~0ull ? 1u << j : 0u;
+    }
+    __syncthreads();
+    if (lane == 0) {
+      reinterpret_cast<Piece*>(sh)[wave] = (Piece)n;
+      reinterpret_cast<Piece*>(sh + 1)[wave] = (Piece)(lo == hi ? f : 0u);
+    }
+    __syncthreads();
+  }
+
+  __device__ __forceinline__ uint64_t bits(int which) const {
+    const uint64_t v = sh[which];
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+  }
+
+  // The first block at or after t (below nblk) with a visible pair, else nblk;
+  // same: its ids need no compare.
+  __device__ __forceinline__ int next(int t, int nblk, int wave, int lane, bool& same) {
+    same = false;
+    while (t < nblk) {
+      if ((t >> 6) != group) load(t >> 6, wave, lane);
+      const uint64_t m = bits(0) >> (t & 63);
+      if (m) {
+        t += __builtin_ctzll(m);
+        same = bits(1) >> (t & 63) & 1;
+        return min(t, nblk);
+      }
+      t = ((t >> 6) + 1) << 6;
+    }
+    return nblk;
+  }
+};
+
+// ============================================================================
 // Kernels on swizzled row-major LDS tiles (attn64.h)
 // ============================================================================
 
@@ -168,6 +264,9 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
   for (int kc = 0; kc < KC; ++kc)
     qreg[kc] = my_q < S ? *reinterpret_cast<const bf16x8*>(Q.row(b, h, my_q) + 16 * kc + 8 * hl) : bf16x8{};
   const int seg_q = (kSeg && my_q < S) ? seg[(size_t)b * S + my_q] : 0;
+  __shared__ uint64_t scan_s[2];
+  SegScan<4> scan;
+  if constexpr (kSeg) scan.template init<kBlockM / 64>(seg + (size_t)b * S, scan_s, S, q0, lane);
 
   f32x16 acc[DB];
 #pragma unroll
@@ -202,8 +301,10 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
     }
   };
 
-  // One 32-key half of a tile in buffer (kt, vt).
-  auto half = [&](const at64::lds_t* kt, const at64::lds_t* vt, int kv0, int sb) __attribute__((always_inline)) {
+  // One 32-key half of a tile in buffer (kt, vt); same: every id of the tile
+  // equals every query's (no compare).
+  auto half = [&](const at64::lds_t* kt, const at64::lds_t* vt, int kv0, int sb,
+                  bool same) __attribute__((always_inline)) {
     f32x16 s = f32x16{};
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc)
@@ -211,7 +312,7 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
     // Row max on raw scores (scale > 0); masked scores become -inf.
     const int kh0 = kv0 + 32 * sb;
     float mraw = -INFINITY;
-    if constexpr (kSeg) {
+    if (kSeg && !same) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int key = kh0 + 8 * (i >> 2) + 4 * hl + (i & 3);
@@ -267,13 +368,15 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
                          pb[c2], acc[db]);
   };
 
-  auto tile = [&](const at64::lds_t* kt, const at64::lds_t* vt, at64::lds_t* nkt, at64::lds_t* nvt, int it) {
+  // Tile `it` from (kt, vt), the tile after it, `nx`, on its way to (nkt, nvt).
+  auto tile = [&](const at64::lds_t* kt, const at64::lds_t* vt, at64::lds_t* nkt, at64::lds_t* nvt, int it, int nx,
+                  bool same) {
     const int kv0 = it * kBlockN;
-    if (it + 1 < ntiles) fill(nkt, nvt, kv0 + kBlockN);
+    if (nx < ntiles) fill(nkt, nvt, nx * kBlockN);
     // Halves whose every key lies past the wave's last query add nothing.
-    if (kv0 <= qw0 + 31) half(kt, vt, kv0, 0);
+    if (kv0 <= qw0 + 31) half(kt, vt, kv0, 0, same);
     __builtin_amdgcn_sched_barrier(0);  // keep the halves' live ranges apart
-    if (kv0 + 32 <= qw0 + 31) half(kt, vt, kv0, 1);
+    if (kv0 + 32 <= qw0 + 31) half(kt, vt, kv0, 1, same);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next tile has landed
     __syncthreads();
   };
@@ -282,12 +385,28 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
   at64::lds_t* const k1s = gemm::lds_cast(fk1);
   at64::lds_t* const v0s = gemm::lds_cast(fv0);
   at64::lds_t* const v1s = gemm::lds_cast(fv1);
-  fill(k0s, v0s, 0);
+  bool same = false, same_n = false;
+  int it = 0;
+  if constexpr (kSeg) it = scan.next(0, ntiles, wave, lane, same);
+  fill(k0s, v0s, it * kBlockN);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
-  for (int it = 0; it < ntiles; it += 2) {
-    tile(k0s, v0s, k1s, v1s, it);
-    if (it + 1 < ntiles) tile(k1s, v1s, k0s, v0s, it + 1);
+  if constexpr (kSeg) {
+    while (true) {
+      int nx = scan.next(it + 1, ntiles, wave, lane, same_n);
+      tile(k0s, v0s, k1s, v1s, it, nx, same);
+      if (nx >= ntiles) break;
+      it = nx;
+      nx = scan.next(it + 1, ntiles, wave, lane, same);
+      tile(k1s, v1s, k0s, v0s, it, nx, same_n);
+      if (nx >= ntiles) break;
+      it = nx;
+    }
+  } else {
+    for (; it < ntiles; it += 2) {
+      tile(k0s, v0s, k1s, v1s, it, it + 1, false);
+      if (it + 1 < ntiles) tile(k1s, v1s, k0s, v0s, it + 1, it + 2, false);
+    }
   }
 
   const float l_tot = l_run + __shfl_xor(l_run, 32);
@@ -307,8 +426,10 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
   }
 }
 
+// (With segment ids the two mask forms need more than 128 registers: three
+// workgroups per CU instead of four.)
 template <bool kSeg>
-__global__ void __launch_bounds__(256, 4)
+__global__ void __launch_bounds__(256, kSeg ? 3 : 4)
     attn_fwd64_kernel(View Q, View K, View V, MutView O, float* __restrict__ lse, const int32_t* __restrict__ seg,
                       int B, int H, int S, float scale_log2) {
   attn_fwd_swz<64, kSeg>(Q, K, V, O, lse, seg, B, H, S, scale_log2);
@@ -359,6 +480,9 @@ __global__ void __launch_bounds__(kBwd64Threads, 2)
   const bool k_ok = my_k < S;
 
   const int seg_k = (kSeg && k_ok) ? seg[(size_t)b * S + my_k] : 0;
+  __shared__ uint64_t scan_s[2];
+  SegScan<8> scan;
+  if constexpr (kSeg) scan.template init<NK / 64>(seg + (size_t)b * S, scan_s, S, k0, lane);
 
   {
     // (Branch-free, so these loads issue together with the K / V loads below.)
@@ -446,8 +570,13 @@ __global__ void __launch_bounds__(kBwd64Threads, 2)
   load_q(qb_first * kBwdM);
   store_q();
 
-  for (int qb = qb_first; qb < nqb; ++qb) {
+  // (The first block is the diagonal one: always visible.)
+  bool same = false, same_n = false;
+  int nx = 0;
+  if constexpr (kSeg) scan.next(qb_first, nqb, wave, lane, same);
+  for (int qb = qb_first; qb < nqb; qb = kSeg ? nx : qb + 1, same = same_n) {
     const int qq0 = qb * kBwdM;
+    if constexpr (kSeg) nx = scan.next(qb + 1, nqb, wave, lane, same_n);
     // (A) Q, dO, lse, delta of this block published.  Only LDS has to be
     // complete here: the previous block's dQ atomics stay in flight.
     GPTRIG_WAIT_LGKM0();
@@ -456,7 +585,10 @@ __global__ void __launch_bounds__(kBwd64Threads, 2)
     // once every wave is done with this block's Q / dO, ahead of the dQ
     // atomics (so that wait never drains them).
     // (The last block re-loads itself: the same code on every iteration.)
-    load_q(qb + 1 < nqb ? qq0 + kBwdM : qq0);
+    if constexpr (kSeg)
+      load_q(nx < nqb ? nx * kBwdM : qq0);
+    else
+      load_q(qb + 1 < nqb ? qq0 + kBwdM : qq0);
 
     const bool wave_active = kw0 <= qq0 + kBwdM - 1 && kw0 < S;
     // One 32-query half of the block.  kMask: the causal / ragged / segment
@@ -521,7 +653,7 @@ __global__ void __launch_bounds__(kBwd64Threads, 2)
     if (!wave_active) {
 #pragma unroll
       for (int c = 0; c < 8; ++c) *(__attribute__((address_space(3))) bf16x4*)(dSt + at64::swz(32 * wave + l32, c) + 4 * hl) = bf16x4{};
-    } else if ((qq0 < kw0 + 31) || (qq0 + kBwdM > S) || (kw0 + 32 > S) || kSeg) {
+    } else if ((qq0 < kw0 + 31) || (qq0 + kBwdM > S) || (kw0 + 32 > S) || (kSeg && !same)) {
       qs_body(0, std::true_type{});
       __builtin_amdgcn_sched_barrier(0);  // keep the two halves' live ranges apart
       qs_body(1, std::true_type{});
@@ -661,6 +793,9 @@ __global__ void __launch_bounds__(kBwd128Threads, 1)
                                              v_rs, (my_k * (int)V.ss + 8 * (2 * kc + hl)) * 2, 0, 0));
   }
   const int seg_k = (kSeg && my_k < S) ? seg[(size_t)b * S + my_k] : 0;
+  __shared__ uint64_t scan_s[2];
+  SegScan<4> scan;
+  if constexpr (kSeg) scan.template init<NK / 64>(seg + (size_t)b * S, scan_s, S, k0, lane);
 #pragma unroll
   for (int r = 0; r < KR; ++r) {
     const int idx = tid + NT * r;
@@ -769,18 +904,26 @@ __global__ void __launch_bounds__(kBwd128Threads, 1)
   load_q(qb_first * M);
   store_q(0);
 
-  auto begin = [&](int qb) {
+  // The query block after qb that is computed.
+  auto after = [&](int qb) {
+    if constexpr (kSeg) {
+      bool same;
+      return scan.next(qb + 1, nqb, wave, lane, same);
+    } else {
+      return qb + 1;
+    }
+  };
+  auto begin = [&](int qb, int nx) {
     // Q / dO / lse / Delta of this block and the previous block's dS^T published.
     GPTRIG_WAIT_LGKM0();
     wg_barrier();
-    load_q(qb + 1 < nqb ? (qb + 1) * M : qb * M);
+    load_q(nx < nqb ? nx * M : qb * M);
   };
-  auto nbuf = [&](int qb) { return ((qb - qb_first) & 1) ^ 1; };  // the buffer of block qb - 1 / qb + 1
 
   // Scores, dS and dV / dK of query block qb against this wave's 32 keys.
-  auto body = [&](int qb, auto mask_tag) {
+  auto body = [&](int qb, int buf, auto mask_tag) {
     constexpr bool kMask = decltype(mask_tag)::value;
-    const int qq0 = qb * M, buf = (qb - qb_first) & 1;
+    const int qq0 = qb * M;
     const at64::lds_t* const Qs = gemm::lds_cast(q_smem) + buf * M * D;
     const at64::lds_t* const dOs = gemm::lds_cast(g_smem) + buf * M * D;
     at64::lds_t* const dSt = gemm::lds_cast(ds_smem) + buf * NK * M;
@@ -846,36 +989,50 @@ __global__ void __launch_bounds__(kBwd128Threads, 1)
 
   // Per wave: the first block (no dQ before it), the blocks before this
   // wave's keys (no scores), the diagonal block (causal mask), the blocks
-  // after it (mask-free unless segment ids are given).  Every wave runs
-  // nqb - qb_first blocks, one barrier each, so the barriers match; no dQ is
+  // after it (mask-free unless segment ids are given).  Every wave runs the
+  // same blocks, one barrier each, so the barriers match; no dQ is
   // conditional inside a phase, so the waits for the prefetched block count
-  // the atomics issued after it instead of draining them.
+  // the atomics issued after it instead of draining them.  (The blocks of the
+  // workgroup's own keys always hold visible pairs, so the first block and the
+  // diagonal blocks are never skipped.)
   const int my_first = min(kw0 / M, nqb);
-  begin(qb_first);
+  int prev = qb_first, buf = 1;  // the last block computed; the buffer of the next
+  int qb = after(qb_first);
+  begin(qb_first, qb);
   if (my_first == qb_first)
-    body(qb_first, std::true_type{});
+    body(qb_first, 0, std::true_type{});
   else
     zero_ds(0);
   store_q(1);
-  int qb = qb_first + 1;
-  for (; qb < my_first; ++qb) {
-    begin(qb);
-    zero_ds(nbuf(qb) ^ 1);
-    dq_step((qb - 1) * M, nbuf(qb));
-    store_q(nbuf(qb));
+  while (qb < my_first) {
+    const int nx = after(qb);
+    begin(qb, nx);
+    zero_ds(buf);
+    dq_step(prev * M, buf ^ 1);
+    store_q(buf ^ 1);
+    prev = qb;
+    qb = nx;
+    buf ^= 1;
   }
   if (qb == my_first && qb < nqb) {
-    begin(qb);
-    body(qb, std::true_type{});
-    store_q(nbuf(qb));
-    dq_step((qb - 1) * M, nbuf(qb));
-    ++qb;
+    const int nx = after(qb);
+    begin(qb, nx);
+    body(qb, buf, std::true_type{});
+    store_q(buf ^ 1);
+    dq_step(prev * M, buf ^ 1);
+    prev = qb;
+    qb = nx;
+    buf ^= 1;
   }
-  for (; qb < nqb; ++qb) {
-    begin(qb);
-    body(qb, std::integral_constant<bool, kSeg>{});
-    store_q(nbuf(qb));
-    dq_step((qb - 1) * M, nbuf(qb));
+  while (qb < nqb) {
+    const int nx = after(qb);
+    begin(qb, nx);
+    body(qb, buf, std::integral_constant<bool, kSeg>{});
+    store_q(buf ^ 1);
+    dq_step(prev * M, buf ^ 1);
+    prev = qb;
+    qb = nx;
+    buf ^= 1;
   }
 
   // dV and dK rows of this wave's keys (lane: key my_k, d = 32db + 8r + 4hl
@@ -926,7 +1083,7 @@ __global__ void __launch_bounds__(kBwd128Threads, 1)
   // The last block's dQ, after the dK / dV stores so no store waits for its atomics.
   GPTRIG_WAIT_LGKM0();
   wg_barrier();
-  dq_step((nqb - 1) * M, (nqb - 1 - qb_first) & 1);
+  dq_step(prev * M, buf ^ 1);
 }
 
 bool strides_ok(const int64_t* st, int n) {

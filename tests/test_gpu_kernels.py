@@ -731,3 +731,62 @@ def test_linear_rejects_bad_shapes():
     for args in bad:
         with pytest.raises(RuntimeError):
             _lib.call(*args)
+
+
+def _attention_float64(q, k, v, do, seg, scale):
+    """Dense masked attention and its gradients in float64 on the GPU, one (batch, head) at a time."""
+
+    B, H, S, D = q.shape
+    out = [torch.empty((B, H, S, D), dtype=torch.float64, device=q.device) for _ in range(4)]
+    at = torch.arange(S, device=q.device)
+    for b in range(B):
+        hide = (at[None, :] > at[:, None]) | (seg[b][None, :] != seg[b][:, None])
+        for h in range(H):
+            qh, kh, vh, gh = (t[b, h].double() for t in (q, k, v, do))
+            p = torch.softmax((qh @ kh.T * scale).masked_fill_(hide, -float("inf")), dim=-1)
+            o = p @ vh
+            ds = p * (gh @ vh.T - (gh * o).sum(-1, keepdim=True)) * scale
+            out[0][b, h], out[1][b, h], out[2][b, h], out[3][b, h] = o, ds @ kh, ds.T @ qh, p.T @ gh
+    return out
+
+
+@pytest.mark.parametrize("S,D,ids", [
+    (64, 64, "one"), (65, 64, "every"),          # a single document; a document per position
+    (321, 128, "blocks"), (1000, 64, "shuffled"),  # tile-aligned documents; ids in no order, with extreme values
+    (4160, 64, "returning"), (4200, 128, "returning"),  # past one group of 64 blocks, an id that comes back later
+])
+def test_attention_skips_only_hidden_blocks(S, D, ids):
+    """Segment ids in every order the entry point takes: blocks outside the
+    owned block's id range are skipped and uniform blocks run without the
+    compare, and the result stays the dense masked attention (the bound of
+    the other attention tests, 2e-2 max-abs, against float64)."""
+
+    from gptrig.kernels import flash_attention as fa
+
+    B, H = 2, 2
+    g = torch.Generator().manual_seed(S + D)
+    at = torch.arange(S)
+    rows = {
+        "one": [at * 0 + 7, at * 0 - 5],
+        "every": [at, -at],
+        "blocks": [at // 64, 10 - at // 128],
+        "shuffled": [torch.tensor([-2 ** 31, -1, 0, 2 ** 31 - 1])[torch.randint(0, 4, (S,), generator=g)],
+                     torch.randint(0, 3, (S // 100 + 1,), generator=g).repeat_interleave(100)[:S]],
+        "returning": [(at // 700) % 3, torch.where((at < 90) | (at > S - 70), 1, 2 + at // 1500)],
+    }[ids]
+    seg = torch.stack(rows).to(torch.int32).to(DEV)
+    q, k, v, do = (torch.randn((B, H, S, D), generator=g).to(torch.bfloat16).to(DEV) for _ in range(4))
+    scale = D ** -0.5
+    print(f"attention document blocks S={S} D={D} ids={ids}", flush=True)
+    o, lse = fa.flash_forward(q, k, v, seg, scale)
+    grads = fa.flash_backward(q, k, v, o, lse, do, seg, scale)
+    for name, got, want in zip(("o", "dq", "dk", "dv"), (o, *grads), _attention_float64(q, k, v, do, seg, scale)):
+        diff = (got.double() - want).abs()
+        peak = float(want.abs().max())
+        print(f"  {name} max-abs {float(diff.max()):.2e} of {peak:.2e}, norm {float(diff.norm()):.2e} of "
+              f"{float(want.norm()):.2e}", flush=True)
+        # Positions alone in their document have a score gradient of exactly 0,
+        # which float32 sums of 2D products of size ~1 leave at ~1e-6; where
+        # gradients reach `peak`, an ulp of bf16 is peak 2^-8.
+        assert float(diff.max()) <= 2e-2 * max(1.0, peak / 4)
+        assert float(diff.norm()) <= 1e-2 * float(want.norm()) + 1e-5 * want.numel() ** 0.5
