@@ -542,6 +542,61 @@ __global__ void __launch_bounds__(gemm::THREADS)
   gemm_f32_tile<AK, BKM>(A, B, M, N, k_begin, k_end, tm, tn, C, ldc, mode, colsum);
 }
 
+// Weight and bias gradients of linears that share their n tokens:
+//   dw[i] (f32 [rows_in, cols_out], +=) = X_i^T dY_i,  X_i bf16 [n, rows_in], dY_i bf16 [n, cols_out],
+//   db[i] (nullable, f32 [cols_out], +=) = column sums of dY_i, from the dY slabs the GEMM stages anyway.
+// One launch covers the tiles of every item.  An item alone has few tiles (a
+// d x d weight at d = 768: 9 for 256 CUs), so alone it needs a deep split
+// over the tokens, and each slice ends in 64 K float atomics, about 60 stages'
+// worth of time; the tiles of several items together fill the chip with a
+// shallow split or none (one writer per tile: a plain read-add-write).
+// Measured: the four linears of a block of width 512 over 8192 tokens, one
+// launch each 238 us a block, eight blocks in one launch 62 us a block; of
+// width 768 over 131072 tokens, 1789 us in four launches, 1638 in one.
+constexpr int kWgradMax = 32;  // items per launch (they travel as kernel arguments)
+struct WgradItem {
+  const bf16 *x, *dy;
+  float *dw, *db;
+  int rows_in, cols_out, first;  // first: the item's first workgroup
+};
+struct WgradGroup {
+  WgradItem item[kWgradMax];
+  int count, n, split;
+};
+
+__global__ void __launch_bounds__(gemm::THREADS) wgrad_kernel(WgradGroup g) {
+  int i = 0;
+  while (i + 1 < g.count && (int)blockIdx.x >= g.item[i + 1].first) ++i;  // uniform
+  const WgradItem w = g.item[i];
+  const int total = (i + 1 < g.count ? g.item[i + 1].first : (int)gridDim.x) - w.first;
+  int tm, tn, split, k_begin, k_end;
+  gemm::split_tile_coords((int)blockIdx.x - w.first, total, w.rows_in, w.cols_out, tm, tn, split);
+  split_range(g.n, g.split, split, k_begin, k_end);
+  // A(m = i, k = t) = X[t][i] (MN-major), B(k = t, n = j) = dY[t][j] (MN-major).
+  gemm_f32_tile<false, false>(Operand{w.x, w.rows_in}, Operand{w.dy, w.cols_out}, w.rows_in, w.cols_out, k_begin, k_end,
+                              tm, tn, w.dw, w.cols_out, g.split > 1 ? 2 : 1, w.db);
+}
+
+// The split over the tokens of a launch of `tiles` tiles: rounds of CUs, each
+// of a slice's stages (rounded up to the main loop's groups of four) plus its
+// epilogue, in stages: about 60 for the atomic add of a tile, 20 for a read-
+// add-write (measured in the FLCE gradient launches).
+int wgrad_split(unsigned tiles, int k_iters) {
+  const int cus = gemm::device_cus();
+  const int most = k_iters / 8 > 1 ? k_iters / 8 : 1;
+  int best = 1;
+  double best_cost = 1e300;
+  for (int s = 1; s <= most && s <= 256; ++s) {
+    const double stages = (double)((ceil_div(k_iters, s) + 3) & ~3) + (s > 1 ? 60.0 : 20.0);
+    const double cost = (double)ceil_div((int64_t)tiles * s, (int64_t)cus) * stages;
+    if (cost < best_cost * 0.999) {
+      best_cost = cost;
+      best = s;
+    }
+  }
+  return best;
+}
+
 // The two gradient GEMMs of the kept-softmax backward in one launch, so that
 // neither leaves the GPU part-empty while the other waits behind it:
 //   dh (+)= G W   A(m = token, k = v) = G^T blocked (MN-major), B = W [V][d] (MN-major),
@@ -1312,24 +1367,40 @@ int gptrig_flce_bwd_keep(const void* hidden, const void* weight, const int32_t* 
   return GPTRIG_OK;
 }
 
-// dW (f32 [rows_in, cols_out], += ) = X^T dY for X bf16 [n, rows_in], dY bf16 [n, cols_out],
-// and (db nullable) db (f32 [cols_out], += ) = column sums of dY: the weight and
-// bias gradients of rig/nn.py:55-56 (linear).  Split over the n tokens with
-// fp32 atomics so the skinny [d_in, d_out] output still fills the GPU; the
-// bias sums come from the dY slabs the GEMM already stages in LDS.
+// The weight and bias gradients of several linears over the same n tokens
+// (rig/nn.py:55-56) in grouped split-K launches; see wgrad_kernel.
+int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* stream) {
+  if (!items) return GPTRIG_E_NULL;
+  if (count < 0 || n <= 0) return GPTRIG_E_SHAPE;
+  for (int i = 0; i < count; ++i) {
+    const gptrig_wgrad& w = items[i];
+    if (!w.x || !w.dy || !w.dw) return GPTRIG_E_NULL;
+    if (w.rows_in <= 0 || w.cols_out <= 0 || w.rows_in % 8 || w.cols_out % 8) return GPTRIG_E_SHAPE;
+    if (((uintptr_t)w.x | (uintptr_t)w.dy) & 15) return GPTRIG_E_SHAPE;
+  }
+  for (int at = 0; at < count; at += kWgradMax) {
+    WgradGroup g{};
+    g.count = count - at < kWgradMax ? count - at : kWgradMax;
+    g.n = n;
+    unsigned tiles = 0;
+    for (int i = 0; i < g.count; ++i) tiles += tiles_of(items[at + i].rows_in, items[at + i].cols_out);
+    g.split = wgrad_split(tiles, ceil_div(n, gemm::BK));
+    unsigned first = 0;
+    for (int i = 0; i < g.count; ++i) {
+      const gptrig_wgrad& w = items[at + i];
+      g.item[i] = WgradItem{(const bf16*)w.x, (const bf16*)w.dy, w.dw, w.db, w.rows_in, w.cols_out, (int)first};
+      first += tiles_of(w.rows_in, w.cols_out) * (unsigned)g.split;
+    }
+    wgrad_kernel<<<first, gemm::THREADS, 0, (hipStream_t)stream>>>(g);
+    GPTRIG_CHECK_LAUNCH();
+  }
+  return GPTRIG_OK;
+}
+
 int gptrig_weight_grad(const void* x, const void* dy, float* dw, float* db, int n, int rows_in, int cols_out,
                        void* stream) {
-  if (!x || !dy || !dw) return GPTRIG_E_NULL;
-  if (n <= 0 || rows_in <= 0 || cols_out <= 0 || rows_in % 8 || cols_out % 8) return GPTRIG_E_SHAPE;
-  if (((uintptr_t)x | (uintptr_t)dy) & 15) return GPTRIG_E_SHAPE;
-  const unsigned tiles = tiles_of(rows_in, cols_out);
-  const int split = gemm::choose_split(tiles, ceil_div(n, gemm::BK));
-  // A(m = i, k = t) = X[t][i] (MN-major), B(k = t, n = j) = dY[t][j] (MN-major).
-  Operand A{(const bf16*)x, rows_in}, B{(const bf16*)dy, cols_out};
-  gemm_f32_kernel<false, false><<<tiles * split, gemm::THREADS, 0, (hipStream_t)stream>>>(A, B, rows_in, cols_out, n,
-                                                                                         split, dw, cols_out, 2, db);
-  GPTRIG_CHECK_LAUNCH();
-  return GPTRIG_OK;
+  const gptrig_wgrad item{x, dy, dw, db, rows_in, cols_out};
+  return gptrig_weight_grads(&item, 1, n, stream);
 }
 
 }  // extern "C"

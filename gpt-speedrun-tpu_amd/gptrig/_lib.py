@@ -21,6 +21,13 @@ L = c_int64
 F = c_float
 Z = c_size_t
 
+
+class WGrad(ctypes.Structure):
+    """``gptrig_wgrad`` of ``include/gptrig.h``."""
+
+    _fields_ = [("x", P), ("dy", P), ("dw", P), ("db", P), ("rows_in", I), ("cols_out", I)]
+
+
 # name -> (restype, argtypes)
 SIGNATURES: dict[str, tuple] = {
     "gptrig_version": (c_char_p, []),
@@ -49,6 +56,7 @@ SIGNATURES: dict[str, tuple] = {
     "gptrig_rmsnorm_bwd": (I, [P, P, P, P, P, P, P, I, P, Z, I, I, P]),
     "gptrig_bias_grad": (I, [P, I, I, P, P]),
     "gptrig_weight_grad": (I, [P, P, P, P, I, I, I, P]),
+    "gptrig_weight_grads": (I, [ctypes.POINTER(WGrad), I, I, P]),
     "gptrig_linear": (I, [P, L, P, L, I, P, P, L, I, I, I, P]),
     "gptrig_linear_gelu": (I, [P, L, P, L, I, P, P, P, L, I, I, I, P]),
     "gptrig_linear_rope": (I, [P, L, P, L, I, P, P, L, I, I, I, P, P, I, I, I, P]),

@@ -300,6 +300,16 @@ class GPTTrainer:
         # marks the point; the step's optimizer update waits for the stream.
         self.wgrad_stream = torch.cuda.Stream(device=self.device)
         self._layer_ready = [torch.cuda.Event() for _ in range(config.layers)]
+        # Layers per weight-gradient launch: enough that each of the 256 CUs has
+        # about 512 stages (32 tokens of a 256 x 256 tile) to run, several times
+        # the epilogue of a split launch: all eight layers of the 60M-class model
+        # at its 8192 tokens per step (8.0 -> 6.7 ms a step).  Where one layer has
+        # that much (the 125M model at 131072 tokens) its linears are launched one
+        # by one: grouped they are 8% faster alone (1638 against 1789 us a layer)
+        # but the step, whose clock the matrix cores' power sets, is 0.3% slower
+        # with their longer workgroups beside the backward of the layers below.
+        tiles = sum(-(-a // 256) * -(-b // 256) for a, b in widths.values())
+        self.wgrad_layers = max(1, -(-512 * 256 // (tiles * -(-T // 32))))
 
     # -- helpers -----------------------------------------------------------------
     def _workspace(self, name: str, nbytes: int) -> torch.Tensor:
@@ -620,13 +630,21 @@ class GPTTrainer:
         _lib.call("gptrig_embedding_bwd", tok.data_ptr(), dx.data_ptr(), A.grad("token_embedding").data_ptr(), N, d,
                   c.vocab_size, stream)
 
-    def _weight_grad(self, prefix: str, inp: torch.Tensor, dout: torch.Tensor) -> None:
-        """dW += inp^T dout and db += sum_rows(dout), both float32."""
+    def _weight_grads(self, layers) -> None:
+        """dW += inp^T dout and db += sum_rows(dout), both float32, for the block linears of ``layers``."""
 
         A = self.arena
-        n, rows_in = inp.shape
-        _lib.call("gptrig_weight_grad", inp.data_ptr(), dout.data_ptr(), A.grad(prefix + "_w").data_ptr(),
-                  A.grad(prefix + "_b").data_ptr(), n, rows_in, dout.shape[1], _lib.stream())
+        tokens = self.config.batch_size * self.config.seq_len
+        items = (_lib.WGrad * (len(layers) * len(self.linears)))()
+        for j, (i, name) in enumerate((i, name) for i in layers for name in self.linears):
+            inp, dout, prefix = self.lin_in[i][name], self.lin_dout[i][name], f"blocks/{i}/{name}"
+            items[j] = _lib.WGrad(inp.data_ptr(), dout.data_ptr(), A.grad(prefix + "_w").data_ptr(),
+                                  A.grad(prefix + "_b").data_ptr(), inp.shape[1], dout.shape[1])
+        if len(layers) > 1:
+            _lib.call("gptrig_weight_grads", items, len(items), tokens, _lib.stream())
+            return
+        for w in items:
+            _lib.call("gptrig_weight_grad", w.x, w.dy, w.dw, w.db, tokens, w.rows_in, w.cols_out, _lib.stream())
 
     # -- the step ----------------------------------------------------------------------
     def train_step(self, x: torch.Tensor, y: torch.Tensor) -> None:
@@ -656,11 +674,11 @@ class GPTTrainer:
         # optimizer update.
         main = torch.cuda.current_stream(self.device)
         side = self.wgrad_stream
-        for i in reversed(range(c.layers)):
-            side.wait_event(self._layer_ready[i])
+        for top in range(c.layers - 1, -1, -self.wgrad_layers):
+            layers = range(top, max(top - self.wgrad_layers, -1), -1)
+            side.wait_event(self._layer_ready[layers[-1]])
             with torch.cuda.stream(side):
-                for name in self.linears:
-                    self._weight_grad(f"blocks/{i}/{name}", self.lin_in[i][name], self.lin_dout[i][name])
+                self._weight_grads(layers)
         main.wait_stream(side)
         self.step_count += 1
         step = self.step_count

@@ -205,6 +205,17 @@ int gptrig_rmsnorm_bwd(const void* dy, const void* x, const void* scale, const f
  * fp32 atomics. */
 int gptrig_weight_grad(const void* x, const void* dy, float* dw, float* db, int n, int rows_in, int cols_out,
                        void* stream);
+/* The same for several linears over the same n tokens, in one launch per 32
+ * items (items is host memory, read before the call returns).  The dw and db
+ * of different items must not overlap. */
+typedef struct {
+  const void* x;  /* bf16 [n, rows_in] */
+  const void* dy; /* bf16 [n, cols_out] */
+  float* dw;      /* f32 [rows_in, cols_out], += */
+  float* db;      /* f32 [cols_out], +=, or NULL */
+  int rows_in, cols_out;
+} gptrig_wgrad;
+int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* stream);
 
 /* Bias gradient of rig/nn.py:55-56 (linear): db f32 [cols] += sum over rows of
  * dy bf16 [rows, cols] (cols % 8 == 0). */

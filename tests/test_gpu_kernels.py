@@ -790,3 +790,51 @@ def test_attention_skips_only_hidden_blocks(S, D, ids):
         # gradients reach `peak`, an ulp of bf16 is peak 2^-8.
         assert float(diff.max()) <= 2e-2 * max(1.0, peak / 4)
         assert float(diff.norm()) <= 1e-2 * float(want.norm()) + 1e-5 * want.numel() ** 0.5
+
+
+@pytest.mark.parametrize("n,shapes", [
+    (1, [(8, 8)]),                                           # one token, one 8 x 8 corner of a tile
+    (40, [(256, 256), (264, 8), (8, 520)]),                  # whole tile, one row block past it, a ragged row of tiles
+    (4096, [(64, 192), (64, 64), (64, 256), (256, 64)]),     # split over the tokens (atomics), uneven last slice
+    (1000, [(512, 1536), (512, 512), (512, 2048), (2048, 512)] * 9),  # 36 items: two launches, no split
+])
+def test_grouped_weight_gradients(n, shapes):
+    """Every item of a grouped launch adds its own X^T dY (and the column sums
+    where asked) to its own gradient, bit-equal inputs aside from the float32
+    summation order.
+
+    Bound: bf16 products are exact in float32 and a sum of n of them rounds at
+    most n times: error <= n 2^-24 of the sum of magnitudes (and one rounding
+    of the accumulated total)."""
+
+    from gptrig import _lib
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV)  # noqa: E731
+    data, items = [], (_lib.WGrad * len(shapes))()
+    for j, (a, b) in enumerate(shapes):
+        x, dy, dw, db = rnd(n, a).bfloat16(), rnd(n, b).bfloat16(), rnd(a, b), rnd(b)
+        data.append((x, dy, dw.clone(), db.clone(), dw, db))
+        items[j] = _lib.WGrad(x.data_ptr(), dy.data_ptr(), dw.data_ptr(), None if j % 3 == 1 else db.data_ptr(), a, b)
+    print(f"grouped weight gradients n={n} items={len(shapes)}", flush=True)
+    _lib.call("gptrig_weight_grads", items, len(shapes), n, _lib.stream())
+    torch.cuda.synchronize()
+    worst = 0.0
+    for j, (x, dy, dw0, db0, dw, db) in enumerate(data):
+        x64, dy64 = x.double(), dy.double()
+        eps = (n + 2) * 2.0 ** -24
+        bound = eps * (x64.abs().T @ dy64.abs() + dw0.double().abs())
+        worst = max(worst, float(((dw.double() - dw0.double() - x64.T @ dy64).abs() / bound).max()))
+        if j % 3 == 1:
+            assert torch.equal(db, db0)
+        else:
+            bound = eps * (dy64.abs().sum(0) + db0.double().abs())
+            worst = max(worst, float(((db.double() - db0.double() - dy64.sum(0)).abs() / bound).max()))
+    print(f"  error / bound {worst:.3f}", flush=True)
+    assert worst <= 1
+    _lib.call("gptrig_weight_grads", items, 0, n, _lib.stream())  # no items: nothing to do
+    with pytest.raises(RuntimeError):
+        _lib.call("gptrig_weight_grads", items, 1, 0, _lib.stream())
+    items[0].cols_out = 12
+    with pytest.raises(RuntimeError):
+        _lib.call("gptrig_weight_grads", items, 1, n, _lib.stream())
