@@ -10,7 +10,7 @@
 //   ballots in slot order), rows = order / top_k, position = order^-1.
 //
 // The routed MLP around it (:1275-1293):
-//   router_logits   fp32 x @ router_w (one wave per token, weights in LDS);
+//   router_logits   fp32 x @ router_w (split weights on the matrix cores);
 //   moe_gather_rows grouped = flat[rows] (token rows in bucket order);
 //   moe_gmm         grouped GEMM over the expert buckets on the MFMA GEMM core,
 //                   epilogue bias (+ GELU, or x GELU' for the backward);
@@ -18,8 +18,9 @@
 //                   of bf16(out * bf16(gate)) -- the .at[rows].add rounding;
 //   moe_stats       mean probability, load, (entropy, top-1 gate, logit RMS);
 // and their backward: combine_bwd, moe_gmm_dw (per-expert weight + bias
-// gradients, split-K fp32 atomics), gather_bwd (the VJP of flat[rows]) and
-// router_bwd (gate/probability softmax VJPs, dx and d router_w).
+// gradients, split-K fp32 atomics) and router_bwd (gate / probability softmax
+// VJPs, dx and d router_w, with the VJP of flat[rows] fused in or, for the
+// separate entry points, after gather_bwd).
 #include "common.h"
 #include "epilogue.h"
 
@@ -28,45 +29,81 @@
 namespace {
 
 constexpr int kMaxExperts = 64;
+constexpr int kFewTopK = 4;
 
+// EP: E rounded up to 4, 8, 16 or 64; the row is held in registers, loaded
+// once (re-reading it for each of the passes cost a memory latency per value:
+// 9.0 -> 4.6 us at 200 tokens, 9.4 -> 5.5 at 32768, 8 experts).
+template <int EP>
 __global__ void route_topk_kernel(const float* __restrict__ logits, float* __restrict__ probs,
                                   int32_t* __restrict__ chosen, float* __restrict__ gate, int T, int E, int k) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= T) return;
-  const float* row = logits + (size_t)t * E;
+  float row[EP];
+#pragma unroll
+  for (int e = 0; e < EP; ++e) row[e] = logits[(size_t)t * E + min(e, E - 1)];
   float mx = -INFINITY;
-  for (int e = 0; e < E; ++e) mx = fmaxf(mx, row[e]);
+#pragma unroll
+  for (int e = 0; e < EP; ++e)
+    if (e < E) mx = fmaxf(mx, row[e]);
   if (probs) {
-    float s = 0.f;
-    for (int e = 0; e < E; ++e) s += expf(row[e] - mx);
-    for (int e = 0; e < E; ++e) probs[(size_t)t * E + e] = expf(row[e] - mx) / s;
+    float ex[EP], s = 0.f;
+#pragma unroll
+    for (int e = 0; e < EP; ++e) {
+      ex[e] = expf(row[e] - mx);
+      if (e < E) s += ex[e];
+    }
+#pragma unroll
+    for (int e = 0; e < EP; ++e)
+      if (e < E) probs[(size_t)t * E + e] = ex[e] / s;
   }
+  // One pass per chosen expert.
   uint64_t taken = 0;
-  float vals[kMaxExperts];
-  int idx[kMaxExperts];
-  for (int j = 0; j < k; ++j) {
+  auto pick = [&](float& bv) {
     int best = -1;
-    float bv = 0.f;
-    for (int e = 0; e < E; ++e) {
-      if (taken >> e & 1) continue;
-      const float x = row[e];
+    bv = 0.f;
+#pragma unroll
+    for (int e = 0; e < EP; ++e) {
       // Strictly greater keeps the lower index on ties; NaN never wins.
-      if (best < 0 || x > bv) {
+      if (e < E && !(taken >> e & 1) && (best < 0 || row[e] > bv)) {
         best = e;
-        bv = x;
+        bv = row[e];
       }
     }
     taken |= 1ull << best;
-    vals[j] = bv;
-    idx[j] = best;
-  }
-  float gm = vals[0];
-  for (int j = 1; j < k; ++j) gm = fmaxf(gm, vals[j]);
-  float gs = 0.f;
-  for (int j = 0; j < k; ++j) gs += expf(vals[j] - gm);
-  for (int j = 0; j < k; ++j) {
-    chosen[(size_t)t * k + j] = idx[j];
-    gate[(size_t)t * k + j] = expf(vals[j] - gm) / gs;
+    return best;
+  };
+  int32_t* const ch = chosen + (size_t)t * k;
+  float* const gt = gate + (size_t)t * k;
+  if (k <= kFewTopK) {  // the chosen logits stay in registers
+    float vals[kFewTopK], gm = 0.f, gs = 0.f;
+#pragma unroll
+    for (int j = 0; j < kFewTopK; ++j) {
+      if (j >= k) break;
+      ch[j] = pick(vals[j]);
+      gm = j == 0 ? vals[0] : fmaxf(gm, vals[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < kFewTopK; ++j) {
+      if (j >= k) break;
+      vals[j] = expf(vals[j] - gm);
+      gs += vals[j];
+    }
+#pragma unroll
+    for (int j = 0; j < kFewTopK; ++j) {
+      if (j >= k) break;
+      gt[j] = vals[j] / gs;
+    }
+  } else {  // ... or wait in the gate row
+    float gm = 0.f, gs = 0.f;
+    for (int j = 0; j < k; ++j) {
+      float v;
+      ch[j] = pick(v);
+      gt[j] = v;
+      gm = j == 0 ? v : fmaxf(gm, v);
+    }
+    for (int j = 0; j < k; ++j) gs += expf(gt[j] - gm);
+    for (int j = 0; j < k; ++j) gt[j] = expf(gt[j] - gm) / gs;
   }
 }
 
@@ -139,74 +176,80 @@ __global__ void __launch_bounds__(kSortBlock) route_place_kernel(const int32_t* 
 }
 
 // ---------------------------------------------------------------------------
-// Router logits (:1259-1264): logits[t][e] = sum_d f32(x[t][d]) * w[d][e].
-// A wave takes 8 tokens at a time: lane = 8 token + g reads the token's
-// 16-byte chunks g, g + 8, ... (each 8-lane group reads 128 contiguous
-// bytes of one row), multiplies them by w rows from LDS, and the 8 lanes of
-// a token add their partial logits with three xor exchanges.
+// Router logits (:1259-1264): logits[t][e] = sum_d f32(x[t][d]) * w[d][e] on
+// the bf16 matrix cores without losing a bit of an operand: x is bf16 already
+// and each float32 weight is split exactly into three bf16 pieces (8
+// significant bits each, by truncation), so a logit is a float32 sum of exact
+// products, three MFMAs per 32 columns.  A wave takes 16 tokens
+// (v_mfma_f32_16x16x32_bf16, columns = experts, the columns past E unused);
+// each lane reads 16 bytes of its token per step straight from memory and the
+// weight pieces from LDS.  Bound by reading x once.
+// Measured: 32768 tokens x 768, 8 experts 20 us (50 MB of x) against 57 us
+// with float32 multiply-adds and 8 lanes per token; 200 x 512 9 against 25.
 // ---------------------------------------------------------------------------
 constexpr int kMaxRouterExperts = 16;
-constexpr int kRouterTokens = 16;  // tokens per wave (two passes of 8)
-constexpr int kMaxRouterWidth = 4096;
+constexpr int kRouterWaves = 4;
 
-// 8 bf16 of row x[t] from column d (d < D), zeros past D.
-__device__ __forceinline__ void load_x8(const bf16* __restrict__ row, int d, int D, float (&xv)[8]) {
-  if (d + 8 <= D && ((D & 7) == 0)) {
-    const bf16x8 v = *reinterpret_cast<const bf16x8*>(row + d);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) xv[j] = (float)v[j];
+// Elements per LDS row of one expert's weight pieces: whole steps of 32 and 8
+// more, so 16 rows read at one column cover all banks.
+__host__ __device__ inline int router_row(int D) { return (D + 31) / 32 * 32 + 8; }
+
+// 8 bf16 of row x from column d, zeros past D.
+template <bool kVec>
+__device__ __forceinline__ bf16x8 load_x8(const bf16* __restrict__ row, int d, int D) {
+  if constexpr (kVec) {
+    return d < D ? *reinterpret_cast<const bf16x8*>(row + d) : bf16x8{};
   } else {
+    bf16x8 v;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) xv[j] = d + j < D ? (float)row[d + j] : 0.f;
+    for (int j = 0; j < 8; ++j) v[j] = d + j < D ? row[d + j] : (bf16)0.f;
+    return v;
   }
 }
 
-template <int EP>
-__global__ void __launch_bounds__(256) router_logits_kernel(const bf16* __restrict__ x, const float* __restrict__ w,
-                                                            float* __restrict__ logits, int T, int D, int E) {
-  extern __shared__ float wsh[];  // [D][EP], zero past E
-  for (int i = threadIdx.x; i < D * EP; i += blockDim.x) {
-    const int d = i / EP, e = i % EP;
-    wsh[i] = e < E ? w[(size_t)d * E + e] : 0.f;
+template <bool kVec>
+__global__ void __launch_bounds__(64 * kRouterWaves)
+    router_logits_kernel(const bf16* __restrict__ x, const float* __restrict__ w, float* __restrict__ logits, int T,
+                         int D, int E) {
+  extern __shared__ __attribute__((aligned(16))) bf16 wsh[];  // [3][E][router_row(D)]
+  const int R = router_row(D);
+  for (int i = threadIdx.x; i < E * R; i += blockDim.x) {
+    const int d = i / E, e = i % E;  // (consecutive threads read consecutive weights)
+    const float v = d < D ? w[(size_t)d * E + e] : 0.f;
+    const uint32_t b0 = __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u;
+    const float r1 = v - __builtin_bit_cast(float, b0);  // exact
+    const uint32_t b1 = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
+    const float r2 = r1 - __builtin_bit_cast(float, b1);  // exact, 8 bits
+    wsh[e * R + d] = (bf16)__builtin_bit_cast(float, b0);
+    wsh[(E + e) * R + d] = (bf16)__builtin_bit_cast(float, b1);
+    wsh[(2 * E + e) * R + d] = (bf16)r2;
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tok = lane >> 3, g = lane & 7;
-  const int wt0 = (blockIdx.x * 4 + wave) * kRouterTokens;
-#pragma unroll 1
-  for (int pass = 0; pass < kRouterTokens / 8; ++pass) {
-    const int t = wt0 + 8 * pass + tok;
-    float acc[EP];
+  const int l16 = lane & 15, q = lane >> 4;
+  const int t0 = (blockIdx.x * kRouterWaves + wave) * 16;
+  const bf16* row = x + (size_t)min(t0 + l16, T - 1) * D;
+  const bf16* wr = wsh + min(l16, E - 1) * R + 8 * q;
+  f32x4 acc[3] = {f32x4{}, f32x4{}, f32x4{}};
+  constexpr int kAhead = 8;  // steps whose loads are in flight together
+  for (int d0 = 0; d0 < D; d0 += 32 * kAhead) {
+    bf16x8 xv[kAhead];
 #pragma unroll
-    for (int e = 0; e < EP; ++e) acc[e] = 0.f;
-    if (t < T) {
-      const bf16* row = x + (size_t)t * D;
-      for (int d = 8 * g; d < D; d += 64) {
-        float xv[8];
-        load_x8(row, d, D, xv);
+    for (int j = 0; j < kAhead; ++j) xv[j] = load_x8<kVec>(row, d0 + 32 * j + 8 * q, D);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          if (d + j >= D) break;
-          const float* wr = wsh + (d + j) * EP;
+    for (int j = 0; j < kAhead; ++j) {
+      const int d = d0 + 32 * j;
+      if (d >= D) break;  // uniform
 #pragma unroll
-          for (int e4 = 0; e4 < EP; e4 += 4) {
-            const f32x4 w4 = *reinterpret_cast<const f32x4*>(wr + e4);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc[e4 + u] = fmaf(xv[j], w4[u], acc[e4 + u]);
-          }
-        }
-      }
+      for (int p = 0; p < 3; ++p)
+        acc[p] = mfma16(xv[j], *reinterpret_cast<const bf16x8*>(wr + p * E * R + d), acc[p]);
     }
+  }
+  if (l16 < E) {
 #pragma unroll
-    for (int e = 0; e < EP; ++e) {
-      acc[e] += __shfl_xor(acc[e], 1);
-      acc[e] += __shfl_xor(acc[e], 2);
-      acc[e] += __shfl_xor(acc[e], 4);
-    }
-    if (t < T) {
-#pragma unroll
-      for (int e = 0; e < EP; ++e)
-        if (e % 8 == g && e < E) logits[(size_t)t * E + e] = acc[e];
+    for (int i = 0; i < 4; ++i) {
+      const int t = t0 + 4 * q + i;  // lane: expert l16, tokens 4 q .. 4 q + 3
+      if (t < T) logits[(size_t)t * E + l16] = acc[2][i] + acc[1][i] + acc[0][i];
     }
   }
 }
@@ -357,24 +400,49 @@ __device__ __forceinline__ void token_slots(const int32_t* __restrict__ position
 
 // combined[t] = bf16 sum, in bucket order, of bf16(out[p] * bf16(gate)):
 // weighted = out * gate[order].astype(bf16); zeros.at[rows].add(weighted).
+// K = top_k where it is 1 or 2 (0: any): every row of a token is then loaded
+// before the first is used (32768 tokens x 768, top 2: 41 -> 27 us).
+template <int K>
 __global__ void __launch_bounds__(256) moe_combine_kernel(const bf16* __restrict__ out, const int32_t* __restrict__ position,
                                                           const float* __restrict__ gate, bf16* __restrict__ combined,
-                                                          int T, int D, int k) {
+                                                          int T, int D, int k_any) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= T) return;
   const int lane = threadIdx.x & 63;
+  const int k = K ? K : k_any;
   int p[kMaxTopK];
   float g[kMaxTopK];
   token_slots(position, gate, t, k, p, g);
-  for (int c = lane * 4; c < D; c += 256) {
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int j = 0; j < k; ++j) {
-      const bf16x4 v = *reinterpret_cast<const bf16x4*>(out + (size_t)p[j] * D + c);
+  constexpr int kU = K ? 4 : 1;  // chunks of 4 columns per lane in flight
+  for (int c0 = lane * 4; c0 < D; c0 += 256 * kU) {
+    float acc[kU][4] = {};
+    if constexpr (K > 0) {
+      bf16x4 v[K][kU];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = (float)(bf16)(acc[q] + (float)(bf16)((float)v[q] * g[j]));
+      for (int j = 0; j < K; ++j)
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+          v[j][u] = c0 + 256 * u < D ? *reinterpret_cast<const bf16x4*>(out + (size_t)p[j] * D + c0 + 256 * u) : bf16x4{};
+#pragma unroll
+      for (int j = 0; j < K; ++j)
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            acc[u][q] = (float)(bf16)(acc[u][q] + (float)(bf16)((float)v[j][u][q] * g[j]));
+    } else {
+      for (int j = 0; j < k; ++j) {
+        const bf16x4 v = *reinterpret_cast<const bf16x4*>(out + (size_t)p[j] * D + c0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[0][q] = (float)(bf16)(acc[0][q] + (float)(bf16)((float)v[q] * g[j]));
+      }
     }
-    bf16x4 o = {(bf16)acc[0], (bf16)acc[1], (bf16)acc[2], (bf16)acc[3]};
-    *reinterpret_cast<bf16x4*>(combined + (size_t)t * D + c) = o;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (c0 + 256 * u >= D) break;
+      bf16x4 o = {(bf16)acc[u][0], (bf16)acc[u][1], (bf16)acc[u][2], (bf16)acc[u][3]};
+      *reinterpret_cast<bf16x4*>(combined + (size_t)t * D + c0 + 256 * u) = o;
+    }
   }
 }
 
@@ -506,62 +574,51 @@ __global__ void stats_finalize_kernel(const int32_t* __restrict__ counts, int T,
 //   dlogits[e] = probs[e] * (dprobs[e] - sum_i probs[i] dprobs[i]) + sum_{j: chosen[j]=e} dchosen[j]
 //   dx[t][d]   = bf16(dx[t][d] + bf16(sum_e dlogits[e] w[d][e]))       (in place)
 //   dw[d][e]  += sum_t f32(x[t][d]) dlogits[e]
-// A workgroup takes a tile of kRouterBwdCols width columns x
-// kRouterBwdTokens tokens.  Its threads first turn each token's gate and
+// A workgroup takes kRouterBwdCols width columns and a run of tokens, in
+// tiles of kRouterBwdTokens.  Its threads first turn each token's gate and
 // probability cotangents into dlogits (LDS); then thread (token lane tl,
-// chunk c) walks tokens tl, tl + 32, ... for the 8 columns 8 c .. 8 c + 7 of
-// the tile: dx[t][chunk] += bf16(dlogits[t] @ w[chunk]^T) (a 16-byte
-// read-modify-write; the 8 chunk threads of a token cover 128 contiguous
-// bytes) and the chunk's dw partial f32 [8][EP] in registers.  The 32 token
-// lanes' partials are summed with xor exchanges and through LDS, and each
-// workgroup adds one value per (column, expert) to dw with an atomic.
-constexpr int kRouterBwdTokens = 1024;
+// chunk c) walks tokens tl, tl + 32, ... of the tile for the 8 columns 8 c ..
+// 8 c + 7: dx[t][chunk] gets bf16(dlogits[t] @ w[chunk]^T) added and the
+// chunk's dw partial f32 [8][EP] grows in registers.  After the last tile the
+// 32 token lanes' partials are summed with xor exchanges and through LDS, and
+// the workgroup adds one value per (column, expert) to dw with an atomic.  The
+// grid is about one workgroup per CU: every workgroup of a column tile adds to
+// the same few cache lines, and those adds run one after the other (128
+// workgroups per column tile: 99 us, 21: 67 us at 32768 tokens x 768; about 0.7
+// us per workgroup of a column tile).
+// kGather >= 0: the row the router's part is added to is not read from dx but
+// is the VJP of grouped = flat[rows], the bf16 sum of the token's rows of
+// dgrouped in bucket order (moe_gather_bwd_kernel's), so dx is written once and
+// never read: at 32768 tokens x 768, top 2, 67 us against 36 + 81 us for the
+// two passes.  kGather is top_k where it is 1 or 2 (0: any), so the loops over
+// a token's slots unroll and their loads go out together; four tokens' loads
+// are in flight per thread.
+constexpr int kRouterBwdTokens = 256;
 constexpr int kRouterBwdCols = 64;
 
-template <int EP>
+template <int EP, int kGather>
 __global__ void __launch_bounds__(256) router_bwd_kernel(const bf16* __restrict__ x, const float* __restrict__ w,
                                                          const float* __restrict__ probs, const int32_t* __restrict__ chosen,
                                                          const float* __restrict__ gate, const float* __restrict__ dgate,
                                                          const float* __restrict__ dmean_probability,
-                                                         bf16* __restrict__ dx, float* __restrict__ dw, int T, int D,
-                                                         int E, int k) {
+                                                         const bf16* __restrict__ dgrouped,
+                                                         const int32_t* __restrict__ position, bf16* __restrict__ dx,
+                                                         float* __restrict__ dw, int T, int D, int E, int k_any,
+                                                         int run) {
+  constexpr bool kFused = kGather >= 0;
+  const int k = kGather > 0 ? kGather : k_any;
   __shared__ __attribute__((aligned(16))) float dl_s[kRouterBwdTokens][EP];
+  __shared__ int pos_s[kFused ? kRouterBwdTokens : 1][kMaxTopK];
   __shared__ float red[4][kRouterBwdCols][EP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int tb = blockIdx.y * kRouterBwdTokens;
-  const int col0 = blockIdx.x * kRouterBwdCols;
-  for (int i = tid; i < kRouterBwdTokens; i += blockDim.x) {
-    const int t = tb + i;
-    float dl[EP];
-#pragma unroll
-    for (int e = 0; e < EP; ++e) dl[e] = 0.f;
-    if (t < T) {
-      if (dmean_probability) {
-        float pd = 0.f;
-#pragma unroll
-        for (int e = 0; e < EP; ++e)
-          if (e < E) pd += probs[(size_t)t * E + e] * (dmean_probability[e] / T);
-#pragma unroll
-        for (int e = 0; e < EP; ++e)
-          if (e < E) dl[e] = probs[(size_t)t * E + e] * (dmean_probability[e] / T - pd);
-      }
-      float gd = 0.f;
-      for (int j = 0; j < k; ++j) gd += gate[(size_t)t * k + j] * dgate[(size_t)t * k + j];
-      for (int j = 0; j < k; ++j) {
-        const float dc = gate[(size_t)t * k + j] * (dgate[(size_t)t * k + j] - gd);
-        const int ce = chosen[(size_t)t * k + j];
-#pragma unroll
-        for (int e = 0; e < EP; ++e)
-          if (e == ce) dl[e] += dc;
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < EP; ++e) dl_s[i][e] = dl[e];
-  }
-  __syncthreads();
+  // Column tiles fastest: the workgroups of one run of tokens run together and
+  // share its rows' cache lines.
+  const int ncol = (D + kRouterBwdCols - 1) / kRouterBwdCols;
+  const int col0 = blockIdx.x % ncol * kRouterBwdCols;
+  const int t_begin = (int)(blockIdx.x / ncol) * run, t_end = min(T, t_begin + run);
   const int c = tid & 7, tl = tid >> 3;  // chunk of the tile, token lane (0 .. 31)
   const int d0 = col0 + 8 * c;
-  const bool vec = (D & 7) == 0 && d0 + 8 <= D;
+  const bool vec = (D & 7) == 0 && d0 + 8 <= D;  // (kFused: D is a multiple of 8)
   float wc[8][EP], dwp[8][EP];
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -570,52 +627,124 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const bf16* __restrict_
       wc[j][e] = (d0 + j < D && e < E) ? w[(size_t)(d0 + j) * E + e] : 0.f;
       dwp[j][e] = 0.f;
     }
-  if (d0 < D) {
-    for (int i = tl; i < kRouterBwdTokens; i += 32) {
-      const int t = tb + i;
-      if (t >= T) break;
-      const bf16* xrow = x + (size_t)t * D + d0;
-      bf16* drow = dx + (size_t)t * D + d0;
-      float xv[8], old[8];
-      if (vec) {
-        const bf16x8 xx = *reinterpret_cast<const bf16x8*>(xrow);
-        const bf16x8 dd = *reinterpret_cast<const bf16x8*>(drow);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          xv[j] = (float)xx[j];
-          old[j] = (float)dd[j];
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          xv[j] = d0 + j < D ? (float)xrow[j] : 0.f;
-          old[j] = d0 + j < D ? (float)drow[j] : 0.f;
-        }
-      }
+  for (int tb = t_begin; tb < t_end; tb += kRouterBwdTokens) {
+    __syncthreads();  // the previous tile's dlogits are read
+    {
+      static_assert(kRouterBwdTokens == 256, "one token per thread");
+      const int t = tb + tid;
       float dl[EP];
 #pragma unroll
-      for (int e4 = 0; e4 < EP; e4 += 4) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(&dl_s[i][e4]);
+      for (int e = 0; e < EP; ++e) dl[e] = 0.f;
+      if (t < t_end) {
+        if (dmean_probability) {
+          float pd = 0.f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) dl[e4 + u] = v[u];
-      }
-      bf16x8 o;
+          for (int e = 0; e < EP; ++e)
+            if (e < E) pd += probs[(size_t)t * E + e] * (dmean_probability[e] / T);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float sj = 0.f;
-#pragma unroll
-        for (int e = 0; e < EP; ++e) {
-          sj = fmaf(dl[e], wc[j][e], sj);
-          dwp[j][e] = fmaf(xv[j], dl[e], dwp[j][e]);
+          for (int e = 0; e < EP; ++e)
+            if (e < E) dl[e] = probs[(size_t)t * E + e] * (dmean_probability[e] / T - pd);
         }
-        o[j] = (bf16)(old[j] + (float)(bf16)sj);
-      }
-      if (vec) {
-        *reinterpret_cast<bf16x8*>(drow) = o;
-      } else {
+        float gd = 0.f;
+        for (int j = 0; j < k; ++j) gd += gate[(size_t)t * k + j] * dgate[(size_t)t * k + j];
+        for (int j = 0; j < k; ++j) {
+          const float dc = gate[(size_t)t * k + j] * (dgate[(size_t)t * k + j] - gd);
+          const int ce = chosen[(size_t)t * k + j];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (d0 + j < D) drow[j] = o[j];
+          for (int e = 0; e < EP; ++e)
+            if (e == ce) dl[e] += dc;
+        }
+        if constexpr (kFused) {
+          int p[kMaxTopK];
+          float g[kMaxTopK];
+          token_slots(position, nullptr, t, k, p, g);
+          for (int j = 0; j < k; ++j) pos_s[tid][j] = p[j];
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < EP; ++e) dl_s[tid][e] = dl[e];
+    }
+    __syncthreads();
+    constexpr int kU = EP <= 8 ? 4 : 2;  // tokens in flight
+    if (d0 < D) {
+      for (int i0 = tl; i0 < kRouterBwdTokens; i0 += 32 * kU) {
+        if (tb + i0 >= t_end) break;
+        bf16x8 xx[kU], old[kU];
+        // (Tokens past the run read its last token's rows; their dlogits are zero and
+        // nothing of them is stored.)
+        int ts[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) ts[u] = min(tb + i0 + 32 * u, t_end - 1);
+        if (kFused || vec) {
+#pragma unroll
+          for (int u = 0; u < kU; ++u) xx[u] = *reinterpret_cast<const bf16x8*>(x + (size_t)ts[u] * D + d0);
+        } else {
+#pragma unroll
+          for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              xx[u][j] = d0 + j < D ? x[(size_t)ts[u] * D + d0 + j] : (bf16)0.f;
+              old[u][j] = d0 + j < D ? dx[(size_t)ts[u] * D + d0 + j] : (bf16)0.f;
+            }
+        }
+        if constexpr (kGather == 1 || kGather == 2) {
+          bf16x8 gv[kU][kGather];
+#pragma unroll
+          for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int j = 0; j < kGather; ++j)
+              gv[u][j] = *reinterpret_cast<const bf16x8*>(dgrouped + (size_t)pos_s[ts[u] - tb][j] * D + d0);
+#pragma unroll
+          for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+              old[u][q] = kGather == 1 ? gv[u][0][q] : (bf16)((float)gv[u][0][q] + (float)gv[u][kGather - 1][q]);
+        } else if constexpr (kFused) {
+#pragma unroll
+          for (int u = 0; u < kU; ++u) {
+            float acc[8] = {};
+            for (int j = 0; j < k; ++j) {
+              const bf16x8 v = *reinterpret_cast<const bf16x8*>(dgrouped + (size_t)pos_s[ts[u] - tb][j] * D + d0);
+#pragma unroll
+              for (int q = 0; q < 8; ++q) acc[q] = (float)(bf16)(acc[q] + (float)v[q]);
+            }
+            old[u] = pack8(acc);
+          }
+        } else if (vec) {
+#pragma unroll
+          for (int u = 0; u < kU; ++u) old[u] = *reinterpret_cast<const bf16x8*>(dx + (size_t)ts[u] * D + d0);
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int i = i0 + 32 * u;
+          float dl[EP];
+#pragma unroll
+          for (int e4 = 0; e4 < EP; e4 += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(&dl_s[i][e4]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dl[e4 + r] = v[r];
+          }
+          bf16x8 o;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            float sj = 0.f;
+#pragma unroll
+            for (int e = 0; e < EP; ++e) {
+              sj = fmaf(dl[e], wc[j][e], sj);
+              dwp[j][e] = fmaf((float)xx[u][j], dl[e], dwp[j][e]);
+            }
+            o[j] = (bf16)((float)old[u][j] + (float)(bf16)sj);
+          }
+          if (tb + i >= t_end) continue;
+          bf16* drow = dx + (size_t)(tb + i) * D + d0;
+          if (kFused || vec) {
+            *reinterpret_cast<bf16x8*>(drow) = o;
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (d0 + j < D) drow[j] = o[j];
+          }
+        }
       }
     }
   }
@@ -639,6 +768,37 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const bf16* __restrict_
   }
 }
 
+template <int EP>
+void launch_router_bwd(unsigned grid, int run, hipStream_t s, const bf16* x, const float* w, const float* probs,
+                       const int32_t* chosen, const float* gate, const float* dgate, const float* dmean,
+                       const bf16* dgrouped, const int32_t* position, bf16* dx, float* dw, int T, int D, int E, int k) {
+  auto* kernel = !dgrouped ? router_bwd_kernel<EP, -1>
+                 : k == 1  ? router_bwd_kernel<EP, 1>
+                 : k == 2  ? router_bwd_kernel<EP, 2>
+                           : router_bwd_kernel<EP, 0>;
+  kernel<<<grid, 256, 0, s>>>(x, w, probs, chosen, gate, dgate, dmean, dgrouped, position, dx, dw, T, D, E, k, run);
+}
+
+int router_bwd(const void* x, const float* router_w, const float* probs, const int32_t* chosen, const float* gate,
+               const float* dgate, const float* dmean_probability, const void* dgrouped, const int32_t* position,
+               void* dx, float* dw_router, int tokens, int width, int experts, int top_k, void* stream) {
+  if (!x || !router_w || !probs || !chosen || !gate || !dgate || !dx || !dw_router) return GPTRIG_E_NULL;
+  if (tokens <= 0 || width <= 0 || experts <= 0 || top_k <= 0 || top_k > experts) return GPTRIG_E_SHAPE;
+  if (experts > kMaxRouterExperts || (size_t)width * experts * sizeof(float) > 32768) return GPTRIG_E_UNSUPPORTED;
+  const int ncol = ceil_div(width, kRouterBwdCols);
+  const int runs = gemm::device_cus() / ncol > 1 ? gemm::device_cus() / ncol : 1;
+  // Tokens per workgroup: an even share, in whole sweeps of the 32 token lanes.
+  const int run = ceil_div(ceil_div(tokens, runs), 32) * 32;
+  const unsigned grid = (unsigned)ncol * (unsigned)ceil_div(tokens, run);
+  (experts <= 4   ? launch_router_bwd<4>
+   : experts <= 8 ? launch_router_bwd<8>
+                  : launch_router_bwd<16>)(grid, run, (hipStream_t)stream, (const bf16*)x, router_w, probs, chosen, gate,
+                                           dgate, dmean_probability, (const bf16*)dgrouped, position, (bf16*)dx,
+                                           dw_router, tokens, width, experts, top_k);
+  GPTRIG_CHECK_LAUNCH();
+  return GPTRIG_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -659,7 +819,11 @@ int gptrig_moe_route(const float* logits, float* probs, int32_t* chosen, float* 
   if (!workspace || workspace_bytes < gptrig_moe_route_workspace_bytes(tokens, experts, top_k))
     return GPTRIG_E_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
-  route_topk_kernel<<<ceil_div(tokens, 128), 128, 0, s>>>(logits, probs, chosen, gate, tokens, experts, top_k);
+  (experts <= 4    ? route_topk_kernel<4>
+   : experts <= 8  ? route_topk_kernel<8>
+   : experts <= 16 ? route_topk_kernel<16>
+                   : route_topk_kernel<kMaxExperts>)<<<ceil_div(tokens, 128), 128, 0, s>>>(logits, probs, chosen, gate,
+                                                                                           tokens, experts, top_k);
   GPTRIG_CHECK_LAUNCH();
   const int n_slots = tokens * top_k, nblocks = ceil_div(n_slots, kSortBlock);
   int32_t* hist = (int32_t*)workspace;
@@ -677,17 +841,11 @@ int gptrig_moe_router_logits(const void* x, const float* router_w, float* logits
   if (!x || !router_w || !logits) return GPTRIG_E_NULL;
   if (tokens <= 0 || width <= 0 || experts <= 0) return GPTRIG_E_SHAPE;
   if (experts > kMaxRouterExperts || (size_t)width * experts * sizeof(float) > 32768) return GPTRIG_E_UNSUPPORTED;
-  const int ep = experts <= 4 ? 4 : experts <= 8 ? 8 : 16;
-  if ((size_t)width * ep * sizeof(float) > 65536) return GPTRIG_E_UNSUPPORTED;
-  const size_t smem = (size_t)width * ep * sizeof(float);
-  const unsigned grid = (unsigned)ceil_div(tokens, 4 * kRouterTokens);
-  hipStream_t s = (hipStream_t)stream;
-  if (ep == 4)
-    router_logits_kernel<4><<<grid, 256, smem, s>>>((const bf16*)x, router_w, logits, tokens, width, experts);
-  else if (ep == 8)
-    router_logits_kernel<8><<<grid, 256, smem, s>>>((const bf16*)x, router_w, logits, tokens, width, experts);
-  else
-    router_logits_kernel<16><<<grid, 256, smem, s>>>((const bf16*)x, router_w, logits, tokens, width, experts);
+  const size_t smem = (size_t)3 * experts * router_row(width) * sizeof(bf16);  // at most 54 KB
+  const unsigned grid = (unsigned)ceil_div(tokens, 16 * kRouterWaves);
+  // 16-byte loads of token rows.
+  (width % 8 == 0 && ((uintptr_t)x & 15) == 0 ? router_logits_kernel<true> : router_logits_kernel<false>)<<<
+      grid, 64 * kRouterWaves, smem, (hipStream_t)stream>>>((const bf16*)x, router_w, logits, tokens, width, experts);
   GPTRIG_CHECK_LAUNCH();
   return GPTRIG_OK;
 }
@@ -762,8 +920,10 @@ int gptrig_moe_combine(const void* out, const int32_t* position, const float* ga
   if (!out || !position || !gate || !combined) return GPTRIG_E_NULL;
   if (tokens <= 0 || width <= 0 || top_k <= 0 || width % 8) return GPTRIG_E_SHAPE;
   if (top_k > kMaxTopK) return GPTRIG_E_UNSUPPORTED;
-  moe_combine_kernel<<<ceil_div(tokens, 4), 256, 0, (hipStream_t)stream>>>((const bf16*)out, position, gate,
-                                                                          (bf16*)combined, tokens, width, top_k);
+  (top_k == 1   ? moe_combine_kernel<1>
+   : top_k == 2 ? moe_combine_kernel<2>
+                : moe_combine_kernel<0>)<<<ceil_div(tokens, 4), 256, 0, (hipStream_t)stream>>>(
+      (const bf16*)out, position, gate, (bf16*)combined, tokens, width, top_k);
   GPTRIG_CHECK_LAUNCH();
   return GPTRIG_OK;
 }
@@ -814,22 +974,19 @@ int gptrig_moe_stats(const float* logits, const float* probs, const float* gate,
 int gptrig_moe_router_bwd(const void* x, const float* router_w, const float* probs, const int32_t* chosen,
                           const float* gate, const float* dgate, const float* dmean_probability, void* dx,
                           float* dw_router, int tokens, int width, int experts, int top_k, void* stream) {
-  if (!x || !router_w || !probs || !chosen || !gate || !dgate || !dx || !dw_router) return GPTRIG_E_NULL;
-  if (tokens <= 0 || width <= 0 || experts <= 0 || top_k <= 0 || top_k > experts) return GPTRIG_E_SHAPE;
-  if (experts > kMaxRouterExperts || (size_t)width * experts * sizeof(float) > 32768) return GPTRIG_E_UNSUPPORTED;
-  const dim3 grid((unsigned)ceil_div(width, kRouterBwdCols), (unsigned)ceil_div(tokens, kRouterBwdTokens));
-  hipStream_t s = (hipStream_t)stream;
-  if (experts <= 4)
-    router_bwd_kernel<4><<<grid, 256, 0, s>>>((const bf16*)x, router_w, probs, chosen, gate, dgate, dmean_probability,
-                                              (bf16*)dx, dw_router, tokens, width, experts, top_k);
-  else if (experts <= 8)
-    router_bwd_kernel<8><<<grid, 256, 0, s>>>((const bf16*)x, router_w, probs, chosen, gate, dgate, dmean_probability,
-                                              (bf16*)dx, dw_router, tokens, width, experts, top_k);
-  else
-    router_bwd_kernel<16><<<grid, 256, 0, s>>>((const bf16*)x, router_w, probs, chosen, gate, dgate,
-                                               dmean_probability, (bf16*)dx, dw_router, tokens, width, experts, top_k);
-  GPTRIG_CHECK_LAUNCH();
-  return GPTRIG_OK;
+  return router_bwd(x, router_w, probs, chosen, gate, dgate, dmean_probability, nullptr, nullptr, dx, dw_router,
+                    tokens, width, experts, top_k, stream);
+}
+
+int gptrig_moe_input_bwd(const void* dgrouped, const int32_t* position, const void* x, const float* router_w,
+                         const float* probs, const int32_t* chosen, const float* gate, const float* dgate,
+                         const float* dmean_probability, void* dx, float* dw_router, int tokens, int width,
+                         int experts, int top_k, void* stream) {
+  if (!dgrouped || !position) return GPTRIG_E_NULL;
+  if (width % 8 || (((uintptr_t)dgrouped | (uintptr_t)x | (uintptr_t)dx) & 15)) return GPTRIG_E_SHAPE;
+  if (top_k > kMaxTopK) return GPTRIG_E_UNSUPPORTED;
+  return router_bwd(x, router_w, probs, chosen, gate, dgate, dmean_probability, dgrouped, position, dx, dw_router,
+                    tokens, width, experts, top_k, stream);
 }
 
 }  // extern "C"

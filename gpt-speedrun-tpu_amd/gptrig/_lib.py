@@ -90,6 +90,7 @@ SIGNATURES: dict[str, tuple] = {
     "gptrig_moe_gather_bwd": (I, [P, P, P, I, I, I, P]),
     "gptrig_moe_stats": (I, [P, P, P, P, I, I, I, P, P, P, P]),
     "gptrig_moe_router_bwd": (I, [P, P, P, P, P, P, P, P, P, I, I, I, I, P]),
+    "gptrig_moe_input_bwd": (I, [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, P]),
 }
 
 _LIB = None

@@ -110,12 +110,11 @@ class _RoutedMLP(torch.autograd.Function):
                   d_up_w.data_ptr(), d_up_b.data_ptr(), R, width, hidden_width, experts, s)
         dgrouped = _gmm(dpre, upw, True, counts, None, 0, None, R, hidden_width, width, experts)
         dx = torch.empty((tokens, width), dtype=BF16, device=dev)
-        _lib.call("gptrig_moe_gather_bwd", dgrouped.data_ptr(), position.data_ptr(), dx.data_ptr(), tokens, width,
-                  top_k, s)
         dmp = None if dmean_probability is None else dmean_probability.to(F32).contiguous()
-        _lib.call("gptrig_moe_router_bwd", flat.data_ptr(), rw.data_ptr(), probs.data_ptr(), chosen.data_ptr(),
-                  gate.data_ptr(), dgate.data_ptr(), None if dmp is None else dmp.data_ptr(), dx.data_ptr(),
-                  d_router.data_ptr(), tokens, width, experts, top_k, s)
+        _lib.call("gptrig_moe_input_bwd", dgrouped.data_ptr(), position.data_ptr(), flat.data_ptr(), rw.data_ptr(),
+                  probs.data_ptr(), chosen.data_ptr(), gate.data_ptr(), dgate.data_ptr(),
+                  None if dmp is None else dmp.data_ptr(), dx.data_ptr(), d_router.data_ptr(), tokens, width, experts,
+                  top_k, s)
         return (dx.reshape(batch, length, width).to(xdt), d_router.to(rdt), d_up_w.to(uwdt), d_up_b.to(ubdt),
                 d_down_w.to(dwdt), d_down_b.to(dbdt), None, None)
 

@@ -422,11 +422,10 @@ class GPTTrainer:
         _lib.call("gptrig_moe_gmm", dpre.data_ptr(), eh, A.w(p + "expert_up_w").data_ptr(), 1, counts.data_ptr(),
                   None, 0, dgrouped.data_ptr(), None, d, R, eh, d, E, s)
         dxn2 = torch.empty((N, d), dtype=BF16, device=dev)
-        _lib.call("gptrig_moe_gather_bwd", dgrouped.data_ptr(), position.data_ptr(), dxn2.data_ptr(), N, d, k, s)
         dmp = (load * (c.router_aux_coefficient * E / c.layers)).contiguous()
-        _lib.call("gptrig_moe_router_bwd", xn2.data_ptr(), A.param(p + "router_w").data_ptr(), probs.data_ptr(),
-                  chosen.data_ptr(), gate.data_ptr(), dgate.data_ptr(), dmp.data_ptr(), dxn2.data_ptr(),
-                  A.grad(p + "router_w").data_ptr(), N, d, E, k, s)
+        _lib.call("gptrig_moe_input_bwd", dgrouped.data_ptr(), position.data_ptr(), xn2.data_ptr(),
+                  A.param(p + "router_w").data_ptr(), probs.data_ptr(), chosen.data_ptr(), gate.data_ptr(),
+                  dgate.data_ptr(), dmp.data_ptr(), dxn2.data_ptr(), A.grad(p + "router_w").data_ptr(), N, d, E, k, s)
         return dxn2
 
     # -- forward / backward of one micro-batch --------------------------------------

@@ -408,6 +408,13 @@ int gptrig_moe_stats(const float* logits, const float* probs, const float* gate,
 int gptrig_moe_router_bwd(const void* x, const float* router_w, const float* probs, const int32_t* chosen,
                           const float* gate, const float* dgate, const float* dmean_probability, void* dx,
                           float* dw_router, int tokens, int width, int experts, int top_k, void* stream);
+/* gptrig_moe_gather_bwd and gptrig_moe_router_bwd in one pass (the same
+ * values; dx is only written): width a multiple of 8, dgrouped, x and dx 16-byte
+ * aligned, top_k <= 8. */
+int gptrig_moe_input_bwd(const void* dgrouped, const int32_t* position, const void* x, const float* router_w,
+                         const float* probs, const int32_t* chosen, const float* gate, const float* dgate,
+                         const float* dmean_probability, void* dx, float* dw_router, int tokens, int width,
+                         int experts, int top_k, void* stream);
 
 #ifdef __cplusplus
 }

@@ -186,3 +186,61 @@ def test_config_e_routing_bit_exact_on_all_tokens():
     assert torch.equal(counts.cpu(), counts_r)
     assert torch.equal(order.cpu().long(), order_r)
     assert torch.equal(rows.cpu().long(), rows_r)
+
+
+@pytest.mark.parametrize("tokens,width,experts", [
+    (1, 8, 1), (15, 40, 3), (64, 256, 16), (65, 520, 8), (200, 96, 5), (33, 36, 4),  # (33, 36): element loads
+])
+def test_router_logits_against_float64(tokens, width, experts):
+    """The split-weight router product at its edges (one token, ragged token
+    tiles, widths with partial steps and without 16-byte loads, every expert
+    count class) against float64.
+
+    Bound: exact products, three float32 sums of ``width`` of them rounded
+    once per 32 and added: 2^-24 (ceil(width / 32) + 3) of the magnitudes."""
+    from gptrig import _lib
+
+    g = torch.Generator().manual_seed(width)
+    x = torch.randn((tokens, width), generator=g).bfloat16().to(DEV)
+    w = (torch.randn((width, experts), generator=g) * 0.3).to(DEV)
+    logits = torch.full((tokens, experts), float("nan"), device=DEV)
+    print(f"router logits tokens={tokens} width={width} experts={experts}", flush=True)
+    _lib.call("gptrig_moe_router_logits", x.data_ptr(), w.data_ptr(), logits.data_ptr(), tokens, width, experts,
+              _lib.stream())
+    x64, w64 = x.double(), w.double()
+    bound = (x64.abs() @ w64.abs()) * 2.0 ** -24 * (-(-width // 32) + 3)
+    excess = float(((logits.double() - x64 @ w64).abs() / bound).max())
+    print(f"  error / bound {excess:.3f}", flush=True)
+    assert excess <= 1
+
+
+@pytest.mark.parametrize("tokens,width,experts,top_k", [
+    (1, 8, 2, 1), (255, 64, 4, 2), (257, 72, 8, 2), (300, 136, 16, 3), (130, 264, 5, 1),
+])
+def test_fused_input_backward_equals_two_passes(tokens, width, experts, top_k):
+    """gptrig_moe_input_bwd against gptrig_moe_gather_bwd then
+    gptrig_moe_router_bwd: dx bit for bit, the router gradient to its float32
+    atomics (each workgroup adds one partial per entry)."""
+    from gptrig import _lib
+
+    g = torch.Generator().manual_seed(tokens + width)
+    R = tokens * top_k
+    x, dgrouped = (torch.randn((n, width), generator=g).bfloat16().to(DEV) for n in (tokens, R))
+    w = (torch.randn((width, experts), generator=g) * 0.1).to(DEV)
+    probs = torch.softmax(torch.randn((tokens, experts), generator=g), -1).to(DEV)
+    chosen = torch.rand((tokens, experts), generator=g).topk(top_k).indices.to(torch.int32).to(DEV)
+    gate = torch.softmax(torch.randn((tokens, top_k), generator=g), -1).to(DEV)
+    dgate, dmean = torch.randn(R, generator=g).to(DEV), torch.randn(experts, generator=g).to(DEV)
+    position = torch.randperm(R, generator=g).to(torch.int32).to(DEV)
+    s = _lib.stream()
+    print(f"input backward tokens={tokens} width={width} experts={experts} top_k={top_k}", flush=True)
+    tail = [probs, chosen, gate, dgate, dmean]
+    dx1, dx2 = (torch.full((tokens, width), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    dw1, dw2 = (torch.ones((width, experts), device=DEV) for _ in range(2))
+    _lib.call("gptrig_moe_gather_bwd", dgrouped.data_ptr(), position.data_ptr(), dx1.data_ptr(), tokens, width, top_k, s)
+    _lib.call("gptrig_moe_router_bwd", x.data_ptr(), w.data_ptr(), *(t.data_ptr() for t in tail), dx1.data_ptr(),
+              dw1.data_ptr(), tokens, width, experts, top_k, s)
+    _lib.call("gptrig_moe_input_bwd", dgrouped.data_ptr(), position.data_ptr(), x.data_ptr(), w.data_ptr(),
+              *(t.data_ptr() for t in tail), dx2.data_ptr(), dw2.data_ptr(), tokens, width, experts, top_k, s)
+    assert torch.equal(dx1, dx2)
+    torch.testing.assert_close(dw1, dw2, rtol=1e-6, atol=1e-5 * float(dw1.abs().max()))
