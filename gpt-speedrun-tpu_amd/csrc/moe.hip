@@ -268,14 +268,13 @@ __global__ void __launch_bounds__(64 * kRouterWaves)
 //       2: out = bf16(bf16(acc) * gelu'(pre))   (pre read, same layout as out)
 // ---------------------------------------------------------------------------
 template <bool kBT, int kMode>
-__global__ void __launch_bounds__(gemm::THREADS)
-    moe_gmm_kernel(const bf16* __restrict__ lhs, int64_t lda,
-                   const bf16* __restrict__ rhs, const int32_t* __restrict__ counts, int E, int K, int N,
-                   const bf16* __restrict__ bias, bf16* __restrict__ out, bf16* __restrict__ pre, int64_t ldo) {
-  __shared__ __attribute__((aligned(16))) float bias_s[gemm::BM];
+__device__ __forceinline__ void moe_gmm_tile(int pid, const bf16* __restrict__ lhs, int64_t lda,
+                                             const bf16* __restrict__ rhs, const int32_t* __restrict__ counts, int E,
+                                             int K, int N, const bf16* __restrict__ bias, bf16* __restrict__ out,
+                                             bf16* __restrict__ pre, int64_t ldo, float* bias_s) {
   const int ntn = (N + gemm::BN - 1) / gemm::BN;
-  const int tn = blockIdx.x % ntn;  // feature tile
-  int tm = blockIdx.x / ntn;        // bucket-row tile of expert e
+  const int tn = pid % ntn;  // feature tile
+  int tm = pid / ntn;        // bucket-row tile of expert e
   int e = 0, off = 0;
   for (; e < E; ++e) {
     const int c = counts[e];
@@ -310,42 +309,36 @@ __global__ void __launch_bounds__(gemm::THREADS)
   gemm_epi::linear_epilogue<kEpi>(acc, tn, tm, N, cnt, ea, bias_s);
 }
 
-// Per-expert weight (+ bias) gradients:
-//   dw[e] (f32 [K][N]) += sum_{r in bucket e} A[r][k] * dy[r][n],
-//   db[e] (f32 [N])    += sum_{r in bucket e} dy[r][n]          (nullable),
-// A [R][K] and dy [R][N] in bucket order.  Grid:
-// E x tiles(K, N) x split; bucket e's rows are split into `split` slices,
-// whose partial tiles are added with fp32 atomics (measured no slower than a
-// read-modify-write when a tile has one writer).
+template <bool kBT, int kMode>
 __global__ void __launch_bounds__(gemm::THREADS)
-    moe_gmm_dw_kernel(const bf16* __restrict__ lhs, int64_t lda,
-                      const bf16* __restrict__ dy, int64_t ldy, const int32_t* __restrict__ counts, int E, int K,
-                      int N, int split, float* __restrict__ dw, float* __restrict__ db) {
-  const int tiles = ((K + gemm::BM - 1) / gemm::BM) * ((N + gemm::BN - 1) / gemm::BN);
-  const int e = blockIdx.x / (tiles * split);
-  const int rem = blockIdx.x % (tiles * split);
-  const int sp = rem / tiles;
+    moe_gmm_kernel(const bf16* __restrict__ lhs, int64_t lda,
+                   const bf16* __restrict__ rhs, const int32_t* __restrict__ counts, int E, int K, int N,
+                   const bf16* __restrict__ bias, bf16* __restrict__ out, bf16* __restrict__ pre, int64_t ldo) {
+  __shared__ __attribute__((aligned(16))) float bias_s[gemm::BM];
+  moe_gmm_tile<kBT, kMode>(blockIdx.x, lhs, lda, rhs, counts, E, K, N, bias, out, pre, ldo, bias_s);
+}
+
+// One tile of an expert's weight (+ bias) gradient over the rows [k_begin,
+// k_end) of its bucket, which starts at row `off`:
+//   dwe (f32 [K][N]) += sum_r A[r][k] * dy[r][n],  dbe (f32 [N], nullable) += sum_r dy[r][n],
+// A [R][K] and dy [R][N] in bucket order; fp32 atomics, or, with store, dwe's
+// tile overwritten (also by an empty row range).
+__device__ __forceinline__ void moe_dw_tile(const bf16* __restrict__ lhs, int64_t lda, const bf16* __restrict__ dy,
+                                            int64_t ldy, int off, int cnt, int k_begin, int k_end, int tile, int K,
+                                            int N, float* __restrict__ dwe, float* __restrict__ dbe, bool store) {
   int tm, tn;
-  gemm::tile_coords(rem % tiles, K, N, tm, tn);
-  int off = 0;
-  for (int i = 0; i < e; ++i) off += counts[i];
-  const int cnt = counts[e];
-  const int kslice = ((cnt + split - 1) / split + gemm::BK - 1) / gemm::BK * gemm::BK;
-  const int k_begin = sp * kslice;
-  const int k_end = min(cnt, k_begin + kslice);
-  if (k_begin >= k_end) return;  // uniform
+  gemm::tile_coords(tile, K, N, tm, tn);
   // A(m = k-index, k = bucket row) MN-major; B(k = bucket row, n) MN-major.
   gemm::Operand A{lhs + (int64_t)off * lda, lda};
   gemm::Operand B{dy + (int64_t)off * ldy, ldy};
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   f32x16 acc[4][2];
   float csum[2] = {0.f, 0.f};
-  const bool do_colsum = db != nullptr;  // shared out over the M tiles
+  const bool do_colsum = dbe != nullptr;  // shared out over the M tiles
   gemm::mainloop_pp<false, false, true>(acc, A, B, K, N, k_begin, k_end, tm * gemm::BM, tn * gemm::BN, csum,
                                         do_colsum ? (K + gemm::BM - 1) / gemm::BM : 0, tm);
   const int hl = lane >> 5, l32 = lane & 31;
   const int wm = wave & 1, wn = wave >> 1;
-  float* dwe = dw + (int64_t)e * K * N;
 #pragma unroll
   for (int nb = 0; nb < 2; ++nb) {
     const int n = tn * gemm::BN + 64 * wn + 32 * nb + l32;
@@ -355,7 +348,11 @@ __global__ void __launch_bounds__(gemm::THREADS)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int m = tm * gemm::BM + 128 * wm + 32 * mb + 8 * (i >> 2) + 4 * hl + (i & 3);
-        if (m < K) atomicAdd(dwe + (int64_t)m * N + n, acc[mb][nb][i]);
+        if (m >= K) continue;
+        if (store)
+          dwe[(int64_t)m * N + n] = acc[mb][nb][i];
+        else
+          atomicAdd(dwe + (int64_t)m * N + n, acc[mb][nb][i]);
       }
   }
   if (do_colsum && wm == 0) {
@@ -363,9 +360,99 @@ __global__ void __launch_bounds__(gemm::THREADS)
     for (int nb = 0; nb < 2; ++nb) {
       const float t = csum[nb] + __shfl_xor(csum[nb], 32);
       const int n = tn * gemm::BN + 64 * wn + 32 * nb + l32;
-      if (hl == 0 && n < N) atomicAdd(db + (int64_t)e * N + n, t);
+      if (hl == 0 && n < N) atomicAdd(dbe + n, t);
     }
   }
+}
+
+// dw[e] += ..., db[e] += ... for every expert.  Grid: E x tiles(K, N) x split;
+// bucket e's rows are split into `split` slices, whose partial tiles are added
+// with fp32 atomics (measured no slower than a read-modify-write when a tile
+// has one writer).
+__global__ void __launch_bounds__(gemm::THREADS)
+    moe_gmm_dw_kernel(const bf16* __restrict__ lhs, int64_t lda,
+                      const bf16* __restrict__ dy, int64_t ldy, const int32_t* __restrict__ counts, int K, int N,
+                      int split, float* __restrict__ dw, float* __restrict__ db) {
+  const int tiles = ((K + gemm::BM - 1) / gemm::BM) * ((N + gemm::BN - 1) / gemm::BN);
+  const int e = blockIdx.x / (tiles * split);
+  const int rem = blockIdx.x % (tiles * split);
+  const int sp = rem / tiles;
+  int off = 0;
+  for (int i = 0; i < e; ++i) off += counts[i];
+  const int cnt = counts[e];
+  const int kslice = ((cnt + split - 1) / split + gemm::BK - 1) / gemm::BK * gemm::BK;
+  const int k_begin = sp * kslice;
+  const int k_end = min(cnt, k_begin + kslice);
+  if (k_begin >= k_end) return;  // uniform
+  moe_dw_tile(lhs, lda, dy, ldy, off, cnt, k_begin, k_end, rem % tiles, K, N, dw + (int64_t)e * K * N,
+              db ? db + (int64_t)e * N : nullptr, false);
+}
+
+// The three backward GEMMs that need only the pre-activation gradient dpre and
+// what the forward kept, in one launch:
+//   down_dw, down_db from (hidden, dout); up_dw, up_db from (grouped, dpre);
+//   dgrouped = dpre up_w^T.
+// Alone, each weight gradient leaves CUs idle (8 experts of 768 x 1536: 144
+// tiles of 256-stage reductions for 256 CUs, 269 us) and so does the end of
+// the input gradient's grid (201 us).  The weight-gradient items come first
+// (the longest, handed out first), the short input-gradient tiles fill the CUs
+// that are free: 32768 tokens x 768, top 2: 473 us for the three against 739.
+// A bucket is cut into slices of `slice` rows (a multiple of BK): its tiles are
+// stored when one slice holds it and added with atomics, to gradients that
+// moe_zero_kernel cleared, when it takes more (an expert with many times its
+// even share must not leave its tiles to a few workgroups).  The slots of a
+// weight are experts + rows / slice slices, the most that any counts need;
+// surplus ones exit.
+struct MoeBwdGemms {
+  const bf16 *grouped, *dpre, *hidden, *dout, *up_w;
+  const int32_t* counts;
+  float *up_dw, *up_db, *down_dw, *down_db;
+  bf16* dgrouped;
+  int width, hidden_width, experts, slice, n_slots, tiles;  // workgroups: n_slots x tiles down, as many up, dgrouped
+};
+
+__global__ void __launch_bounds__(gemm::THREADS) moe_bwd_gemms_kernel(MoeBwdGemms g) {
+  __shared__ __attribute__((aligned(16))) float bias_s[gemm::BM];
+  const int n_dw = g.n_slots * g.tiles;
+  const int b = blockIdx.x;
+  if (b < 2 * n_dw) {
+    const bool down = b < n_dw;  // uniform
+    const int item = down ? b : b - n_dw;
+    int slot = item / g.tiles, e = 0, off = 0;
+    for (; e < g.experts; ++e) {
+      const int c = g.counts[e];
+      const int n = c <= g.slice ? 1 : (c + g.slice - 1) / g.slice;  // (an empty bucket stores zeros)
+      if (slot < n) break;
+      slot -= n;
+      off += c;
+    }
+    if (e >= g.experts) return;  // uniform: surplus slot
+    const int cnt = g.counts[e];
+    const int K = down ? g.hidden_width : g.width, N = down ? g.width : g.hidden_width;
+    moe_dw_tile(down ? g.hidden : g.grouped, K, down ? g.dout : g.dpre, N, off, cnt, slot * g.slice,
+                min(cnt, (slot + 1) * g.slice), item % g.tiles, K, N,
+                (down ? g.down_dw : g.up_dw) + (int64_t)e * K * N, (down ? g.down_db : g.up_db) + (int64_t)e * N,
+                cnt <= g.slice);
+  } else {
+    moe_gmm_tile<true, 0>(b - 2 * n_dw, g.dpre, g.hidden_width, g.up_w, g.counts, g.experts, g.hidden_width, g.width,
+                          nullptr, g.dgrouped, nullptr, g.width, bias_s);
+  }
+}
+
+// Clears what moe_bwd_gemms_kernel adds to: the bias gradients, and the weight
+// gradients of the experts with more than one slice.  Grid: (x, experts).
+__global__ void __launch_bounds__(256) moe_zero_kernel(MoeBwdGemms g) {
+  const int e = blockIdx.y;
+  const int i0 = (blockIdx.x * blockDim.x + threadIdx.x) * 4, step = gridDim.x * blockDim.x * 4;
+  auto clear = [&](float* p, int64_t n) {
+    for (int64_t i = i0; i < n; i += step) *reinterpret_cast<f32x4*>(p + i) = f32x4{};
+  };
+  clear(g.up_db + (int64_t)e * g.hidden_width, g.hidden_width);
+  clear(g.down_db + (int64_t)e * g.width, g.width);
+  if (g.counts[e] <= g.slice) return;
+  const int64_t nw = (int64_t)g.width * g.hidden_width;
+  clear(g.up_dw + e * nw, nw);
+  clear(g.down_dw + e * nw, nw);
 }
 
 // grouped[p] = x[rows[p]] (flat[rows], :1278): one wave per bucket row.
@@ -910,7 +997,55 @@ int gptrig_moe_gmm_dw(const void* lhs, int64_t lda, const void* dy, int64_t ldy,
   const int split = cells >= gemm::device_cus() ? 1 : gemm::choose_split(tiles * experts,
                                                                          ceil_div(ceil_div(rows, experts), gemm::BK));
   moe_gmm_dw_kernel<<<tiles * experts * split, gemm::THREADS, 0, (hipStream_t)stream>>>(
-      (const bf16*)lhs, lda, (const bf16*)dy, ldy, counts, experts, k, n, split, dw, db);
+      (const bf16*)lhs, lda, (const bf16*)dy, ldy, counts, k, n, split, dw, db);
+  GPTRIG_CHECK_LAUNCH();
+  return GPTRIG_OK;
+}
+
+int gptrig_moe_bwd_gemms(const void* grouped, const void* dpre, const void* hidden, const void* dout, const void* up_w,
+                         const int32_t* counts, float* up_dw, float* up_db, float* down_dw, float* down_db,
+                         void* dgrouped, int rows, int width, int hidden_width, int experts, void* stream) {
+  if (!grouped || !dpre || !hidden || !dout || !up_w || !counts || !up_dw || !up_db || !down_dw || !down_db || !dgrouped)
+    return GPTRIG_E_NULL;
+  if (rows <= 0 || width <= 0 || hidden_width <= 0 || experts <= 0 || width % 8 || hidden_width % 8)
+    return GPTRIG_E_SHAPE;
+  if (((uintptr_t)grouped | (uintptr_t)dpre | (uintptr_t)hidden | (uintptr_t)dout | (uintptr_t)up_w |
+       (uintptr_t)dgrouped | (uintptr_t)up_dw | (uintptr_t)up_db | (uintptr_t)down_dw | (uintptr_t)down_db) & 15)
+    return GPTRIG_E_SHAPE;
+  if (experts > kMaxExperts) return GPTRIG_E_UNSUPPORTED;
+  hipStream_t s = (hipStream_t)stream;
+  const int cus = gemm::device_cus();
+  // Both weights have the same number of 256 x 256 tiles.
+  const int tiles = ceil_div(hidden_width, gemm::BM) * ceil_div(width, gemm::BN);
+  const int n_dx = (ceil_div(rows, gemm::BM) + experts) * ceil_div(width, gemm::BN);
+  // Slices per evenly filled bucket, from the estimated makespan: stages of 32
+  // rows plus an epilogue (10 for a plain store, 60 for the atomic add of a
+  // tile, measured in the FLCE gradient launches), the longest items first.
+  const int stages = ceil_div(ceil_div(rows, experts), gemm::BK);
+  const double dx_cost = (double)ceil_div(rows, gemm::BM) * ceil_div(width, gemm::BN) *
+                         ((double)ceil_div(hidden_width, gemm::BK) + 10.0);
+  int split = 1;
+  double best = 1e300;
+  for (int k = 1; k <= 64 && (k == 1 || stages / k >= 8); ++k) {
+    const double item = ceil_div(stages, k) + (k > 1 ? 60.0 : 10.0);
+    const int64_t items = 2ll * tiles * experts * k;
+    const double rounds = (double)ceil_div(items, (int64_t)cus) * item;
+    const double even = ((double)items * item + dx_cost) / cus;
+    const double cost = rounds > even ? rounds : even;
+    if (cost < best * 0.999) {
+      best = cost;
+      split = k;
+    }
+  }
+  // One slice holds a bucket of up to twice the even share.
+  const int64_t slice = split == 1 ? 2ll * stages * gemm::BK : (int64_t)ceil_div(stages, split) * gemm::BK;
+  const int slots = experts + (int)(rows / slice);
+  MoeBwdGemms g{(const bf16*)grouped, (const bf16*)dpre, (const bf16*)hidden, (const bf16*)dout, (const bf16*)up_w,
+                counts, up_dw, up_db, down_dw, down_db, (bf16*)dgrouped, width, hidden_width, experts,
+                (int)(slice < (1 << 30) ? slice : (1 << 30)), slots, tiles};
+  moe_zero_kernel<<<dim3(32, (unsigned)experts), 256, 0, s>>>(g);
+  GPTRIG_CHECK_LAUNCH();
+  moe_bwd_gemms_kernel<<<2u * (unsigned)slots * (unsigned)tiles + (unsigned)n_dx, gemm::THREADS, 0, s>>>(g);
   GPTRIG_CHECK_LAUNCH();
   return GPTRIG_OK;
 }

@@ -85,6 +85,7 @@ SIGNATURES: dict[str, tuple] = {
     "gptrig_moe_gather_rows": (I, [P, P, P, I, I, P]),
     "gptrig_moe_gmm": (I, [P, L, P, I, P, P, I, P, P, L, I, I, I, I, P]),
     "gptrig_moe_gmm_dw": (I, [P, L, P, L, P, P, P, I, I, I, I, P]),
+    "gptrig_moe_bwd_gemms": (I, [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, P]),
     "gptrig_moe_combine": (I, [P, P, P, P, I, I, I, P]),
     "gptrig_moe_combine_bwd": (I, [P, P, P, P, P, P, I, I, I, P]),
     "gptrig_moe_gather_bwd": (I, [P, P, P, I, I, I, P]),

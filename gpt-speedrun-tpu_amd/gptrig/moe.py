@@ -96,19 +96,18 @@ class _RoutedMLP(torch.autograd.Function):
         dgate = torch.empty(R, dtype=F32, device=dev)
         _lib.call("gptrig_moe_combine_bwd", dc.data_ptr(), out.data_ptr(), position.data_ptr(), gate.data_ptr(),
                   dout.data_ptr(), dgate.data_ptr(), tokens, width, top_k, s)
-        d_up_w = torch.zeros((experts, width, hidden_width), dtype=F32, device=dev)
-        d_up_b = torch.zeros((experts, hidden_width), dtype=F32, device=dev)
-        d_down_w = torch.zeros((experts, hidden_width, width), dtype=F32, device=dev)
-        d_down_b = torch.zeros((experts, width), dtype=F32, device=dev)
+        d_up_w = torch.empty((experts, width, hidden_width), dtype=F32, device=dev)
+        d_up_b = torch.empty((experts, hidden_width), dtype=F32, device=dev)
+        d_down_w = torch.empty((experts, hidden_width, width), dtype=F32, device=dev)
+        d_down_b = torch.empty((experts, width), dtype=F32, device=dev)
         d_router = torch.zeros((width, experts), dtype=F32, device=dev)
-        # Down projection: dW, db from (hidden, dout); d(pre) = (dout W^T) * gelu'(pre).
-        _lib.call("gptrig_moe_gmm_dw", hidden.data_ptr(), hidden_width, dout.data_ptr(), width, counts.data_ptr(),
-                  d_down_w.data_ptr(), d_down_b.data_ptr(), R, hidden_width, width, experts, s)
+        # d(pre) = (dout W_down^T) * gelu'(pre); then the weight gradients of both
+        # projections and d(grouped) = dpre W_up^T.
         dpre = _gmm(dout, dnw, True, counts, None, 2, pre, R, width, hidden_width, experts)
-        # Up projection: dW, db from (grouped, dpre); d(grouped) = dpre W^T.
-        _lib.call("gptrig_moe_gmm_dw", grouped.data_ptr(), width, dpre.data_ptr(), hidden_width, counts.data_ptr(),
-                  d_up_w.data_ptr(), d_up_b.data_ptr(), R, width, hidden_width, experts, s)
-        dgrouped = _gmm(dpre, upw, True, counts, None, 0, None, R, hidden_width, width, experts)
+        dgrouped = torch.empty((R, width), dtype=BF16, device=dev)
+        _lib.call("gptrig_moe_bwd_gemms", grouped.data_ptr(), dpre.data_ptr(), hidden.data_ptr(), dout.data_ptr(),
+                  upw.data_ptr(), counts.data_ptr(), d_up_w.data_ptr(), d_up_b.data_ptr(), d_down_w.data_ptr(),
+                  d_down_b.data_ptr(), dgrouped.data_ptr(), R, width, hidden_width, experts, s)
         dx = torch.empty((tokens, width), dtype=BF16, device=dev)
         dmp = None if dmean_probability is None else dmean_probability.to(F32).contiguous()
         _lib.call("gptrig_moe_input_bwd", dgrouped.data_ptr(), position.data_ptr(), flat.data_ptr(), rw.data_ptr(),

@@ -379,6 +379,19 @@ int gptrig_moe_gmm(const void* lhs, int64_t lda, const void* rhs, int rhs_transp
 int gptrig_moe_gmm_dw(const void* lhs, int64_t lda, const void* dy, int64_t ldy, const int32_t* counts, float* dw,
                       float* db, int rows, int k, int n, int experts, void* stream);
 
+/* The backward's products that need only dpre (the gradient of the
+ * pre-activation, gptrig_moe_gmm mode 2) and what the forward kept, in one
+ * launch: up_dw f32 [experts, width, hidden_width], up_db f32 [experts,
+ * hidden_width] from (grouped, dpre); down_dw f32 [experts, hidden_width,
+ * width], down_db f32 [experts, width] from (hidden, dout), as
+ * gptrig_moe_gmm_dw but overwritten, not added to; dgrouped bf16 [rows, width]
+ * = dpre up_w^T as gptrig_moe_gmm mode 0 with the transposed up_w bf16
+ * [experts, width, hidden_width].  width and hidden_width multiples of 8, all
+ * pointers but counts 16-byte aligned, rows contiguous. */
+int gptrig_moe_bwd_gemms(const void* grouped, const void* dpre, const void* hidden, const void* dout, const void* up_w,
+                         const int32_t* counts, float* up_dw, float* up_db, float* down_dw, float* down_db,
+                         void* dgrouped, int rows, int width, int hidden_width, int experts, void* stream);
+
 /* Gated combine (reference_moe/train.py:1287-1288): combined bf16 [tokens,
  * width] = sum over the token's top_k bucket rows, in bucket order, of
  * bf16(out[p] * bf16(gate)), accumulated in bf16 like zeros.at[rows].add.

@@ -244,3 +244,48 @@ def test_fused_input_backward_equals_two_passes(tokens, width, experts, top_k):
               *(t.data_ptr() for t in tail), dx2.data_ptr(), dw2.data_ptr(), tokens, width, experts, top_k, s)
     assert torch.equal(dx1, dx2)
     torch.testing.assert_close(dw1, dw2, rtol=1e-6, atol=1e-5 * float(dw1.abs().max()))
+
+
+@pytest.mark.parametrize("counts,width,hidden", [
+    ([5], 8, 16),                        # one expert, a corner of a tile
+    ([0, 33, 0, 7], 264, 72),            # empty experts (their gradients are zero), ragged tiles
+    ([3000, 10, 0, 200], 64, 520),       # one expert far over the even share: sliced, added with atomics
+    ([700, 650, 720, 690, 10, 1, 0, 629], 256, 256),
+])
+def test_backward_gemms_in_one_launch(counts, width, hidden):
+    """gptrig_moe_bwd_gemms against float64 for every kind of bucket: stored,
+    sliced and empty ones; the outputs start as NaN.
+
+    Bound: bf16 products are exact in float32 and a sum of n rounds at most n
+    times, 2^-24 n of the magnitudes; dgrouped is rounded to bf16 once."""
+    from gptrig import _lib
+
+    g = torch.Generator().manual_seed(width + hidden)
+    E, R = len(counts), sum(counts)
+    rnd = lambda *s: torch.randn(s, generator=g).bfloat16().to(DEV)  # noqa: E731
+    grouped, dpre, hid, dout, up_w = rnd(R, width), rnd(R, hidden), rnd(R, hidden), rnd(R, width), rnd(E, width, hidden)
+    cnt = torch.tensor(counts, dtype=torch.int32, device=DEV)
+    nan = lambda *s, dtype=torch.float32: torch.full(s, float("nan"), dtype=dtype, device=DEV)  # noqa: E731
+    up_dw, up_db, down_dw, down_db = nan(E, width, hidden), nan(E, hidden), nan(E, hidden, width), nan(E, width)
+    dgrouped = nan(R, width, dtype=torch.bfloat16)
+    print(f"routed backward products counts={counts} width={width} hidden={hidden}", flush=True)
+    _lib.call("gptrig_moe_bwd_gemms", grouped.data_ptr(), dpre.data_ptr(), hid.data_ptr(), dout.data_ptr(),
+              up_w.data_ptr(), cnt.data_ptr(), up_dw.data_ptr(), up_db.data_ptr(), down_dw.data_ptr(),
+              down_db.data_ptr(), dgrouped.data_ptr(), R, width, hidden, E, _lib.stream())
+    worst, at = 0.0, 0
+    for e, n in enumerate(counts):
+        a, p, h, o = (t[at:at + n].double() for t in (grouped, dpre, hid, dout))
+        eps = (n + 2) * 2.0 ** -24
+        for got, x, y in ((up_dw[e], a, p), (down_dw[e], h, o)):
+            bound = eps * (x.abs().T @ y.abs()) + 1e-30
+            worst = max(worst, float(((got.double() - x.T @ y).abs() / bound).max()))
+        for got, y in ((up_db[e], p), (down_db[e], o)):
+            worst = max(worst, float(((got.double() - y.sum(0)).abs() / (eps * y.abs().sum(0) + 1e-30)).max()))
+        w = up_w[e].double()
+        want = p @ w.T
+        bound = (hidden + 2) * 2.0 ** -24 * (p.abs() @ w.abs().T) + 2.0 ** -8 * want.abs() + 1e-30
+        if n:
+            worst = max(worst, float(((dgrouped[at:at + n].double() - want).abs() / bound).max()))
+        at += n
+    print(f"  error / bound {worst:.3f}", flush=True)
+    assert worst <= 1
