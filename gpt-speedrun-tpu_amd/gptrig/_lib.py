@@ -68,6 +68,7 @@ SIGNATURES: dict[str, tuple] = {
     "gptrig_rope_table": (I, [P, P, I, I, P]),
     "gptrig_rope_fwd": (I, [P, L, I, I, I, I, P, P, P]),
     "gptrig_rope_bwd": (I, [P, L, I, I, I, I, P, P, P]),
+    "gptrig_rope_copy": (I, [P, L, L, L, P, I, I, I, I, I, P, P, P]),
     "gptrig_bias_rope_fwd": (I, [P, L, I, I, P, I, I, I, P, P, P]),
     "gptrig_embedding_fwd": (I, [P, P, P, I, I, I, P]),
     "gptrig_embedding_bwd": (I, [P, P, P, I, I, I, P]),

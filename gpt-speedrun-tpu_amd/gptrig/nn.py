@@ -131,20 +131,34 @@ def bias_rope_inplace(buf: torch.Tensor, bias: torch.Tensor, seq: int, heads: in
               head_dim, c.data_ptr(), s.data_ptr(), _lib.stream())
 
 
+def _rotated(x: torch.Tensor, backward: bool) -> torch.Tensor:
+    """The rotation of a bf16 BTHD tensor of any strides into a new contiguous one."""
+
+    B, S, H, D = x.shape
+    if x.numel() >= 2 ** 34:  # past the out-of-place pass's 32-bit chunk index
+        y = x.contiguous().clone()
+        rope_inplace(y, H * D, B * S, S, H, D, backward=backward)
+        return y
+    if x.stride(3) != 1 or any(s % 8 for s in x.stride()[:3]) or x.data_ptr() % 16:
+        x = x.contiguous()
+        if x.data_ptr() % 16:
+            x = x.clone()
+    y = torch.empty((B, S, H, D), dtype=x.dtype, device=x.device)
+    if y.numel():
+        c, s = rope_tables(S, D, x.device)
+        _lib.call("gptrig_rope_copy", x.data_ptr(), *x.stride()[:3], y.data_ptr(), B, S, H, D, int(backward),
+                  c.data_ptr(), s.data_ptr(), _lib.stream())
+    return y
+
+
 class _Rotary(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):
-        B, S, H, D = x.shape
-        y = x.contiguous().clone()
-        rope_inplace(y, H * D, B * S, S, H, D)
-        return y
+        return _rotated(x, False)
 
     @staticmethod
     def backward(ctx, dy):
-        B, S, H, D = dy.shape
-        g = dy.to(BF16).contiguous().clone()
-        rope_inplace(g, H * D, B * S, S, H, D, backward=True)
-        return g
+        return _rotated(dy.to(BF16), True)
 
 
 def apply_rotary(x: torch.Tensor) -> torch.Tensor:

@@ -276,6 +276,14 @@ int gptrig_rope_fwd(void* x, int64_t row_stride, int rows, int seq, int heads, i
                     const void* sin_table, void* stream);
 int gptrig_rope_bwd(void* dx, int64_t row_stride, int rows, int seq, int heads, int head_dim,
                     const void* cos_table, const void* sin_table, void* stream);
+/* The rotation (its transpose with backward != 0) out of place: y bf16 [batch,
+ * seq, heads, head_dim] contiguous from a view x with element strides
+ * stride_b, stride_s, stride_h (multiples of 8) and unit stride along head_dim
+ * (a multiple of 8); x and y 16-byte aligned, y must not overlap x, fewer than
+ * 2^34 elements. */
+int gptrig_rope_copy(const void* x, int64_t stride_b, int64_t stride_s, int64_t stride_h, void* y, int batch, int seq,
+                     int heads, int head_dim, int backward, const void* cos_table, const void* sin_table,
+                     void* stream);
 /* The fused projection's bias add and the RoPE of its q / k columns in one
  * in-place pass (rig/nn.py:55-56 then :36-52, recipes/reference/train.py:
  * 1136-1142): columns [0, cols) of each row become bf16(x + bias[column]),

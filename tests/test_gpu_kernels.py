@@ -838,3 +838,33 @@ def test_grouped_weight_gradients(n, shapes):
     items[0].cols_out = 12
     with pytest.raises(RuntimeError):
         _lib.call("gptrig_weight_grads", items, 1, n, _lib.stream())
+
+
+@pytest.mark.parametrize("B,S,H,D,layout", [
+    (1, 1, 1, 8, "contiguous"), (2, 33, 3, 64, "packed"), (1, 129, 2, 128, "heads first"),
+    (3, 20, 5, 24, "odd base"), (2, 7, 2, 16, "expanded"), (1, 5, 3, 8, "strided dims"), (0, 4, 2, 8, "contiguous"),
+])
+def test_apply_rotary_of_any_strides(B, S, H, D, layout):
+    """The out-of-place rotation, forward and backward, equals the oracle bit
+    for bit whatever the strides, base and size of the input and gradient."""
+
+    from gptrig import nn
+
+    x = {
+        "contiguous": lambda: randn((B, S, H, D), 1),
+        "packed": lambda: randn((B, S, 3, H, D), 2)[:, :, 1],
+        "heads first": lambda: randn((B, H, S, D), 3).transpose(1, 2),
+        "odd base": lambda: randn((B * S * H * D + 3,), 4)[3:].view(B, S, H, D),
+        "expanded": lambda: randn((1, S, 1, D), 5).expand(B, S, H, D),
+        "strided dims": lambda: randn((B, S, H, 2 * D), 6)[..., ::2],
+    }[layout]()
+    # The same strides on the device (a copy to it would compact the view).
+    storage = torch.empty(x.untyped_storage().nbytes() // 2, dtype=torch.bfloat16)
+    storage.copy_(torch.as_strided(x, storage.shape, (1,), 0))
+    on = lambda: torch.as_strided(storage.to(DEV), x.shape, x.stride(), x.storage_offset())  # noqa: E731
+    print(f"apply_rotary {tuple(x.shape)} {layout} strides {x.stride()}", flush=True)
+    xg = on().requires_grad_()
+    y = nn.apply_rotary(xg)
+    assert y.is_contiguous() and torch.equal(y.detach().cpu(), onn.apply_rotary(x))
+    (dx,) = torch.autograd.grad(y, xg, on())
+    assert torch.equal(dx.cpu(), onn.apply_rotary_backward(x))
