@@ -768,6 +768,28 @@ __global__ void cast_f32_bf16_kernel(const float* __restrict__ x, bf16* __restri
   }
 }
 
+// Several such casts in one launch (blockIdx.y = the array).
+struct CastMany {
+  const float* x[8];
+  bf16* y[8];
+  int64_t n[8];
+};
+__global__ void __launch_bounds__(256) cast_many_kernel(CastMany c) {
+  const float* const x = c.x[blockIdx.y];
+  bf16* const y = c.y[blockIdx.y];
+  const int64_t n = c.n[blockIdx.y];
+  // (Both arrays are 16-byte aligned.)
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (int64_t)gridDim.x * 2048) {
+    if (i + 8 <= n) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(x + i), b = *reinterpret_cast<const f32x4*>(x + i + 4);
+      *reinterpret_cast<bf16x8*>(y + i) = bf16x8{(bf16)a[0], (bf16)a[1], (bf16)a[2], (bf16)a[3],
+                                                 (bf16)b[0], (bf16)b[1], (bf16)b[2], (bf16)b[3]};
+    } else {
+      for (int64_t j = i; j < n; ++j) y[j] = (bf16)x[j];
+    }
+  }
+}
+
 // out += weight * sum(x)  (fp32 atomics, one per block)
 __global__ void __launch_bounds__(256) weighted_sum_kernel(const float* __restrict__ x, int64_t n, float weight,
                                                            float* __restrict__ out) {
@@ -1128,6 +1150,27 @@ int gptrig_cast_f32_bf16(const float* x, void* y, int64_t n, void* stream) {
   if (n < 0) return GPTRIG_E_SHAPE;
   if (n == 0) return GPTRIG_OK;
   cast_f32_bf16_kernel<<<ceil_div(ceil_div(n, 4), 256), 256, 0, (hipStream_t)stream>>>(x, (bf16*)y, n);
+  GPTRIG_CHECK_LAUNCH();
+  return GPTRIG_OK;
+}
+
+int gptrig_cast_f32_bf16_many(const float* const* x, void* const* y, const int64_t* n, int count, void* stream) {
+  if (count < 0 || count > 8) return GPTRIG_E_SHAPE;
+  if (count == 0) return GPTRIG_OK;
+  if (!x || !y || !n) return GPTRIG_E_NULL;
+  CastMany c{};
+  int64_t most = 0;
+  for (int i = 0; i < count; ++i) {
+    if (!x[i] || !y[i]) return GPTRIG_E_NULL;
+    if (n[i] < 0 || (((uintptr_t)x[i] | (uintptr_t)y[i]) & 15)) return GPTRIG_E_SHAPE;
+    c.x[i] = x[i];
+    c.y[i] = (bf16*)y[i];
+    c.n[i] = n[i];
+    most = n[i] > most ? n[i] : most;
+  }
+  if (most == 0) return GPTRIG_OK;
+  const int64_t blocks = (most + 2047) / 2048;
+  cast_many_kernel<<<dim3((unsigned)(blocks < 4096 ? blocks : 4096), (unsigned)count), 256, 0, (hipStream_t)stream>>>(c);
   GPTRIG_CHECK_LAUNCH();
   return GPTRIG_OK;
 }

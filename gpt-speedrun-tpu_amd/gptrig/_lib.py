@@ -77,6 +77,7 @@ SIGNATURES: dict[str, tuple] = {
     "gptrig_finalize_norm": (I, [P, I, F, P, P, P, F, P, P]),
     "gptrig_transpose_bf16": (I, [P, P, I, I, P]),
     "gptrig_cast_f32_bf16": (I, [P, P, L, P]),
+    "gptrig_cast_f32_bf16_many": (I, [P, P, P, I, P]),
     "gptrig_weighted_sum": (I, [P, L, F, P, P]),
     "gptrig_masked_sum": (I, [P, P, L, P, P]),
     "gptrig_fill_f32": (I, [P, L, F, P]),
@@ -92,6 +93,10 @@ SIGNATURES: dict[str, tuple] = {
     "gptrig_moe_gather_bwd": (I, [P, P, P, I, I, I, P]),
     "gptrig_moe_stats": (I, [P, P, P, P, I, I, I, P, P, P, P]),
     "gptrig_moe_router_bwd": (I, [P, P, P, P, P, P, P, P, P, I, I, I, I, P]),
+    "gptrig_routed_saved_bytes": (Z, [I, I, I, I, I]),
+    "gptrig_routed_scratch_bytes": (Z, [I, I, I, I, I, I]),
+    "gptrig_routed_fwd": (I, [P, P, P, P, P, P, P, P, P, P, P, Z, P, Z, I, I, I, I, I, P]),
+    "gptrig_routed_bwd": (I, [P, P, P, P, P, P, P, Z, P, P, P, P, P, P, P, Z, I, I, I, I, I, P]),
     "gptrig_moe_input_bwd": (I, [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, P]),
 }
 
@@ -133,7 +138,9 @@ def query(name: str, *args) -> int:
 def stream() -> int:
     """Handle of torch's current HIP stream on the current device."""
 
-    return torch.cuda.current_stream().cuda_stream
+    # (The raw handle: torch.cuda.current_stream() builds a Stream object around
+    # it, 4 us a call on the host, as much as a launch.)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

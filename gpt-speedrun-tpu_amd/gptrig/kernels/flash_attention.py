@@ -13,6 +13,7 @@ zero-padded to the next kernel size, which leaves scores unchanged.
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import Callable, Literal
 
@@ -118,16 +119,16 @@ def validate_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
 def _kernel_view(t: torch.Tensor) -> torch.Tensor:
     """A BHSD view the kernel accepts: unit last stride, 8-element strides, 16-byte base."""
 
-    if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:3]) or t.data_ptr() % 16:
+    a, b, c, d = t.stride()
+    if d != 1 or (a | b | c) % 8 or t.data_ptr() % 16:
         t = t.contiguous()
     return t
 
 
-def _strides(*ts: torch.Tensor) -> torch.Tensor:
-    flat = []
-    for t in ts:
-        flat.extend(t.stride()[:3])
-    return torch.tensor(flat, dtype=torch.int64)
+def _strides(*ts: torch.Tensor):
+    """The (batch, head, seq) strides of each tensor as the int64 array the entry points read."""
+
+    return (ctypes.c_int64 * (3 * len(ts)))(*(s for t in ts for s in t.stride()[:3]))
 
 
 def flash_forward(q, k, v, segment_ids, scale: float):
@@ -139,7 +140,7 @@ def flash_forward(q, k, v, segment_ids, scale: float):
     lse = torch.empty((B, H, S), dtype=torch.float32, device=q.device)
     st = _strides(q, k, v, o)
     _lib.call("gptrig_attn_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.ptr(segment_ids), o.data_ptr(),
-              lse.data_ptr(), B, H, S, D, st.data_ptr(), float(scale), _lib.stream())
+              lse.data_ptr(), B, H, S, D, st, float(scale), _lib.stream())
     return o, lse
 
 
@@ -153,7 +154,7 @@ def flash_backward(q, k, v, o, lse, do, segment_ids, scale: float):
     st = _strides(q, k, v, o, do, dq, dk, dv)
     _lib.call("gptrig_attn_bwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
               lse.data_ptr(), _lib.ptr(segment_ids), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(),
-              ws.numel(), B, H, S, D, st.data_ptr(), float(scale), _lib.stream())
+              ws.numel(), B, H, S, D, st, float(scale), _lib.stream())
     return dq, dk, dv
 
 

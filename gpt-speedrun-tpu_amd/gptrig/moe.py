@@ -10,6 +10,8 @@ run entirely in ``libgptrig.so``; torch only allocates.
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -39,12 +41,22 @@ def _route(flat: torch.Tensor, router_w: torch.Tensor, experts: int, top_k: int)
     return logits, probs, chosen, gate, counts, rows, position
 
 
-def _gmm(lhs, rhs, transposed: bool, counts, bias, mode: int, pre, rows: int, k: int, n: int,
-         experts: int) -> torch.Tensor:
-    out = torch.empty((rows, n), dtype=BF16, device=lhs.device)
-    _lib.call("gptrig_moe_gmm", lhs.data_ptr(), lhs.stride(0), rhs.data_ptr(), int(transposed), counts.data_ptr(),
-              None if bias is None else bias.data_ptr(), mode, out.data_ptr(), None if pre is None else pre.data_ptr(),
-              n, rows, k, n, experts, _lib.stream())
+def _bf16(*tensors: torch.Tensor) -> list[torch.Tensor]:
+    """Contiguous bf16 copies (float32 tensors in one launch); bf16 ones as they are."""
+
+    out = [t if t.dtype == F32 else t.to(BF16).contiguous() for t in tensors]
+    todo = [i for i, t in enumerate(out) if t.dtype == F32]
+    if not todo:
+        return out
+    src = [out[i].contiguous() for i in todo]
+    src = [t.clone() if t.data_ptr() % 16 else t for t in src]  # (a view into an arena at an odd element)
+    dst = [torch.empty(t.shape, dtype=BF16, device=t.device) for t in src]
+    n = len(src)
+    _lib.call("gptrig_cast_f32_bf16_many", (ctypes.c_void_p * n)(*(t.data_ptr() for t in src)),
+              (ctypes.c_void_p * n)(*(t.data_ptr() for t in dst)), (ctypes.c_int64 * n)(*(t.numel() for t in src)), n,
+              _lib.stream())
+    for i, t in zip(todo, dst):
+        out[i] = t
     return out
 
 
@@ -54,66 +66,47 @@ class _RoutedMLP(torch.autograd.Function):
         batch, length, width = x.shape
         tokens = batch * length
         hidden_width = up_w.shape[-1]
-        R = tokens * top_k
+        dev = x.device
         flat = x.reshape(tokens, width).to(BF16).contiguous()
         rw = router_w.to(F32).contiguous()
-        logits, probs, chosen, gate, counts, rows, position = _route(flat, rw, experts, top_k)
-        upw, upb = up_w.to(BF16).contiguous(), up_b.to(BF16).contiguous()
-        dnw, dnb = down_w.to(BF16).contiguous(), down_b.to(BF16).contiguous()
-        grouped = torch.empty((R, width), dtype=BF16, device=x.device)
-        _lib.call("gptrig_moe_gather_rows", flat.data_ptr(), rows.data_ptr(), grouped.data_ptr(), R, width,
+        upw, upb, dnw, dnb = _bf16(up_w, up_b, down_w, down_b)
+        sizes = (tokens, width, hidden_width, experts, top_k)
+        saved = _lib.workspace(_lib.query("gptrig_routed_saved_bytes", *sizes), dev)
+        scratch = _lib.workspace(_lib.query("gptrig_routed_scratch_bytes", *sizes, 0), dev)
+        combined = torch.empty((tokens, width), dtype=BF16, device=dev)
+        mean_probability = torch.empty(experts, dtype=F32, device=dev)
+        load = torch.empty(experts, dtype=F32, device=dev)
+        summary = torch.empty(3, dtype=F32, device=dev)
+        _lib.call("gptrig_routed_fwd", flat.data_ptr(), rw.data_ptr(), upw.data_ptr(), upb.data_ptr(), dnw.data_ptr(),
+                  dnb.data_ptr(), combined.data_ptr(), mean_probability.data_ptr(), load.data_ptr(),
+                  summary.data_ptr(), saved.data_ptr(), saved.numel(), scratch.data_ptr(), scratch.numel(), *sizes,
                   _lib.stream())
-        pre = torch.empty((R, hidden_width), dtype=BF16, device=x.device)
-        hidden = _gmm(grouped, upw, False, counts, upb, 1, pre, R, width, hidden_width, experts)
-        out = _gmm(hidden, dnw, False, counts, dnb, 0, None, R, hidden_width, width, experts)
-        combined = torch.empty((tokens, width), dtype=BF16, device=x.device)
-        s = _lib.stream()
-        _lib.call("gptrig_moe_combine", out.data_ptr(), position.data_ptr(), gate.data_ptr(), combined.data_ptr(),
-                  tokens, width, top_k, s)
-        mean_probability = torch.empty(experts, dtype=F32, device=x.device)
-        load = torch.empty(experts, dtype=F32, device=x.device)
-        summary = torch.empty(3, dtype=F32, device=x.device)
-        _lib.call("gptrig_moe_stats", logits.data_ptr(), probs.data_ptr(), gate.data_ptr(), counts.data_ptr(), tokens,
-                  experts, top_k, mean_probability.data_ptr(), load.data_ptr(), summary.data_ptr(), s)
-        ctx.save_for_backward(flat, grouped, rw, upw, dnw, probs, chosen, gate, counts, position, pre, hidden, out)
-        ctx.meta = (batch, length, width, hidden_width, experts, top_k, x.dtype, router_w.dtype, up_w.dtype,
-                    up_b.dtype, down_w.dtype, down_b.dtype)
+        ctx.save_for_backward(flat, rw, upw, dnw, saved)
+        ctx.meta = (batch, length, sizes, x.dtype, router_w.dtype, up_w.dtype, up_b.dtype, down_w.dtype, down_b.dtype)
         ctx.mark_non_differentiable(load, summary)
         return combined.reshape(batch, length, width).to(x.dtype), mean_probability, load, summary
 
     @staticmethod
     def backward(ctx, dcombined, dmean_probability, _dload, _dsummary):
-        flat, grouped, rw, upw, dnw, probs, chosen, gate, counts, position, pre, hidden, out = ctx.saved_tensors
-        batch, length, width, hidden_width, experts, top_k, xdt, rdt, uwdt, ubdt, dwdt, dbdt = ctx.meta
-        tokens = batch * length
-        R = tokens * top_k
+        flat, rw, upw, dnw, saved = ctx.saved_tensors
+        batch, length, sizes, xdt, rdt, uwdt, ubdt, dwdt, dbdt = ctx.meta
+        tokens, width, hidden_width, experts, top_k = sizes
         dev = flat.device
-        s = _lib.stream()
         if dcombined is None:
             dcombined = torch.zeros((tokens, width), dtype=BF16, device=dev)
         dc = dcombined.reshape(tokens, width).to(BF16).contiguous()
-        dout = torch.empty((R, width), dtype=BF16, device=dev)
-        dgate = torch.empty(R, dtype=F32, device=dev)
-        _lib.call("gptrig_moe_combine_bwd", dc.data_ptr(), out.data_ptr(), position.data_ptr(), gate.data_ptr(),
-                  dout.data_ptr(), dgate.data_ptr(), tokens, width, top_k, s)
+        dmp = None if dmean_probability is None else dmean_probability.to(F32).contiguous()
+        dx = torch.empty((tokens, width), dtype=BF16, device=dev)
         d_up_w = torch.empty((experts, width, hidden_width), dtype=F32, device=dev)
         d_up_b = torch.empty((experts, hidden_width), dtype=F32, device=dev)
         d_down_w = torch.empty((experts, hidden_width, width), dtype=F32, device=dev)
         d_down_b = torch.empty((experts, width), dtype=F32, device=dev)
-        d_router = torch.zeros((width, experts), dtype=F32, device=dev)
-        # d(pre) = (dout W_down^T) * gelu'(pre); then the weight gradients of both
-        # projections and d(grouped) = dpre W_up^T.
-        dpre = _gmm(dout, dnw, True, counts, None, 2, pre, R, width, hidden_width, experts)
-        dgrouped = torch.empty((R, width), dtype=BF16, device=dev)
-        _lib.call("gptrig_moe_bwd_gemms", grouped.data_ptr(), dpre.data_ptr(), hidden.data_ptr(), dout.data_ptr(),
-                  upw.data_ptr(), counts.data_ptr(), d_up_w.data_ptr(), d_up_b.data_ptr(), d_down_w.data_ptr(),
-                  d_down_b.data_ptr(), dgrouped.data_ptr(), R, width, hidden_width, experts, s)
-        dx = torch.empty((tokens, width), dtype=BF16, device=dev)
-        dmp = None if dmean_probability is None else dmean_probability.to(F32).contiguous()
-        _lib.call("gptrig_moe_input_bwd", dgrouped.data_ptr(), position.data_ptr(), flat.data_ptr(), rw.data_ptr(),
-                  probs.data_ptr(), chosen.data_ptr(), gate.data_ptr(), dgate.data_ptr(),
-                  None if dmp is None else dmp.data_ptr(), dx.data_ptr(), d_router.data_ptr(), tokens, width, experts,
-                  top_k, s)
+        d_router = torch.empty((width, experts), dtype=F32, device=dev)
+        scratch = _lib.workspace(_lib.query("gptrig_routed_scratch_bytes", *sizes, 1), dev)
+        _lib.call("gptrig_routed_bwd", dc.data_ptr(), _lib.ptr(dmp), flat.data_ptr(), rw.data_ptr(), upw.data_ptr(),
+                  dnw.data_ptr(), saved.data_ptr(), saved.numel(), dx.data_ptr(), d_router.data_ptr(),
+                  d_up_w.data_ptr(), d_up_b.data_ptr(), d_down_w.data_ptr(), d_down_b.data_ptr(), scratch.data_ptr(),
+                  scratch.numel(), *sizes, _lib.stream())
         return (dx.reshape(batch, length, width).to(xdt), d_router.to(rdt), d_up_w.to(uwdt), d_up_b.to(ubdt),
                 d_down_w.to(dwdt), d_down_b.to(dbdt), None, None)
 

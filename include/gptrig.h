@@ -329,6 +329,9 @@ int gptrig_transpose_bf16(const void* src, void* dst, int rows, int cols, void* 
 
 /* Small helpers of the step: f32 -> bf16 cast, out += weight * sum(x), fill. */
 int gptrig_cast_f32_bf16(const float* x, void* y, int64_t n, void* stream);
+/* Up to 8 such casts in one launch; x, y and n are host arrays of `count`, the
+ * arrays they name 16-byte aligned. */
+int gptrig_cast_f32_bf16_many(const float* const* x, void* const* y, const int64_t* n, int count, void* stream);
 int gptrig_weighted_sum(const float* x, int64_t n, float weight, float* out, void* stream);
 /* Masked loss sum of eval_step (recipes/reference/train.py:1493-1525):
  * out[0] += sum(x * mask), out[1] += sum(mask), x and mask f32 [n]. */
@@ -436,6 +439,26 @@ int gptrig_moe_input_bwd(const void* dgrouped, const int32_t* position, const vo
                          const float* probs, const int32_t* chosen, const float* gate, const float* dgate,
                          const float* dmean_probability, void* dx, float* dw_router, int tokens, int width,
                          int experts, int top_k, void* stream);
+
+/* routed_mlp_local (reference_moe/train.py:1230-1307) and its VJP, the entry
+ * points above in order behind one call each.  x bf16 [tokens, width],
+ * router_w f32 [width, experts], up_w / down_w bf16 [experts, width, hidden] /
+ * [experts, hidden, width], up_b / down_b bf16; outputs as gptrig_moe_combine
+ * and gptrig_moe_stats.  saved (gptrig_routed_saved_bytes) carries what the
+ * backward needs from the forward; scratch (gptrig_routed_scratch_bytes of the
+ * direction) is free again when the call's work is done.  Both 256-byte
+ * aligned.  The backward overwrites its gradients (f32 but dx, bf16);
+ * dmean_probability may be NULL. */
+size_t gptrig_routed_saved_bytes(int tokens, int width, int hidden, int experts, int top_k);
+size_t gptrig_routed_scratch_bytes(int tokens, int width, int hidden, int experts, int top_k, int backward);
+int gptrig_routed_fwd(const void* x, const float* router_w, const void* up_w, const void* up_b, const void* down_w,
+                      const void* down_b, void* combined, float* mean_probability, float* load, float* summary,
+                      void* saved, size_t saved_bytes, void* scratch, size_t scratch_bytes, int tokens, int width,
+                      int hidden, int experts, int top_k, void* stream);
+int gptrig_routed_bwd(const void* dcombined, const float* dmean_probability, const void* x, const float* router_w,
+                      const void* up_w, const void* down_w, void* saved, size_t saved_bytes, void* dx, float* d_router,
+                      float* d_up_w, float* d_up_b, float* d_down_w, float* d_down_b, void* scratch,
+                      size_t scratch_bytes, int tokens, int width, int hidden, int experts, int top_k, void* stream);
 
 #ifdef __cplusplus
 }

@@ -289,3 +289,33 @@ def test_backward_gemms_in_one_launch(counts, width, hidden):
         at += n
     print(f"  error / bound {worst:.3f}", flush=True)
     assert worst <= 1
+
+
+@pytest.mark.parametrize("dtypes,offset", [("ffff", 0), ("fbfb", 0), ("ffff", 1), ("bbbb", 0), ("hfff", 0)])
+def test_routed_weights_of_any_dtype_and_base(dtypes, offset):
+    """The weight casts in front of the routed MLP: float32 parameters
+    (16-byte aligned or not, sizes with a tail of 8), bf16 and half ones give
+    the layer the same bf16 operands as .to(bfloat16), and gradients come back in
+    each parameter's dtype."""
+    from gptrig import _lib
+    from gptrig.moe import _bf16, routed_mlp_local
+
+    kinds = {"f": torch.float32, "b": torch.bfloat16, "h": torch.float16}
+    x, router_w, *params = draw(1, 9, 24, 40, 3, 3)
+    on = []
+    for t, k in zip(params, dtypes):
+        flat = torch.zeros(t.numel() + offset, dtype=kinds[k], device=DEV)
+        flat[offset:] = t.reshape(-1).to(kinds[k]).to(DEV)
+        on.append(flat[offset:].view(t.shape))
+    print(f"routed weights {dtypes} base {[t.data_ptr() % 16 for t in on]}", flush=True)
+    for got, t in zip(_bf16(*on), on):
+        assert got.is_contiguous() and torch.equal(got, t.to(torch.bfloat16))
+    leaves = [t.detach().requires_grad_() for t in on]
+    out, *_ = routed_mlp_local(x.to(DEV), router_w.to(DEV), *leaves, experts=3, top_k=2)
+    grads = torch.autograd.grad(out.float().sum(), leaves)
+    assert all(g.dtype == t.dtype and g.shape == t.shape and torch.isfinite(g).all() for g, t in zip(grads, leaves))
+    same = [t.detach().to(torch.bfloat16).requires_grad_() for t in on]
+    ref, *_ = routed_mlp_local(x.to(DEV), router_w.to(DEV), *same, experts=3, top_k=2)
+    assert torch.equal(out, ref)
+    saved = _lib.query("gptrig_routed_saved_bytes", 9, 24, 40, 3, 2)
+    assert saved > 0 and _lib.query("gptrig_routed_saved_bytes", 0, 24, 40, 3, 2) == 0
