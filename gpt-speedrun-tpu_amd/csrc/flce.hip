@@ -1138,6 +1138,31 @@ KeepPlan keep_plan(int n, int d, int vocab, bool accumulate) {
   return best;
 }
 
+// dW (+)= G^T h and dh = G W of one token chunk: gt blocked with `blk` rows per
+// 32 tokens, dh through the f32 [n, d] buffer dh_acc to bf16.
+int grad_gemms_launch(const KeepPlan& plan, bf16* gt, int blk, const bf16* h, const bf16* w, void* dhidden,
+                      float* dh_acc, float* dweight, bool accumulate, int n, int d, int vocab, hipStream_t s) {
+  if (!accumulate && plan.dw_mode == 2) {
+    const int64_t total = (int64_t)vocab * d;
+    zero_f32_kernel<<<ceil_div(ceil_div(total, 4), 256), 256, 0, s>>>(dweight, total);
+    GPTRIG_CHECK_LAUNCH();
+  }
+  const int64_t total = (int64_t)n * d;
+  if (plan.dh_mode == 2) {
+    zero_f32_kernel<<<ceil_div(ceil_div(total, 4), 256), 256, 0, s>>>(dh_acc, total);
+    GPTRIG_CHECK_LAUNCH();
+  }
+  const unsigned n_dh = tiles_of(n, d) * (unsigned)plan.dh_split;
+  const unsigned n_dw = tiles_of(vocab, d) * (unsigned)plan.dw_split;
+  flce_keep_gemms_kernel<<<n_dh + n_dw, gemm::THREADS, 0, s>>>(
+      Operand{gt, n, blk}, Operand{w, d}, Operand{h, d}, n, d, vocab, plan.dh_split, plan.dw_split, dh_acc,
+      plan.dh_mode, dweight, plan.dw_mode, (int)n_dh, (int)n_dw, plan.dh_first);
+  GPTRIG_CHECK_LAUNCH();
+  f32_to_bf16_kernel<<<ceil_div(ceil_div(total, 4), 256), 256, 0, s>>>(dh_acc, (bf16*)dhidden, total);
+  GPTRIG_CHECK_LAUNCH();
+  return GPTRIG_OK;
+}
+
 int flce_fwd_launch(const void* hidden, const void* weight, const int32_t* targets, float* losses, float* lse,
                     void* workspace, int n, int d, int vocab, int semantic_vocab, hipStream_t s, void* keep) {
   const int ntiles = ceil_div(vocab, BM);
@@ -1335,18 +1360,7 @@ int gptrig_flce_bwd_keep(const void* hidden, const void* weight, const int32_t* 
   // (flce_keep_gemms_kernel), split as keep_plan estimates fastest.  With few
   // tokens per call (a token chunk of a bounded run) the dW tiles are short and
   // the dh tiles long; with many, both are long enough to need no split.
-  const int vc = vocab;
   const KeepPlan plan = keep_plan(n, d, vocab, accumulate_dweight != 0);
-  if (!accumulate_dweight && plan.dw_mode == 2) {
-    const int64_t total = (int64_t)vocab * d;
-    zero_f32_kernel<<<ceil_div(ceil_div(total, 4), 256), 256, 0, s>>>(dweight, total);
-    GPTRIG_CHECK_LAUNCH();
-  }
-  if (plan.dh_mode == 2) {
-    const int64_t total = (int64_t)n * d;
-    zero_f32_kernel<<<ceil_div(ceil_div(total, 4), 256), 256, 0, s>>>(dh_acc, total);
-    GPTRIG_CHECK_LAUNCH();
-  }
   const int halves = 2 * ceil_div(vocab, BM);
   flce_keep_alpha_kernel<<<dim3((unsigned)ceil_div(n / 4, 256), (unsigned)halves), 256, 0, s>>>(
       alpha, halves, n, semantic_vocab, targets, lse, cotangent, cotangent_scale);
@@ -1355,15 +1369,90 @@ int gptrig_flce_bwd_keep(const void* hidden, const void* weight, const int32_t* 
   flce_keep_rescale_kernel<<<rgrid, 256, 0, s>>>(gt, alpha, n, vocab, semantic_vocab, targets, cotangent,
                                                   cotangent_scale);
   GPTRIG_CHECK_LAUNCH();
-  const unsigned n_dh = tiles_of(n, d) * (unsigned)plan.dh_split;
-  const unsigned n_dw = tiles_of(vc, d) * (unsigned)plan.dw_split;
-  flce_keep_gemms_kernel<<<n_dh + n_dw, gemm::THREADS, 0, s>>>(
-      Operand{gt, n, keep_rows(vocab)}, Operand{Wp, d}, Operand{Hp, d}, n, d, vc, plan.dh_split, plan.dw_split, dh_acc,
-      plan.dh_mode, dweight, plan.dw_mode, (int)n_dh, (int)n_dw, plan.dh_first);
-  GPTRIG_CHECK_LAUNCH();
-  const int64_t total = (int64_t)n * d;
-  f32_to_bf16_kernel<<<ceil_div(ceil_div(total, 4), 256), 256, 0, s>>>(dh_acc, (bf16*)dhidden, total);
-  GPTRIG_CHECK_LAUNCH();
+  return grad_gemms_launch(plan, gt, keep_rows(vocab), Hp, Wp, dhidden, dh_acc, dweight, accumulate_dweight != 0, n, d,
+                           vocab, s);
+}
+
+// Bytes of gptrig_flce_bwd_tokens' workspace per token of a chunk: the bf16
+// G^T column and the f32 dh row.
+static int64_t token_bytes(int d, int vocab) { return 2ll * vocab + 4ll * d; }
+
+int gptrig_flce_token_chunk(int n, int d, int vocab, int64_t max_bytes) {
+  if (n <= 0 || d <= 0 || vocab <= 0) return 0;
+  // (A chunk's columns are stored in blocks of 32 tokens; 4 KB for alignment.)
+  const int64_t fit = (max_bytes - 4096) / token_bytes(d, vocab) / 32 * 32;
+  if (fit >= n) return n;
+  if (fit < BN) return 0;
+  // Whole token tiles; the size whose chunks cost least, each its logit tiles
+  // in rounds of CUs (d / 32 stages and about 8 for the epilogue), the two
+  // products (V / 32 stages for each dh tile, n / 32 and about 20 for each dW
+  // tile, which reads and writes its 256 KB) and about 30 stages of launches.
+  const double cus = gemm::device_cus();
+  int best = BN;
+  double best_cost = 1e300;
+  for (int t = BN; t <= fit; t += BN) {
+    const double k1 = (double)ceil_div((int64_t)tiles_of(vocab, t), (int64_t)cus) * (d / 32.0 + 8.0);
+    const double products = (tiles_of(t, d) * (vocab / 32.0) + tiles_of(vocab, d) * (t / 32.0 + 20.0)) / cus;
+    const double cost = ceil_div(n, t) * (k1 + products + 30.0);
+    if (cost < best_cost * 0.999) {
+      best_cost = cost;
+      best = t;
+    }
+  }
+  return best;
+}
+
+size_t gptrig_flce_bwd_tokens_workspace_bytes(int n, int d, int vocab, int token_chunk) {
+  if (n <= 0 || d <= 0 || vocab <= 0 || token_chunk <= 0) return 0;
+  const int c = token_chunk < n ? token_chunk : n;
+  return align256((size_t)vocab * ceil_div(c, 32) * 32 * sizeof(bf16)) + align256((size_t)c * d * sizeof(float));
+}
+
+// The recompute backward over token chunks: per chunk the logit gradient of the
+// whole vocabulary (one launch), then both products in one launch.  A chunk's
+// dh is complete (no float32 carry over launches) and its dW tiles have one
+// writer each, where the vocabulary chunks of gptrig_flce_bwd need 51 launches
+// of a few short items at V 50304, added with atomics.  Measured at d 768, V
+// 50304, backward alone, vocabulary chunks of 2048 / token chunks within 154
+// MB (the size of dweight): 128 tokens 1353 / 96 us, 1024 1429 / 285, 4096 2244
+// / 1183, 16384 5727 / 4605; faster at every count tried for d 512, 576, 768
+// and 1024.
+int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t* targets, const float* lse,
+                           const float* cotangent, float cotangent_scale, void* dhidden, float* dweight,
+                           int accumulate_dweight, void* workspace, size_t workspace_bytes, int n, int d, int vocab,
+                           int semantic_vocab, int token_chunk, void* stream) {
+  if (!hidden || !weight || !targets || !lse || !dhidden || !dweight || !workspace) return GPTRIG_E_NULL;
+  if (n <= 0 || d <= 0 || vocab <= 0 || d % 64) return GPTRIG_E_SHAPE;
+  if (semantic_vocab <= 0 || semantic_vocab > vocab) return GPTRIG_E_SHAPE;
+  if (n % 8) return GPTRIG_E_UNSUPPORTED;  // 16-byte rows of the MN-major operands
+  if (token_chunk <= 0 || (token_chunk < n && token_chunk % 32)) return GPTRIG_E_SHAPE;
+  if (workspace_bytes < gptrig_flce_bwd_tokens_workspace_bytes(n, d, vocab, token_chunk)) return GPTRIG_E_WORKSPACE;
+  if (((uintptr_t)hidden | (uintptr_t)weight | (uintptr_t)workspace | (uintptr_t)dweight | (uintptr_t)dhidden) & 15)
+    return GPTRIG_E_SHAPE;
+  const int chunk = token_chunk < n ? token_chunk : n;
+  bf16* gt = (bf16*)workspace;
+  float* dh_acc = (float*)((char*)workspace + align256((size_t)vocab * ceil_div(chunk, 32) * 32 * sizeof(bf16)));
+  hipStream_t s = (hipStream_t)stream;
+  const bf16* Wp = (const bf16*)weight;
+  for (int t0 = 0; t0 < n; t0 += chunk) {
+    const int c = n - t0 < chunk ? n - t0 : chunk;
+    const bf16* Hp = (const bf16*)hidden + (size_t)t0 * d;
+    const float* cot = cotangent ? cotangent + t0 : nullptr;
+    const unsigned tiles = tiles_of(vocab, c), cus = (unsigned)gemm::device_cus();
+    if (d % (4 * gemm::BK) == 0)
+      flce_grad_persistent_kernel<<<tiles < cus ? tiles : cus, gemm::THREADS, 0, s>>>(
+          Operand{Wp, d}, Operand{Hp, d}, vocab, c, d, 0, semantic_vocab, targets + t0, lse + t0, cot, cotangent_scale,
+          gt);
+    else
+      flce_grad_kernel<<<tiles, gemm::THREADS, 0, s>>>(Operand{Wp, d}, Operand{Hp, d}, vocab, c, d, 0, semantic_vocab,
+                                                       targets + t0, lse + t0, cot, cotangent_scale, gt);
+    GPTRIG_CHECK_LAUNCH();
+    const bool add = accumulate_dweight || t0 > 0;
+    // (Planned for whole token tiles, so ragged token counts share a plan.)
+    const int status = grad_gemms_launch(keep_plan(ceil_div(c, BN) * BN, d, vocab, add), gt, vocab, Hp, Wp,
+                                         (bf16*)dhidden + (size_t)t0 * d, dh_acc, dweight, add, c, d, vocab, s);
+    if (status != GPTRIG_OK) return status;
+  }
   return GPTRIG_OK;
 }
 

@@ -125,6 +125,19 @@ int gptrig_flce_bwd(const void* hidden, const void* weight, const int32_t* targe
                     int accumulate_dweight, void* workspace, size_t workspace_bytes, int n, int d, int vocab,
                     int semantic_vocab, int vocab_chunk, void* stream);
 
+/* The same backward cut into token chunks instead: per chunk the logit
+ * gradient over the whole vocabulary (bf16 [vocab, token_chunk] and the f32
+ * [token_chunk, d] dh, the workspace), then both products.  token_chunk >= n
+ * (one chunk) or a multiple of 32; gptrig_flce_token_chunk chooses the one
+ * expected fastest whose workspace takes at most max_bytes (0 if not even 256
+ * tokens, or all n, fit).  dhidden 16-byte aligned. */
+int gptrig_flce_token_chunk(int n, int d, int vocab, int64_t max_bytes);
+size_t gptrig_flce_bwd_tokens_workspace_bytes(int n, int d, int vocab, int token_chunk);
+int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t* targets, const float* lse,
+                           const float* cotangent, float cotangent_scale, void* dhidden, float* dweight,
+                           int accumulate_dweight, void* workspace, size_t workspace_bytes, int n, int d, int vocab,
+                           int semantic_vocab, int token_chunk, void* stream);
+
 /* The same forward and backward with float32 compute, the reference's
  * compute_dtype=float32 (rig/kernels/linear_cross_entropy.py:38-41,
  * _tile_logits :92-112): hidden f32 [n, d], weight f32 [vocab, d], every

@@ -437,3 +437,89 @@ def test_float32_nan_rows_stay_in_their_rows():
     rest = torch.arange(200, device=DEV) != 7
     assert torch.isnan(l1[7]) and torch.isnan(dh1[7]).all()
     assert torch.equal(l0[rest], l1[rest]) and torch.equal(dh0[rest], dh1[rest])
+
+
+@pytest.mark.parametrize("n,d,V,sv,chunk", [
+    (8, 64, 40, 33, 8),          # one chunk far below a tile; d not a multiple of 128
+    (264, 128, 300, 300, 264),   # one chunk, 8 tokens past a tile
+    (520, 192, 700, 650, 256),   # three chunks, the last of 8 tokens
+    (600, 128, 1100, 1024, 96),  # chunks below a tile, the last of 24 tokens
+    (1032, 256, 513, 513, 512),  # one vocabulary row past two tiles
+])
+def test_token_chunk_backward_against_float64(n, d, V, sv, chunk):
+    """gptrig_flce_bwd_tokens at its edges (chunks and tails that are no token
+    tile, ragged vocabularies, storage rows without a class, invalid targets),
+    overwriting and accumulating dweight, against float64.
+
+    Bound: bf16 keeps 8 significant bits, so a rounding moves a value by up to
+    2^-8 of itself.  Each logit gradient is rounded once (dw: 2^-8 of the sum of
+    magnitudes) and dh once more (2^-7 in all); float32 sums, the exponential
+    and lse add less than 2^-14."""
+    from gptrig import _lib
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    g = torch.Generator().manual_seed(n + V)
+    h = torch.randn((n, d), generator=g).bfloat16().to(DEV)
+    w = (torch.randn((V, d), generator=g) * 0.1).bfloat16().to(DEV)
+    t = torch.randint(0, sv, (n,), generator=g, dtype=torch.int32)
+    t[1], t[5] = -1, sv
+    t = t.to(DEV)
+    ct = torch.rand(n, generator=g).to(DEV)
+    _, lse = lce.flce_forward(h, w, t, sv)
+    print(f"flce token chunks n={n} d={d} V={V} sv={sv} chunk={chunk}", flush=True)
+    ws = _lib.workspace(_lib.query("gptrig_flce_bwd_tokens_workspace_bytes", n, d, V, chunk), DEV)
+    base = torch.randn((V, d), generator=g).to(DEV)
+    got = []
+    for accumulate in (0, 1):
+        dh = torch.full((n, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+        dw = base.clone() if accumulate else torch.full((V, d), float("nan"), device=DEV)
+        _lib.call("gptrig_flce_bwd_tokens", h.data_ptr(), w.data_ptr(), t.data_ptr(), lse.data_ptr(), ct.data_ptr(),
+                  0.0, dh.data_ptr(), dw.data_ptr(), accumulate, ws.data_ptr(), ws.numel(), n, d, V, sv, chunk,
+                  _lib.stream())
+        got.append((dh, dw - base if accumulate else dw))
+    h64, w64, t64 = h.double(), w.double(), t.long()
+    valid = (t64 >= 0) & (t64 < sv)
+    logits = h64 @ w64[:sv].T
+    c = torch.where(valid, ct.double(), 0.0)[:, None]
+    grad = torch.zeros((n, V), dtype=torch.float64, device=DEV)
+    grad[:, :sv] = torch.softmax(logits, -1) * c
+    grad.scatter_add_(1, t64.clamp(0, sv - 1)[:, None], -c)
+    for dh, dw in got:
+        for name, x, ref, mag, eps in (("dh", dh, grad @ w64, grad.abs() @ w64.abs(), 2.0 ** -7),
+                                       ("dw", dw, grad.T @ h64, grad.abs().T @ h64.abs(), 2.0 ** -8)):
+            excess = float(((x.double() - ref).abs() / ((eps + 2.0 ** -14) * mag + 1e-6)).max())
+            print(f"  {name} error / bound {excess:.3f}", flush=True)
+            assert excess <= 1
+    assert (got[0][1][sv:] == 0).all()
+
+
+def test_public_backward_route_and_memory():
+    """The token chunk the public call takes: within the memory it may use,
+    whole tokens where they fit, and none for a tile below the default (whose
+    gradients agree with the default's)."""
+    from gptrig import _lib
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    V = 50304
+    for n in (8, 128, 1000, 4096, 16384, 65536):
+        for d in (64, 512, 576, 768, 1024):
+            for tile in (256, 1792, 2048, 4096, V + 256):
+                chunk = lce.token_chunk(n, d, V, lce.chunk_for(tile))
+                if tile < 2048:
+                    assert chunk == 0
+                elif chunk:
+                    assert chunk == n or (chunk < n and chunk % 256 == 0)
+                    assert _lib.query("gptrig_flce_bwd_tokens_workspace_bytes", n, d, V, chunk) <= max(
+                        4 * n * lce.chunk_for(tile), 4 * V * d * 17 // 16)
+    assert lce.token_chunk(128, 768, V, 2048) == 128 and lce.token_chunk(16384, 768, V, 2048) % 256 == 0
+    g = torch.Generator().manual_seed(3)
+    h, w = torch.randn((300, 72), generator=g).to(DEV), (torch.randn((5000, 72), generator=g) * 0.1).to(DEV)
+    t = torch.randint(0, 4990, (300,), generator=g, dtype=torch.int32).to(DEV)
+    print("flce public route: default tile against 512", flush=True)
+    grads = []
+    for tile in (2048, 512):
+        hg, wg = h.clone().requires_grad_(), w.clone().requires_grad_()
+        lce.tiled_tied_cross_entropy(hg, wg, t, semantic_vocab_size=4990, vocab_tile_size=tile).backward()
+        grads.append((hg.grad, wg.grad))
+    for a, b in zip(*grads):  # one bf16 rounding of dh apart at most
+        assert float((a - b).norm()) <= 2.0 ** -9 * float(b.norm())
