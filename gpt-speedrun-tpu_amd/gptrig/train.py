@@ -77,7 +77,8 @@ class GPTConfig:
     # tiled loss (linear_cross_entropy.py:1-24, at most [tokens, vocab_tile_size]
     # fp32 logits live): the micro-batch's tokens are cut into chunks whose
     # kept fp16 probabilities [vocab, chunk] take at most tokens x
-    # vocab_tile_size x 4 bytes, and each chunk's forward and backward run
+    # vocab_tile_size x 4 bytes, or as much as the head's float32 gradient
+    # where that is more (flce_token_chunk), and each chunk's forward and backward run
     # back to back (the loss is the step's last node, so its cotangent is
     # known).  True: one chunk over all tokens ([vocab, tokens] fp16, 6.6 GB
     # at 65536 tokens; fastest on one MI355X).
@@ -167,21 +168,26 @@ def init_params(config: GPTConfig, seed: int) -> dict[str, np.ndarray]:
     return flat
 
 
-def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool) -> int:
+def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool, width: int = 0) -> int:
     """Tokens per kept-softmax FLCE chunk of a micro-batch.
 
     ``whole``: all of them.  Otherwise the largest multiple of 64 tokens whose
     kept buffer (``gptrig_flce_keep_bytes``: fp16 probabilities over the
     padded vocabulary plus the per-row maxima) fits ``tokens x
     vocab_tile_size x 4`` bytes, the reference's fp32 ``[tokens,
-    vocab_tile_size]`` live logits (``linear_cross_entropy.py:1-24``), at
-    least 64; then evened out over the chunks it needs.
+    vocab_tile_size]`` live logits (``linear_cross_entropy.py:1-24``), or, with
+    ``width``, the size of the head's float32 gradient ``[vocab, width]`` that
+    the step holds anyway, whichever is larger; at least 64; then evened out
+    over the chunks it needs.  (A micro-batch of a few thousand tokens is cut
+    into 13 chunks of a few hundred by the first bound alone, and a chunk's
+    launches take about 150 us however few its tokens are: at width 512, 8192
+    tokens, 2.40 ms in chunks of 640 against 2.0 ms in chunks of about 1000.)
     """
 
     if whole:
         return tokens
     per64 = _lib.query("gptrig_flce_keep_bytes", 64, vocab)
-    budget = tokens * vocab_tile_size * 4
+    budget = max(tokens * vocab_tile_size * 4, vocab * width * 4)
     cap = max(1, budget // per64) * 64
     if cap >= tokens:
         return tokens
@@ -535,7 +541,7 @@ class GPTTrainer:
         # instead of recomputing the logits GEMM; each token chunk runs its
         # forward and backward back to back (bounded by vocab_tile_size unless
         # flce_whole_vocab).  The head gradient accumulates over chunks.
-        chunk = flce_token_chunk(N, c.vocab_size, c.vocab_tile_size, c.flce_whole_vocab) \
+        chunk = flce_token_chunk(N, c.vocab_size, c.vocab_tile_size, c.flce_whole_vocab, d) \
             if d % 128 == 0 and N % 8 == 0 else 0
         if chunk:
             keep = self._workspace("flce_keep", _lib.query("gptrig_flce_keep_bytes", chunk, c.vocab_size))
