@@ -16,7 +16,8 @@ log-sum-exp, probabilities and accumulation are float32.  Any width is
 accepted: widths that are not a multiple of 64 are zero-padded, which leaves
 every logit unchanged.  With ``compute_dtype=torch.float32`` every product and
 sum is float32 (``gptrig_flce32_*``: the same tiled algorithm on float32
-operands, a float32 ``[tokens, chunk]`` logit-gradient workspace); gradients
+operands, a float32 ``[tokens, chunk]`` logit-gradient workspace, ``vocab_rows32``
+rows a chunk, and the products' partial sums, each at most as large); gradients
 come back in the inputs' dtypes, as the reference casts them (``:297-302``).
 """
 
@@ -295,6 +296,21 @@ def flce32_backward(h, w, t1, lse, cotangent, cotangent_scale: float, semantic_v
     return dh, dw
 
 
+def vocab_rows32(n_tokens: int, width: int, vocab: int, vocab_tile_size: int) -> int:
+    """Vocabulary rows per chunk of the float32 backward: the requested tile,
+    or, from the default tile up, as many as keep the float32 ``[tokens, rows]``
+    logit gradient within half of the weight gradient that the call returns.
+
+    A chunk of 2048 rows holds few 128 x 128 tiles for 256 CUs and costs its
+    launches' latency 25 times at V 50304 (d 512, 128 tokens: 1343 us against
+    169 with one chunk; 2048 tokens: 2308 against 1876 with 8192 rows).  A tile
+    below the default asks for a smaller working set and is taken as it is."""
+
+    if vocab_tile_size < DEFAULT_VOCAB_TILE_SIZE:
+        return vocab_tile_size
+    return min(max(vocab_tile_size, vocab * width // (2 * n_tokens)), max(vocab, vocab_tile_size))
+
+
 def _flatten32(hidden, embedding, targets):
     d = hidden.shape[-1]
     return (hidden.reshape(-1, d).to(torch.float32).contiguous(), embedding.to(torch.float32).contiguous(),
@@ -317,7 +333,7 @@ class _TiledLosses32(torch.autograd.Function):
         h, w, t1, lse = ctx.saved_tensors
         sv, chunk, hshape, hdtype, edtype = ctx.cfg
         cot = ct.reshape(-1).to(torch.float32).contiguous()
-        dh, dw = flce32_backward(h, w, t1, lse, cot, 0.0, sv, chunk)
+        dh, dw = flce32_backward(h, w, t1, lse, cot, 0.0, sv, vocab_rows32(*h.shape, w.shape[0], chunk))
         return dh.reshape(hshape).to(hdtype), dw.to(edtype), None, None, None
 
 
@@ -338,7 +354,7 @@ class _TiledMean32(torch.autograd.Function):
         sv, chunk, hshape, hdtype, edtype = ctx.cfg
         n = h.shape[0]
         cot = (ct.to(torch.float32) / n).expand(n).contiguous()
-        dh, dw = flce32_backward(h, w, t1, lse, cot, 0.0, sv, chunk)
+        dh, dw = flce32_backward(h, w, t1, lse, cot, 0.0, sv, vocab_rows32(*h.shape, w.shape[0], chunk))
         return dh.reshape(hshape).to(hdtype), dw.to(edtype), None, None, None
 
 

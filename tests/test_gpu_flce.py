@@ -523,3 +523,30 @@ def test_public_backward_route_and_memory():
         grads.append((hg.grad, wg.grad))
     for a, b in zip(*grads):  # one bf16 rounding of dh apart at most
         assert float((a - b).norm()) <= 2.0 ** -9 * float(b.norm())
+
+
+def test_float32_chunk_rows_follow_the_tile_and_the_weight_gradient():
+    """The float32 backward's chunk: the tile itself below the default,
+    otherwise at least the tile, and the logit gradient within the tile's or half
+    the weight gradient's size; one short call through the larger chunk."""
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    V = 50304
+    for n in (1, 128, 2048, 16384):
+        for d in (5, 64, 512):
+            for tile in (1, 2047, 2048, 4096, 10 * V):
+                rows = lce.vocab_rows32(n, d, V, tile)
+                assert rows == tile if tile < 2048 else rows >= tile
+                assert rows <= max(tile, V) and (rows == tile or 4 * n * rows <= 2 * V * d)
+    g = torch.Generator().manual_seed(8)
+    h, w = torch.randn((40, 48), generator=g).to(DEV), torch.randn((4500, 48), generator=g).to(DEV)
+    t = torch.randint(0, 4400, (40,), generator=g, dtype=torch.int32).to(DEV)
+    print("flce float32 default tile (two chunks' worth of rows) against 1024", flush=True)
+    grads = []
+    for tile in (2048, 1024):
+        hg, wg = h.clone().requires_grad_(), w.clone().requires_grad_()
+        lce.tiled_tied_cross_entropy(hg, wg, t, semantic_vocab_size=4400, vocab_tile_size=tile,
+                                     compute_dtype=torch.float32).backward()
+        grads.append((hg.grad, wg.grad))
+    for a, b in zip(*grads):  # the same float32 sums in another order
+        assert float((a - b).norm()) <= 1e-6 * float(b.norm())
