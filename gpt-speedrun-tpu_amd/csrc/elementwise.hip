@@ -835,10 +835,29 @@ __global__ void __launch_bounds__(256) masked_sum_kernel(const float* __restrict
 // padding column), 16-byte loads along src rows, 2-byte stores along dst rows
 // grouped so a wave writes 64 consecutive elements.
 // ----------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) transpose_bf16_kernel(const bf16* __restrict__ src, bf16* __restrict__ dst,
-                                                             int rows, int cols) {
+// One launch takes up to kTransposeMax matrices: alone, the weights of a small
+// model are launches of a few tiles each (width 512, 32 matrices a step: 32 x
+// 4.5 us against 26 us in one launch).
+constexpr int kTransposeMax = 64;
+struct TransposeItem {
+  const bf16* src;
+  bf16* dst;
+  int rows, cols, first;  // first: the item's first workgroup
+};
+struct TransposeGroup {
+  TransposeItem item[kTransposeMax];
+  int count;
+};
+
+__global__ void __launch_bounds__(256) transpose_bf16_kernel(TransposeGroup g) {
   __shared__ bf16 tile[64][65];
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+  int it = 0;
+  while (it + 1 < g.count && (int)blockIdx.x >= g.item[it + 1].first) ++it;  // uniform
+  const bf16* __restrict__ src = g.item[it].src;
+  bf16* __restrict__ dst = g.item[it].dst;
+  const int rows = g.item[it].rows, cols = g.item[it].cols;
+  const int b = (int)blockIdx.x - g.item[it].first, col_tiles = (cols + 63) / 64;
+  const int r0 = b / col_tiles * 64, c0 = b % col_tiles * 64;
   const int tid = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -962,14 +981,33 @@ int gptrig_bias_grad(const void* dy, int rows, int cols, float* db, void* stream
   return GPTRIG_OK;
 }
 
-int gptrig_transpose_bf16(const void* src, void* dst, int rows, int cols, void* stream) {
-  if (!src || !dst) return GPTRIG_E_NULL;
-  if (rows <= 0 || cols <= 0 || cols % 8) return GPTRIG_E_SHAPE;
-  if (((uintptr_t)src) & 15) return GPTRIG_E_SHAPE;
-  transpose_bf16_kernel<<<dim3(ceil_div(cols, 64), ceil_div(rows, 64)), 256, 0, (hipStream_t)stream>>>(
-      (const bf16*)src, (bf16*)dst, rows, cols);
-  GPTRIG_CHECK_LAUNCH();
+int gptrig_transpose_bf16_many(const gptrig_transpose* items, int count, void* stream) {
+  if (count < 0) return GPTRIG_E_SHAPE;
+  if (count > 0 && !items) return GPTRIG_E_NULL;
+  for (int i = 0; i < count; ++i) {
+    if (!items[i].src || !items[i].dst) return GPTRIG_E_NULL;
+    if (items[i].rows <= 0 || items[i].cols <= 0 || items[i].cols % 8) return GPTRIG_E_SHAPE;
+    if (((uintptr_t)items[i].src) & 15) return GPTRIG_E_SHAPE;
+  }
+  for (int at = 0; at < count; at += kTransposeMax) {
+    TransposeGroup g{};
+    g.count = count - at < kTransposeMax ? count - at : kTransposeMax;
+    int64_t first = 0;
+    for (int i = 0; i < g.count; ++i) {
+      const gptrig_transpose& t = items[at + i];
+      g.item[i] = TransposeItem{(const bf16*)t.src, (bf16*)t.dst, t.rows, t.cols, (int)first};
+      first += (int64_t)ceil_div(t.cols, 64) * ceil_div(t.rows, 64);
+    }
+    if (first >= (1ll << 31)) return GPTRIG_E_SHAPE;
+    transpose_bf16_kernel<<<(unsigned)first, 256, 0, (hipStream_t)stream>>>(g);
+    GPTRIG_CHECK_LAUNCH();
+  }
   return GPTRIG_OK;
+}
+
+int gptrig_transpose_bf16(const void* src, void* dst, int rows, int cols, void* stream) {
+  const gptrig_transpose item{src, dst, rows, cols};
+  return gptrig_transpose_bf16_many(&item, 1, stream);
 }
 
 int gptrig_gelu_fwd(const void* x, void* y, int64_t n, void* stream) {

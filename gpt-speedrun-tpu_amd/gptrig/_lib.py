@@ -28,6 +28,12 @@ class WGrad(ctypes.Structure):
     _fields_ = [("x", P), ("dy", P), ("dw", P), ("db", P), ("rows_in", I), ("cols_out", I)]
 
 
+class Transpose(ctypes.Structure):
+    """``gptrig_transpose`` of ``include/gptrig.h``."""
+
+    _fields_ = [("src", P), ("dst", P), ("rows", I), ("cols", I)]
+
+
 # name -> (restype, argtypes)
 SIGNATURES: dict[str, tuple] = {
     "gptrig_version": (c_char_p, []),
@@ -79,6 +85,7 @@ SIGNATURES: dict[str, tuple] = {
     "gptrig_sq_norm_partials": (I, [P, L, I, P, P]),
     "gptrig_finalize_norm": (I, [P, I, F, P, P, P, F, P, P]),
     "gptrig_transpose_bf16": (I, [P, P, I, I, P]),
+    "gptrig_transpose_bf16_many": (I, [ctypes.POINTER(Transpose), I, P]),
     "gptrig_cast_f32_bf16": (I, [P, P, L, P]),
     "gptrig_cast_f32_bf16_many": (I, [P, P, P, I, P]),
     "gptrig_weighted_sum": (I, [P, L, F, P, P]),

@@ -230,9 +230,9 @@ class ParamArena:
         self.refresh_transposed()
 
     def refresh_transposed(self) -> None:
-        for k, t in self.transposed.items():
-            rows, cols = self.shapes[k]
-            _lib.call("gptrig_transpose_bf16", self.w(k).data_ptr(), t.data_ptr(), rows, cols, _lib.stream())
+        items = (_lib.Transpose * len(self.transposed))(
+            *(_lib.Transpose(self.w(k).data_ptr(), t.data_ptr(), *self.shapes[k]) for k, t in self.transposed.items()))
+        _lib.call("gptrig_transpose_bf16_many", items, len(items), _lib.stream())
 
     def wt(self, path):
         """bf16 ``param.T`` of a block linear weight, refreshed after every update."""

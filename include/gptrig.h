@@ -339,6 +339,14 @@ int gptrig_finalize_norm(const float* partials, int parts, float grad_clip, floa
  * the K-major copy of a linear weight (rig/nn.py:55-56), which the forward
  * GEMM reads faster than the [d_in, d_out] layout. */
 int gptrig_transpose_bf16(const void* src, void* dst, int rows, int cols, void* stream);
+/* Several of them, in one launch per 64 (items is host memory, read before the
+ * call returns). */
+typedef struct {
+  const void* src; /* bf16 [rows, cols], 16-byte aligned */
+  void* dst;       /* bf16 [cols, rows] */
+  int rows, cols;
+} gptrig_transpose;
+int gptrig_transpose_bf16_many(const gptrig_transpose* items, int count, void* stream);
 
 /* Small helpers of the step: f32 -> bf16 cast, out += weight * sum(x), fill. */
 int gptrig_cast_f32_bf16(const float* x, void* y, int64_t n, void* stream);

@@ -868,3 +868,22 @@ def test_apply_rotary_of_any_strides(B, S, H, D, layout):
     assert y.is_contiguous() and torch.equal(y.detach().cpu(), onn.apply_rotary(x))
     (dx,) = torch.autograd.grad(y, xg, on())
     assert torch.equal(dx.cpu(), onn.apply_rotary_backward(x))
+
+
+def test_many_transposes_in_one_launch():
+    """70 matrices (two launches) of ragged sizes, each transposed bit for bit; none and bad ones."""
+
+    from gptrig import _lib
+
+    g = torch.Generator().manual_seed(4)
+    shapes = [(1, 8), (64, 64), (65, 72), (300, 8), (7, 200)] * 14
+    src = [torch.randn(s, generator=g).to(torch.bfloat16).to(DEV) for s in shapes]
+    dst = [torch.empty((c, r), dtype=torch.bfloat16, device=DEV) for r, c in shapes]
+    items = (_lib.Transpose * 70)(*(_lib.Transpose(a.data_ptr(), b.data_ptr(), *a.shape) for a, b in zip(src, dst)))
+    print("70 transposes", flush=True)
+    _lib.call("gptrig_transpose_bf16_many", items, 70, _lib.stream())
+    _lib.call("gptrig_transpose_bf16_many", items, 0, _lib.stream())
+    assert all(torch.equal(b, a.t()) for a, b in zip(src, dst))
+    items[3].cols = 12
+    with pytest.raises(RuntimeError):
+        _lib.call("gptrig_transpose_bf16_many", items, 70, _lib.stream())
