@@ -139,14 +139,16 @@ def _rotated(x: torch.Tensor, backward: bool) -> torch.Tensor:
         y = x.contiguous().clone()
         rope_inplace(y, H * D, B * S, S, H, D, backward=backward)
         return y
-    if x.stride(3) != 1 or any(s % 8 for s in x.stride()[:3]) or x.data_ptr() % 16:
+    strides = x.stride()[:3]
+    if x.stride(3) != 1 or any(s % 8 for s in strides) or x.data_ptr() % 16:
         x = x.contiguous()
         if x.data_ptr() % 16:
             x = x.clone()
+        strides = (S * H * D, H * D, D)  # (dimensions of size 1 may keep any stride)
     y = torch.empty((B, S, H, D), dtype=x.dtype, device=x.device)
     if y.numel():
         c, s = rope_tables(S, D, x.device)
-        _lib.call("gptrig_rope_copy", x.data_ptr(), *x.stride()[:3], y.data_ptr(), B, S, H, D, int(backward),
+        _lib.call("gptrig_rope_copy", x.data_ptr(), *strides, y.data_ptr(), B, S, H, D, int(backward),
                   c.data_ptr(), s.data_ptr(), _lib.stream())
     return y
 

@@ -843,6 +843,7 @@ def test_grouped_weight_gradients(n, shapes):
 @pytest.mark.parametrize("B,S,H,D,layout", [
     (1, 1, 1, 8, "contiguous"), (2, 33, 3, 64, "packed"), (1, 129, 2, 128, "heads first"),
     (3, 20, 5, 24, "odd base"), (2, 7, 2, 16, "expanded"), (1, 5, 3, 8, "strided dims"), (0, 4, 2, 8, "contiguous"),
+    (1, 6, 1, 16, "odd unit strides"),
 ])
 def test_apply_rotary_of_any_strides(B, S, H, D, layout):
     """The out-of-place rotation, forward and backward, equals the oracle bit
@@ -857,6 +858,7 @@ def test_apply_rotary_of_any_strides(B, S, H, D, layout):
         "odd base": lambda: randn((B * S * H * D + 3,), 4)[3:].view(B, S, H, D),
         "expanded": lambda: randn((1, S, 1, D), 5).expand(B, S, H, D),
         "strided dims": lambda: randn((B, S, H, 2 * D), 6)[..., ::2],
+        "odd unit strides": lambda: torch.as_strided(randn((S * D,), 7), (B, S, H, D), (3, D, 5, 1)),
     }[layout]()
     # The same strides on the device (a copy to it would compact the view).
     storage = torch.empty(x.untyped_storage().nbytes() // 2, dtype=torch.bfloat16)
