@@ -368,11 +368,15 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
                          pb[c2], acc[db]);
   };
 
-  // Tile `it` from (kt, vt), the tile after it, `nx`, on its way to (nkt, nvt).
+  // Tile `it` from (kt, vt), the tile after it (with segment ids `nx`) on its way to (nkt, nvt).
   auto tile = [&](const at64::lds_t* kt, const at64::lds_t* vt, at64::lds_t* nkt, at64::lds_t* nvt, int it, int nx,
                   bool same) {
     const int kv0 = it * kBlockN;
-    if (nx < ntiles) fill(nkt, nvt, nx * kBlockN);
+    if constexpr (kSeg) {
+      if (nx < ntiles) fill(nkt, nvt, nx * kBlockN);
+    } else {
+      if (it + 1 < ntiles) fill(nkt, nvt, kv0 + kBlockN);
+    }
     // Halves whose every key lies past the wave's last query add nothing.
     if (kv0 <= qw0 + 31) half(kt, vt, kv0, 0, same);
     __builtin_amdgcn_sched_barrier(0);  // keep the halves' live ranges apart
@@ -404,8 +408,8 @@ __device__ __forceinline__ void attn_fwd_swz(View Q, View K, View V, MutView O, 
     }
   } else {
     for (; it < ntiles; it += 2) {
-      tile(k0s, v0s, k1s, v1s, it, it + 1, false);
-      if (it + 1 < ntiles) tile(k1s, v1s, k0s, v0s, it + 1, it + 2, false);
+      tile(k0s, v0s, k1s, v1s, it, 0, false);
+      if (it + 1 < ntiles) tile(k1s, v1s, k0s, v0s, it + 1, 0, false);
     }
   }
 
