@@ -23,6 +23,10 @@
 //            from one half and K1 of chunk c into the other, its workgroups
 //            taking items from per-XCD token-block counters and never
 //            waiting for one another (the stream orders the launches).
+//   backward in token chunks (gptrig_flce_bwd_tokens, the public call's path
+//            from the default tile up): K1 over the whole vocabulary for a
+//            chunk of tokens, then both products in one launch
+//            (flce_keep_gemms_kernel).
 //   kept-softmax forward / backward (a token chunk at a time, its kept
 //            buffer bounded by the caller): the forward also stores fp16
 //            exp(logit - max) in 4-row x 32-token groups; the backward

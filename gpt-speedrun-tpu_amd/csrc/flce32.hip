@@ -16,7 +16,8 @@
 // the MFMA's float32 accumulator).  What is dropped is below 2^-22 of a
 // product, less than the rounding of a float32 sum of a few products.
 // Relative error of dh and dW against 64 bits at 2048 tokens, d 512, V 50304:
-// 2.8e-7, against 8.1e-7 for one float32 multiply-add chain per output on the
+// 2.8e-7 (5.1e-7 with the longer sums of 6288-row chunks), against 8.1e-7 for
+// one float32 multiply-add chain per output on the
 // vector ALU (fewer roundings of the running sum); at every size tried (1..2048
 // tokens, d 1..768, V 1..50304) no larger than that chain's.
 // A bf16 MFMA has 16 times the float32 MFMA's rate, so six of them are 2.7
@@ -32,12 +33,13 @@
 // weight nor a buffer for its planes.  ~50 KB of LDS and under 170 registers
 // let three workgroups share a CU, so one's loads, splits and epilogue run
 // under another's MFMAs.
-// Measured at 2048 tokens, d 512, V 50304, chunk 2048, against 64 x 64 vector-
-// ALU tiles: logits 592 us (178 TFLOP/s, 1.07 PFLOP/s of MFMA) against 1430,
-// forward + backward 2.83 ms against 23.0.  What bounds it now: the chunk's
-// launches (37 us logit gradient, 55 us the two products, 25 chunks) hold one or
-// two workgroups per CU at this size, so a stage's serial parts (fragment reads,
-// 24 MFMAs, split, barrier) overlap only partly.
+// Measured at 2048 tokens, d 512, V 50304, against 64 x 64 vector-ALU tiles:
+// logits 592 us (178 TFLOP/s, 1.07 PFLOP/s of MFMA) against 1430, forward +
+// backward 2.83 ms in chunks of 2048 rows (2.51 in the 6288 the front end takes)
+// against 23.0.  What bounds it now: a chunk of 2048 rows (37 us logit gradient,
+// 55 us the two products) holds one or two workgroups per CU at this size, so a
+// stage's serial parts (fragment reads, 24 MFMAs, split, barrier) overlap only
+// partly; larger ones run at the logits' rate.
 #include "gemm_core.h"
 
 #include <math.h>
