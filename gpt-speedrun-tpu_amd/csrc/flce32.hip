@@ -231,8 +231,12 @@ __device__ __forceinline__ void tile32(f32x16 (&acc)[2][2], Mat A, Mat B, int m_
 
 // Bytes of the rows of a tile that exist (at most kT of `ld` floats), and a
 // lane offset past any of them even with a row's offset added: such accesses
-// read zeros or are dropped.
+// read zeros or are dropped.  That takes a resource of at most 2^31 bytes: rows
+// of at most kMaxRow32 floats, which the host's token blocks (block32) and its
+// check of d see to.
 constexpr uint32_t kOff32Drop = 0x80000000u;
+constexpr int kMaxRow32 = 1 << 22;
+static_assert((int64_t)kT * kMaxRow32 * 4 <= (int64_t)kOff32Drop, "");
 __device__ __forceinline__ uint32_t row_bytes32(int rows, int ld) {
   return 4u * (uint32_t)((rows < kT ? rows : kT) * ld);
 }
@@ -485,6 +489,16 @@ int64_t gt_ld(int n) { return ((int64_t)n + 3) & ~(int64_t)3; }
 
 int64_t tiles32(int64_t rows, int64_t cols) { return ((rows + kT - 1) / kT) * ((cols + kT - 1) / kT); }
 
+// Tokens a launch takes: at most kMaxRow32 (the rows of G^T stay addressable by
+// 32-bit byte offsets) and fewer than 2^24 tiles with `rows` vocabulary rows (a
+// grid has fewer than 2^32 threads).  Both directions walk the tokens in such
+// blocks; up to 4 million tokens are one block for 65,000 rows.
+int block32(int n, int64_t rows) {
+  const int64_t most = ((1ll << 24) - 1) / tiles32(rows, 1) * kT;
+  const int64_t b = most < kT ? kT : most < kMaxRow32 ? most : kMaxRow32;
+  return (int)(b < n ? b : n);
+}
+
 // Slices of a gradient product of rows x d outputs over `depth`: enough
 // workgroups for one per CU (256 are assumed; a fixed number keeps the
 // workspace query independent of the device), slices at least 8 stages deep,
@@ -499,7 +513,7 @@ int slices32(int64_t rows, int d, int depth, int64_t budget) {
 }
 
 struct Plan32 {
-  int chunk, dh_slices, dw_slices;
+  int block, chunk, dh_slices, dw_slices;
   int64_t ld;
   size_t gt_bytes, dh_bytes, dw_bytes;  // workspace: G^T, dh partials, dW partials (0: written in place)
 };
@@ -507,6 +521,7 @@ struct Plan32 {
 Plan32 plan32(int n, int d, int vocab, int vocab_chunk) {
   Plan32 p;
   p.chunk = chunk32(vocab, vocab_chunk);
+  p.block = n = block32(n, p.chunk);
   p.ld = gt_ld(n);
   const int64_t gt = (int64_t)p.chunk * p.ld;
   p.dh_slices = slices32(n, d, p.chunk, gt);
@@ -529,6 +544,7 @@ extern "C" {
 size_t gptrig_flce32_fwd_workspace_bytes(int n, int d, int vocab) {
   (void)d;
   if (n <= 0 || vocab <= 0) return 0;
+  n = block32(n, vocab);
   const size_t ntiles = (size_t)((vocab + kT - 1) / kT);
   return align256(ntiles * n * sizeof(float2)) + align256((size_t)n * sizeof(float));
 }
@@ -542,19 +558,23 @@ int gptrig_flce32_fwd(const float* hidden, const float* weight, const int32_t* t
   if (workspace_bytes < gptrig_flce32_fwd_workspace_bytes(n, d, vocab)) return GPTRIG_E_WORKSPACE;
   if ((int64_t)n * d >= (1ll << 31) || (int64_t)vocab * d >= (1ll << 31)) return GPTRIG_E_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-  const int ntiles = (vocab + kT - 1) / kT;
+  const int ntiles = (vocab + kT - 1) / kT, block = block32(n, vocab);
   float2* partial = (float2*)workspace;
-  float* tlogit = (float*)((char*)workspace + align256((size_t)ntiles * n * sizeof(float2)));
-  // logits[v][token] = sum_d W[v][d] h[token][d]
-  const unsigned grid = (unsigned)tiles32(vocab, n);
-  (vec32(hidden, weight, d) ? stats32_kernel<true> : stats32_kernel<false>)<<<grid, kThreads, 0, s>>>(
-      weight, hidden, vocab, n, d, semantic_vocab, partial);
-  GPTRIG_CHECK_LAUNCH();
-  target32_kernel<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(hidden, weight, targets, n, d, semantic_vocab, tlogit);
-  GPTRIG_CHECK_LAUNCH();
-  combine32_kernel<<<(unsigned)((n + 63) / 64), 64 * kCombineWaves, 0, s>>>(partial, ntiles, n, semantic_vocab,
-                                                                             targets, tlogit, lse, losses);
-  GPTRIG_CHECK_LAUNCH();
+  float* tlogit = (float*)((char*)workspace + align256((size_t)ntiles * block * sizeof(float2)));
+  for (int64_t t0 = 0; t0 < n; t0 += block) {
+    const int nb = (int)(n - t0 < block ? n - t0 : block);
+    const float* hb = hidden + t0 * d;
+    // logits[v][token] = sum_d W[v][d] h[token][d]
+    const unsigned grid = (unsigned)tiles32(vocab, nb);
+    (vec32(hb, weight, d) ? stats32_kernel<true> : stats32_kernel<false>)<<<grid, kThreads, 0, s>>>(
+        weight, hb, vocab, nb, d, semantic_vocab, partial);
+    GPTRIG_CHECK_LAUNCH();
+    target32_kernel<<<(unsigned)((nb + 3) / 4), 256, 0, s>>>(hb, weight, targets + t0, nb, d, semantic_vocab, tlogit);
+    GPTRIG_CHECK_LAUNCH();
+    combine32_kernel<<<(unsigned)((nb + 63) / 64), 64 * kCombineWaves, 0, s>>>(
+        partial, ntiles, nb, semantic_vocab, targets + t0, tlogit, lse + t0, losses + t0);
+    GPTRIG_CHECK_LAUNCH();
+  }
   return GPTRIG_OK;
 }
 
@@ -573,38 +593,46 @@ int gptrig_flce32_bwd(const float* hidden, const float* weight, const int32_t* t
   if (semantic_vocab <= 0 || semantic_vocab > vocab) return GPTRIG_E_SHAPE;
   if (workspace_bytes < gptrig_flce32_bwd_workspace_bytes(n, d, vocab, vocab_chunk)) return GPTRIG_E_WORKSPACE;
   if ((int64_t)n * d >= (1ll << 31) || (int64_t)vocab * d >= (1ll << 31)) return GPTRIG_E_SHAPE;
+  if (d > kMaxRow32) return GPTRIG_E_SHAPE;
   hipStream_t s = (hipStream_t)stream;
   const Plan32 p = plan32(n, d, vocab, vocab_chunk);
   float* G = (float*)workspace;
   float* dh_parts = (float*)((char*)workspace + p.gt_bytes);
   float* dw_parts = (float*)((char*)workspace + p.gt_bytes + p.dh_bytes);
-  const int64_t nd = (int64_t)n * d;
-  const bool vec = vec32(hidden, weight, d) && ((uintptr_t)workspace & 15) == 0;
-  for (int v0 = 0; v0 < vocab; v0 += p.chunk) {
-    const int c = vocab - v0 < p.chunk ? vocab - v0 : p.chunk;
-    const float* Wc = weight + (int64_t)v0 * d;
-    float* dWc = dweight + (int64_t)v0 * d;
-    const int64_t cd = (int64_t)c * d;
-    (vec ? grad32_kernel<true> : grad32_kernel<false>)<<<(unsigned)tiles32(c, n), kThreads, 0, s>>>(
-        Wc, hidden, c, n, d, v0, semantic_vocab, targets, lse, cotangent, cotangent_scale, G, (int)p.ld);
-    GPTRIG_CHECK_LAUNCH();
-    // dW[chunk] (+)= G^T h (the dynamic_update_slice of :279-283) and
-    // dh += G W[chunk] (the reference's grad_hidden carry, :247).
-    const Out32 dw{p.dw_bytes ? dw_parts : dWc, p.dw_slices, cd, !p.dw_bytes && accumulate_dweight != 0};
-    const Out32 dh{p.dh_bytes ? dh_parts : dhidden, p.dh_slices, nd, v0 > 0};
-    const int64_t n_dw = tiles32(c, d) * p.dw_slices, n_dh = tiles32(n, d) * p.dh_slices;
-    (vec ? grads32_kernel<true> : grads32_kernel<false>)<<<(unsigned)(n_dw + n_dh), kThreads, 0, s>>>(
-        G, (int)p.ld, Wc, hidden, c, n, d, dw, dh, (int)n_dw);
-    GPTRIG_CHECK_LAUNCH();
-    if (p.dw_bytes) {
-      sum32_kernel<<<(unsigned)((cd + 255) / 256), 256, 0, s>>>(dw_parts, p.dw_slices, cd, dWc,
-                                                                accumulate_dweight != 0);
+  for (int64_t t0 = 0; t0 < n; t0 += p.block) {
+    const int nb = (int)(n - t0 < p.block ? n - t0 : p.block);
+    const float* hb = hidden + t0 * d;
+    float* dhb = dhidden + t0 * d;
+    const float* cot = cotangent ? cotangent + t0 : nullptr;
+    const int ld = (int)gt_ld(nb);
+    const int64_t nd = (int64_t)nb * d;
+    const bool add = accumulate_dweight || t0 > 0;
+    const bool vec = vec32(hb, weight, d) && ((uintptr_t)workspace & 15) == 0;
+    for (int v0 = 0; v0 < vocab; v0 += p.chunk) {
+      const int c = vocab - v0 < p.chunk ? vocab - v0 : p.chunk;
+      const float* Wc = weight + (int64_t)v0 * d;
+      float* dWc = dweight + (int64_t)v0 * d;
+      const int64_t cd = (int64_t)c * d;
+      (vec ? grad32_kernel<true> : grad32_kernel<false>)<<<(unsigned)tiles32(c, nb), kThreads, 0, s>>>(
+          Wc, hb, c, nb, d, v0, semantic_vocab, targets + t0, lse + t0, cot, cotangent_scale, G, ld);
+      GPTRIG_CHECK_LAUNCH();
+      // dW[chunk] (+)= G^T h (the dynamic_update_slice of :279-283) and
+      // dh += G W[chunk] (the reference's grad_hidden carry, :247).
+      const Out32 dw{p.dw_bytes ? dw_parts : dWc, p.dw_slices, cd, !p.dw_bytes && add};
+      const Out32 dh{p.dh_bytes ? dh_parts : dhb, p.dh_slices, nd, v0 > 0};
+      const int64_t n_dw = tiles32(c, d) * p.dw_slices, n_dh = tiles32(nb, d) * p.dh_slices;
+      (vec ? grads32_kernel<true> : grads32_kernel<false>)<<<(unsigned)(n_dw + n_dh), kThreads, 0, s>>>(
+          G, ld, Wc, hb, c, nb, d, dw, dh, (int)n_dw);
+      GPTRIG_CHECK_LAUNCH();
+      if (p.dw_bytes) {
+        sum32_kernel<<<(unsigned)((cd + 255) / 256), 256, 0, s>>>(dw_parts, p.dw_slices, cd, dWc, add);
+        GPTRIG_CHECK_LAUNCH();
+      }
+    }
+    if (p.dh_bytes) {
+      sum32_kernel<<<(unsigned)((nd + 255) / 256), 256, 0, s>>>(dh_parts, p.dh_slices, nd, dhb, 0);
       GPTRIG_CHECK_LAUNCH();
     }
-  }
-  if (p.dh_bytes) {
-    sum32_kernel<<<(unsigned)((nd + 255) / 256), 256, 0, s>>>(dh_parts, p.dh_slices, nd, dhidden, 0);
-    GPTRIG_CHECK_LAUNCH();
   }
   return GPTRIG_OK;
 }

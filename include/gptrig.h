@@ -146,7 +146,9 @@ int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t
  * rounded up to 64) with a float32 [n, chunk] logit-gradient workspace, the
  * reference's [n, vocab_tile_size] bound, plus partial sums of the two gradient
  * products, each at most as large, and writes dhidden f32 [n, d] and
- * dweight f32 [vocab, d] (+= with accumulate_dweight).  Any n, d.  Results do
+ * dweight f32 [vocab, d] (+= with accumulate_dweight).  n * d and vocab * d
+ * below 2^31, the backward's d at most 2^22; both directions walk more than
+ * 2^22 tokens in blocks (n is then a block in the bounds above).  Results do
  * not depend on the order of the workgroups (no atomics).  The products run on
  * the bf16 matrix cores from exact three-way splits of the float32 operands,
  * so an infinite operand gives NaN where a float32 product may give an infinity. */

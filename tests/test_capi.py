@@ -108,6 +108,26 @@ def test_backward_workspace_is_bounded_by_the_vocab_tile():
     assert lce.chunk_for(1) == 256 and lce.chunk_for(2048) == 2048 and lce.chunk_for(2049) == 2304
 
 
+def test_float32_loss_walks_many_tokens_in_blocks():
+    """The float32 kernels address 128 rows of the logit gradient (or of a
+    gradient of width d) by 32-bit byte offsets: 2^22 floats a row.  More
+    tokens are walked in blocks, which the workspace shows, and a wider d is
+    refused; a launch also stays below 2^24 tiles."""
+    limit = 1 << 22
+    for n in (limit, limit + 1, 5_000_000, 1 << 23, (1 << 24) + 3):
+        ws = _lib.query("gptrig_flce32_bwd_workspace_bytes", n, 8, 64, 64)
+        assert 4 * 64 * limit <= ws <= 4 * 64 * limit + (1 << 20), n  # (and partial sums of 64 x 8 values)
+    tiles = lambda rows: -(-rows // 128)  # noqa: E731
+    for vocab in (65536, 1 << 20, (1 << 24) + 5):
+        fwd = _lib.query("gptrig_flce32_fwd_workspace_bytes", 1 << 21, 8, vocab)
+        block = fwd // (8 * tiles(vocab) + 4)  # 8 bytes per (tile, token), 4 per token, and the alignment
+        assert tiles(block) * tiles(vocab) < 1 << 24 and block >= 128
+    lib = _lib.lib()
+    dummy = ctypes.c_void_p(16)
+    assert lib.gptrig_flce32_bwd(dummy, dummy, dummy, dummy, None, ctypes.c_float(1.0), dummy, dummy, 0, dummy,
+                                 ctypes.c_size_t(1 << 62), 2, limit + 1, 3, 3, 64, None) == -2
+
+
 def test_trainer_whole_vocabulary_chunk_opt_in():
     # The trainer's explicit opt-in: one chunk covering the whole vocabulary
     # while its bf16 G^T fits 8 GiB, else the fewest equal 256-row-tile chunks.

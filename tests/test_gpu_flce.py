@@ -418,6 +418,45 @@ def test_float32_split_products_at_tile_edges(n, d, V, sv, tile, offset):
     torch.testing.assert_close(total, base + runs[0][2], rtol=0, atol=float(base.abs().max()) * 2.0 ** -22)
 
 
+def test_float32_tokens_past_one_block():
+    """More tokens than one launch addresses (2^22): a whole block and a ragged
+    one of 133 tokens, whose rows are padded to 136 columns, against float64.
+
+    Bound as above with k = 8 and 72 for the logits and dh; dw's sum runs over
+    the tokens, with a rounding per MFMA and one per block."""
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    n, d, V = (1 << 22) + 133, 8, 72
+    g = torch.Generator(device=DEV).manual_seed(3)
+    h = torch.randn((n, d), generator=g, device=DEV)
+    w = torch.randn((V, d), generator=g, device=DEV) * 0.3
+    t = torch.randint(0, V, (n,), generator=g, device=DEV, dtype=torch.int32)
+    ct = torch.rand(n, generator=g, device=DEV)
+    print(f"flce float32 n={n} d={d} V={V}", flush=True)
+    losses, lse = lce.flce32_forward(h, w, t, V)
+    dh, dw = lce.flce32_backward(h, w, t, lse, ct, 0.0, V, 64)
+    dw64 = torch.zeros((V, d), dtype=torch.float64, device=DEV)
+    mag64 = torch.zeros_like(dw64)
+    w64 = w.double()
+    eps = 2.0 ** -20  # of a logit, lse or dh: a few float32 roundings of sums of magnitudes up to ~20
+    for i in range(0, n, 1 << 20):
+        at = slice(i, i + (1 << 20))
+        h64, t64 = h[at].double(), t[at].long()[:, None]
+        logits = h64 @ w64.T
+        lse64 = torch.logsumexp(logits, -1)
+        assert float((lse[at].double() - lse64).abs().max()) <= 16 * eps
+        assert float((losses[at].double() - (lse64 - logits.gather(1, t64)[:, 0])).abs().max()) <= 32 * eps
+        grad = torch.exp(logits - lse64[:, None]) * ct[at].double()[:, None]
+        grad.scatter_add_(1, t64, -ct[at].double()[:, None])
+        assert float((dh[at].double() - grad @ w64).abs().max()) <= 32 * eps
+        dw64 += grad.T @ h64
+        mag64 += grad.abs().T @ h64.abs()
+    # (Roundings of a running sum of 2^22 terms: at random signs about the root of their number.)
+    excess = float(((dw.double() - dw64).abs() / mag64).max())
+    print(f"  dw error / magnitudes {excess:.2e}", flush=True)
+    assert excess <= (n // 16) ** 0.5 * 2.0 ** -22
+
+
 def test_float32_nan_rows_stay_in_their_rows():
     """A NaN hidden row gives a NaN loss and hidden gradient for its token
     alone; the other tokens' losses and hidden gradients are untouched."""
