@@ -883,8 +883,9 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 int resolve_chunk(int vocab, int vocab_chunk) {
   const int chunk = vocab_chunk > 0 ? vocab_chunk : kDefaultChunk;
-  const int full = ceil_div(vocab, BM) * BM;
-  return chunk > full ? full : chunk;
+  const int64_t full = ((int64_t)vocab + BM - 1) / BM * BM, most = gemm::kMaxBlk / BM * BM;  // (G^T blocks: chunk rows)
+  const int64_t c = chunk > full ? full : chunk;
+  return (int)(c > most ? most : c);
 }
 
 // Pipelined chunk layout: two halves of `half` vocabulary rows each inside the
@@ -1348,6 +1349,7 @@ int gptrig_flce_bwd_keep(const void* hidden, const void* weight, const int32_t* 
   if (n <= 0 || d <= 0 || vocab <= 0 || d % 64) return GPTRIG_E_SHAPE;
   if (semantic_vocab <= 0 || semantic_vocab > vocab) return GPTRIG_E_SHAPE;
   if (n % 8) return GPTRIG_E_UNSUPPORTED;
+  if (vocab > gemm::kMaxBlk - 3) return GPTRIG_E_UNSUPPORTED;  // rows of a G^T block, rounded up to 4
   if (keep_bytes < gptrig_flce_keep_bytes(n, vocab)) return GPTRIG_E_WORKSPACE;
   if (workspace_bytes < gptrig_flce_bwd_keep_workspace_bytes(n, d)) return GPTRIG_E_WORKSPACE;
   if (((uintptr_t)hidden | (uintptr_t)weight | (uintptr_t)workspace | (uintptr_t)dweight | (uintptr_t)keep |
@@ -1382,7 +1384,7 @@ int gptrig_flce_bwd_keep(const void* hidden, const void* weight, const int32_t* 
 static int64_t token_bytes(int d, int vocab) { return 2ll * vocab + 4ll * d; }
 
 int gptrig_flce_token_chunk(int n, int d, int vocab, int64_t max_bytes) {
-  if (n <= 0 || d <= 0 || vocab <= 0) return 0;
+  if (n <= 0 || d <= 0 || vocab <= 0 || vocab > gemm::kMaxBlk) return 0;
   // (A chunk's columns are stored in blocks of 32 tokens; 4 KB for alignment.)
   const int64_t fit = (max_bytes - 4096) / token_bytes(d, vocab) / 32 * 32;
   if (fit >= n) return n;
@@ -1429,6 +1431,7 @@ int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t
   if (n <= 0 || d <= 0 || vocab <= 0 || d % 64) return GPTRIG_E_SHAPE;
   if (semantic_vocab <= 0 || semantic_vocab > vocab) return GPTRIG_E_SHAPE;
   if (n % 8) return GPTRIG_E_UNSUPPORTED;  // 16-byte rows of the MN-major operands
+  if (vocab > gemm::kMaxBlk) return GPTRIG_E_UNSUPPORTED;  // rows of a G^T block
   if (token_chunk <= 0 || (token_chunk < n && token_chunk % 32)) return GPTRIG_E_SHAPE;
   if (workspace_bytes < gptrig_flce_bwd_tokens_workspace_bytes(n, d, vocab, token_chunk)) return GPTRIG_E_WORKSPACE;
   if (((uintptr_t)hidden | (uintptr_t)weight | (uintptr_t)workspace | (uintptr_t)dweight | (uintptr_t)dhidden) & 15)

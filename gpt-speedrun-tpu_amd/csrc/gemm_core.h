@@ -109,6 +109,9 @@ struct Src {
 
 constexpr uint32_t kRsrcRange = 0x7FFFFFFFu;  // bytes a stage's resource covers
 constexpr uint32_t kOffZero = 0xFFFFFFF0u;    // past the range: the copy reads zeros
+// Largest Operand::blk: a 256-wide MN-major tile spans eight column blocks, so a
+// lane's offset reaches 448 blk bytes and the rows of one stage.
+constexpr int kMaxBlk = (int)((kRsrcRange - 4096u) / 448u);
 
 template <bool KMAJOR>
 __device__ __forceinline__ Src make_src(Operand op, int mn0, int k_begin, int MN, int k_end, int wave, int lane) {

@@ -168,8 +168,13 @@ def init_params(config: GPTConfig, seed: int) -> dict[str, np.ndarray]:
     return flat
 
 
+# The kept-softmax backward's row limit (``gptrig_flce_bwd_keep``).
+KEEP_MAX_VOCAB = 4_793_478
+
+
 def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool, width: int = 0) -> int:
-    """Tokens per kept-softmax FLCE chunk of a micro-batch.
+    """Tokens per kept-softmax FLCE chunk of a micro-batch (0: more than
+    ``KEEP_MAX_VOCAB`` rows, which take the recompute backward).
 
     ``whole``: all of them.  Otherwise the largest multiple of 64 tokens whose
     kept buffer (``gptrig_flce_keep_bytes``: fp16 probabilities over the
@@ -184,6 +189,8 @@ def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool,
     tokens, 2.40 ms in chunks of 640 against 2.0 ms in chunks of about 1000.)
     """
 
+    if vocab > KEEP_MAX_VOCAB:
+        return 0
     if whole:
         return tokens
     per64 = _lib.query("gptrig_flce_keep_bytes", 64, vocab)
@@ -576,8 +583,8 @@ class GPTTrainer:
 
         # ---- backward ----
         if not chunk:
-            # (d not a multiple of 128) the recompute backward over vocabulary
-            # chunks of vocab_tile_size, or one chunk with flce_whole_vocab.
+            # (d not a multiple of 128, or a vocabulary past KEEP_MAX_VOCAB) the
+            # recompute backward over vocabulary chunks of vocab_tile_size, or one chunk with flce_whole_vocab.
             vchunk = lce.grad_chunk(N, c.vocab_size) if c.flce_whole_vocab else lce.chunk_for(c.vocab_tile_size)
             ws = self._workspace("flce_bwd",
                                  _lib.query("gptrig_flce_bwd_workspace_bytes", N, d, c.vocab_size, vchunk))

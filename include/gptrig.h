@@ -130,7 +130,10 @@ int gptrig_flce_bwd(const void* hidden, const void* weight, const int32_t* targe
  * [token_chunk, d] dh, the workspace), then both products.  token_chunk >= n
  * (one chunk) or a multiple of 32; gptrig_flce_token_chunk chooses the one
  * expected fastest whose workspace takes at most max_bytes (0 if not even 256
- * tokens, or all n, fit).  dhidden 16-byte aligned. */
+ * tokens, or all n, fit).  dhidden 16-byte aligned.  At most 4,793,481
+ * vocabulary rows, whose 32-token blocks a tile addresses by 32-bit offsets
+ * (else 0 and GPTRIG_E_UNSUPPORTED; gptrig_flce_bwd takes more, in chunks of at
+ * most as many). */
 int gptrig_flce_token_chunk(int n, int d, int vocab, int64_t max_bytes);
 size_t gptrig_flce_bwd_tokens_workspace_bytes(int n, int d, int vocab, int token_chunk);
 int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t* targets, const float* lse,
@@ -174,7 +177,8 @@ int gptrig_flce32_bwd(const float* hidden, const float* weight, const int32_t* t
  * 65536, when asked for the whole vocabulary), accumulating dweight.  Same
  * losses and lse as gptrig_flce_fwd; gradient values as gptrig_flce_bwd's up
  * to one fp16 rounding of each probability before its bf16 rounding.  d a
- * multiple of 128 and n of 8 (else GPTRIG_E_UNSUPPORTED).  keep: gptrig_flce_keep_bytes(n, vocab) bytes, 16-byte
+ * multiple of 128, n of 8 and, in the backward, at most 4,793,478 rows (else
+ * GPTRIG_E_UNSUPPORTED).  keep: gptrig_flce_keep_bytes(n, vocab) bytes, 16-byte
  * aligned, written by the forward and consumed (overwritten) by the backward,
  * which must see the forward's lse.  The backward's workspace is the f32
  * [n, d] dh accumulator. */

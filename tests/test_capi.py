@@ -128,6 +128,31 @@ def test_float32_loss_walks_many_tokens_in_blocks():
                                  ctypes.c_size_t(1 << 62), 2, limit + 1, 3, 3, 64, None) == -2
 
 
+def test_blocked_logit_gradients_stay_addressable():
+    """A 256-token tile of the blocked logit gradient spans 448 bytes times its
+    rows, addressed by 32-bit offsets into a range of 2^31 - 1: larger
+    vocabularies take no token chunk, chunks of rows are capped, and the entry
+    points whose blocks hold the whole vocabulary refuse."""
+    most = (2 ** 31 - 1 - 4096) // 448
+    budget = 1 << 40
+    assert _lib.query("gptrig_flce_token_chunk", 4096, 128, most, budget) == 4096
+    assert _lib.query("gptrig_flce_token_chunk", 4096, 128, most + 1, budget) == 0
+    assert _lib.query("gptrig_flce_token_chunk", 4096, 128, 5_000_000, budget) == 0
+    rows = most // 256 * 256
+    ws = _lib.query("gptrig_flce_bwd_workspace_bytes", 64, 64, 20_000_000, 19_999_744)
+    assert 2 * 64 * rows <= ws <= 2 * 64 * rows + 4 * 64 * 64 + 64 * 20_000_000 // 128 + 4096
+    lib = _lib.lib()
+    dummy, big = ctypes.c_void_p(16), ctypes.c_size_t(1 << 62)
+    assert lib.gptrig_flce_bwd_tokens(dummy, dummy, dummy, dummy, None, ctypes.c_float(1.0), dummy, dummy, 0, dummy, big,
+                                      64, 64, most + 1, most + 1, 64, None) == -4
+    assert lib.gptrig_flce_bwd_keep(dummy, dummy, dummy, dummy, None, ctypes.c_float(1.0), dummy, dummy, 0, dummy, big,
+                                    dummy, big, 64, 128, most, most, None) == -4
+    from gptrig.train import KEEP_MAX_VOCAB, flce_token_chunk
+
+    assert KEEP_MAX_VOCAB == most - 3
+    assert flce_token_chunk(64, most - 3, 2048, True) == 64 and flce_token_chunk(64, most - 2, 2048, True) == 0
+
+
 def test_trainer_whole_vocabulary_chunk_opt_in():
     # The trainer's explicit opt-in: one chunk covering the whole vocabulary
     # while its bf16 G^T fits 8 GiB, else the fewest equal 256-row-tile chunks.

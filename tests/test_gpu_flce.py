@@ -532,6 +532,39 @@ def test_token_chunk_backward_against_float64(n, d, V, sv, chunk):
     assert (got[0][1][sv:] == 0).all()
 
 
+def test_public_backward_of_a_very_large_vocabulary():
+    """The default public call past the rows whose 32-token blocks stay
+    addressable (4,793,481): dh of every token of a 256-token tile and dw, against
+    float64 (in slices of the vocabulary); 2^-7 of the magnitudes (two bf16
+    roundings) as above."""
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    n, d, V = 256, 64, 4_793_481 + 100
+    g = torch.Generator(device=DEV).manual_seed(9)
+    h = torch.randn((n, d), generator=g, device=DEV).bfloat16().requires_grad_()
+    w = (torch.randn((V, d), generator=g, device=DEV) * 0.3).bfloat16().requires_grad_()
+    t = torch.randint(0, V, (n,), generator=g, device=DEV, dtype=torch.int32)
+    assert lce.token_chunk(n, d, V, lce.chunk_for(2048)) == 0
+    print(f"flce public backward n={n} d={d} V={V}", flush=True)
+    lce.tiled_tied_cross_entropy(h, w, t, semantic_vocab_size=V).backward()
+    h64, t64 = h.detach().double(), t.long()
+    cut = [slice(i, min(i + (1 << 17), V)) for i in range(0, V, 1 << 17)]
+    lse = torch.logsumexp(torch.stack([torch.logsumexp(h64 @ w.detach()[c].double().T, -1) for c in cut], -1), -1)
+    dh, mag, worst = torch.zeros_like(h64), torch.zeros_like(h64), 0.0
+    for c in cut:
+        w64 = w.detach()[c].double()
+        grad = torch.exp(h64 @ w64.T - lse[:, None]) / n
+        mine = ((t64 >= c.start) & (t64 < c.stop)).nonzero()[:, 0]
+        grad[mine, t64[mine] - c.start] -= 1.0 / n
+        dh += grad @ w64
+        mag += grad.abs() @ w64.abs()
+        bound = 2.0 ** -7 * (grad.abs().T @ h64.abs()) + 1e-9
+        worst = max(worst, float(((w.grad[c].double() - grad.T @ h64).abs() / bound).max()))
+    excess = float(((h.grad.double() - dh).abs() / (2.0 ** -7 * mag + 1e-9)).max())
+    print(f"  error / bound: dh {excess:.3f}, dw {worst:.3f}", flush=True)
+    assert excess <= 1 and worst <= 1
+
+
 def test_public_backward_route_and_memory():
     """The token chunk the public call takes: within the memory it may use,
     whole tokens where they fit, and none for a tile below the default (whose
