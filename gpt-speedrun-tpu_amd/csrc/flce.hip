@@ -565,7 +565,7 @@ struct WgradItem {
 };
 struct WgradGroup {
   WgradItem item[kWgradMax];
-  int count, n, split;
+  int count, n, split, mode;  // mode: gemm_f32_tile's
 };
 
 __global__ void __launch_bounds__(gemm::THREADS) wgrad_kernel(WgradGroup g) {
@@ -578,20 +578,21 @@ __global__ void __launch_bounds__(gemm::THREADS) wgrad_kernel(WgradGroup g) {
   split_range(g.n, g.split, split, k_begin, k_end);
   // A(m = i, k = t) = X[t][i] (MN-major), B(k = t, n = j) = dY[t][j] (MN-major).
   gemm_f32_tile<false, false>(Operand{w.x, w.rows_in}, Operand{w.dy, w.cols_out}, w.rows_in, w.cols_out, k_begin, k_end,
-                              tm, tn, w.dw, w.cols_out, g.split > 1 ? 2 : 1, w.db);
+                              tm, tn, w.dw, w.cols_out, g.mode, w.db);
 }
 
 // The split over the tokens of a launch of `tiles` tiles: rounds of CUs, each
 // of a slice's stages (rounded up to the main loop's groups of four) plus its
 // epilogue, in stages: about 60 for the atomic add of a tile, 20 for a read-
-// add-write (measured in the FLCE gradient launches).
-int wgrad_split(unsigned tiles, int k_iters) {
+// add-write (measured in the FLCE gradient launches), which one slice per tile
+// takes unless the caller asks for atomics.
+int wgrad_split(unsigned tiles, int k_iters, bool atomic) {
   const int cus = gemm::device_cus();
   const int most = k_iters / 8 > 1 ? k_iters / 8 : 1;
   int best = 1;
   double best_cost = 1e300;
   for (int s = 1; s <= most && s <= 256; ++s) {
-    const double stages = (double)((ceil_div(k_iters, s) + 3) & ~3) + (s > 1 ? 60.0 : 20.0);
+    const double stages = (double)((ceil_div(k_iters, s) + 3) & ~3) + (s > 1 || atomic ? 60.0 : 20.0);
     const double cost = (double)ceil_div((int64_t)tiles * s, (int64_t)cus) * stages;
     if (cost < best_cost * 0.999) {
       best_cost = cost;
@@ -1465,7 +1466,7 @@ int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t
 
 // The weight and bias gradients of several linears over the same n tokens
 // (rig/nn.py:55-56) in grouped split-K launches; see wgrad_kernel.
-int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* stream) {
+static int weight_grads(const gptrig_wgrad* items, int count, int n, bool atomic, void* stream) {
   if (!items) return GPTRIG_E_NULL;
   if (count < 0 || n <= 0) return GPTRIG_E_SHAPE;
   for (int i = 0; i < count; ++i) {
@@ -1480,7 +1481,8 @@ int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* strea
     g.n = n;
     unsigned tiles = 0;
     for (int i = 0; i < g.count; ++i) tiles += tiles_of(items[at + i].rows_in, items[at + i].cols_out);
-    g.split = wgrad_split(tiles, ceil_div(n, gemm::BK));
+    g.split = wgrad_split(tiles, ceil_div(n, gemm::BK), atomic);
+    g.mode = atomic || g.split > 1 ? 2 : 1;
     unsigned first = 0;
     for (int i = 0; i < g.count; ++i) {
       const gptrig_wgrad& w = items[at + i];
@@ -1493,10 +1495,14 @@ int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* strea
   return GPTRIG_OK;
 }
 
+int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* stream) {
+  return weight_grads(items, count, n, false, stream);
+}
+
 int gptrig_weight_grad(const void* x, const void* dy, float* dw, float* db, int n, int rows_in, int cols_out,
                        void* stream) {
   const gptrig_wgrad item{x, dy, dw, db, rows_in, cols_out};
-  return gptrig_weight_grads(&item, 1, n, stream);
+  return weight_grads(&item, 1, n, true, stream);
 }
 
 }  // extern "C"

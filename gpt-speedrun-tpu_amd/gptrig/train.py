@@ -25,6 +25,7 @@ which equals the reference's single-batch token mean.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass, field
 
@@ -652,11 +653,12 @@ class GPTTrainer:
             inp, dout, prefix = self.lin_in[i][name], self.lin_dout[i][name], f"blocks/{i}/{name}"
             items[j] = _lib.WGrad(inp.data_ptr(), dout.data_ptr(), A.grad(prefix + "_w").data_ptr(),
                                   A.grad(prefix + "_b").data_ptr(), inp.shape[1], dout.shape[1])
+        # (Only this stream writes the gradients of the linears.)
         if len(layers) > 1:
             _lib.call("gptrig_weight_grads", items, len(items), tokens, _lib.stream())
             return
         for w in items:
-            _lib.call("gptrig_weight_grad", w.x, w.dy, w.dw, w.db, tokens, w.rows_in, w.cols_out, _lib.stream())
+            _lib.call("gptrig_weight_grads", ctypes.byref(w), 1, tokens, _lib.stream())
 
     # -- the step ----------------------------------------------------------------------
     def train_step(self, x: torch.Tensor, y: torch.Tensor) -> None:

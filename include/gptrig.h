@@ -221,12 +221,14 @@ int gptrig_rmsnorm_bwd(const void* dy, const void* x, const void* scale, const f
  * dw f32 [rows_in, cols_out] += x^T dy for x bf16 [n, rows_in], dy bf16
  * [n, cols_out] (rows_in, cols_out multiples of 8), and, when db is not NULL,
  * db f32 [cols_out] += column sums of dy in the same pass.  Accumulates with
- * fp32 atomics. */
+ * fp32 atomics: calls on several streams may add to one dw and db. */
 int gptrig_weight_grad(const void* x, const void* dy, float* dw, float* db, int n, int rows_in, int cols_out,
                        void* stream);
 /* The same for several linears over the same n tokens, in one launch per 32
  * items (items is host memory, read before the call returns).  The dw and db
- * of different items must not overlap. */
+ * of different items must not overlap, and nothing else may write a dw while
+ * the call's work runs: a dw tile with one slice of the tokens is read, added
+ * to and written without atomics. */
 typedef struct {
   const void* x;  /* bf16 [n, rows_in] */
   const void* dy; /* bf16 [n, cols_out] */

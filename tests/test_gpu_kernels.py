@@ -840,6 +840,31 @@ def test_grouped_weight_gradients(n, shapes):
         _lib.call("gptrig_weight_grads", items, 1, n, _lib.stream())
 
 
+def test_weight_gradients_of_two_streams_into_one():
+    """gptrig_weight_grad adds atomically, so calls on two streams may share a
+    dw and db, also where one slice covers the tokens (64 of them: few enough).
+
+    Bound: every value is a multiple of 2^-4 and the sums stay below 2^18, so all
+    float32 sums are exact."""
+
+    from gptrig import _lib
+
+    n, rows_in, cols_out, calls = 64, 264, 512, 40
+    g = torch.Generator(device=DEV).manual_seed(12)
+    x, dy = (torch.randint(-8, 9, (n, c), generator=g, device=DEV).div(4).bfloat16() for c in (rows_in, cols_out))
+    dw, db = torch.zeros((rows_in, cols_out), device=DEV), torch.zeros(cols_out, device=DEV)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    print("weight gradients on two streams", flush=True)
+    for _ in range(calls):
+        for s in streams:
+            _lib.call("gptrig_weight_grad", x.data_ptr(), dy.data_ptr(), dw.data_ptr(), db.data_ptr(), n, rows_in,
+                      cols_out, s.cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(dw.double(), 2 * calls * (x.double().T @ dy.double()))
+    assert torch.equal(db.double(), 2 * calls * dy.double().sum(0))
+
+
 @pytest.mark.parametrize("B,S,H,D,layout", [
     (1, 1, 1, 8, "contiguous"), (2, 33, 3, 64, "packed"), (1, 129, 2, 128, "heads first"),
     (3, 20, 5, 24, "odd base"), (2, 7, 2, 16, "expanded"), (1, 5, 3, 8, "strided dims"), (0, 4, 2, 8, "contiguous"),
