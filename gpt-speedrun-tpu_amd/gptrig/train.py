@@ -78,10 +78,10 @@ class GPTConfig:
     # tiled loss (linear_cross_entropy.py:1-24, at most [tokens, vocab_tile_size]
     # fp32 logits live): the micro-batch's tokens are cut into chunks whose
     # kept fp16 probabilities [vocab, chunk] take at most tokens x
-    # vocab_tile_size x 4 bytes, or as much as the head's float32 gradient
-    # where that is more (flce_token_chunk), and each chunk's forward and backward run
-    # back to back (the loss is the step's last node, so its cotangent is
-    # known).  True: one chunk over all tokens ([vocab, tokens] fp16, 6.6 GB
+    # vocab_tile_size x 4 bytes, or, from the default tile up, as much as the
+    # head's float32 gradient where that is more (flce_token_chunk), and each
+    # chunk's forward and backward run back to back (the loss is the step's last
+    # node, so its cotangent is known).  True: one chunk over all tokens ([vocab, tokens] fp16, 6.6 GB
     # at 65536 tokens; fastest on one MI355X).
     flce_whole_vocab: bool = False
     optimizer: OptimizerConfig = field(default_factory=OptimizerConfig)
@@ -181,10 +181,11 @@ def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool,
     kept buffer (``gptrig_flce_keep_bytes``: fp16 probabilities over the
     padded vocabulary plus the per-row maxima) fits ``tokens x
     vocab_tile_size x 4`` bytes, the reference's fp32 ``[tokens,
-    vocab_tile_size]`` live logits (``linear_cross_entropy.py:1-24``), or, with
-    ``width``, the size of the head's float32 gradient ``[vocab, width]`` that
-    the step holds anyway, whichever is larger; at least 64; then evened out
-    over the chunks it needs.  (A micro-batch of a few thousand tokens is cut
+    vocab_tile_size]`` live logits (``linear_cross_entropy.py:1-24``), or, from
+    the default tile up and with ``width``, the size of the head's float32
+    gradient ``[vocab, width]`` that the step holds anyway, whichever is larger
+    (a tile below the default asks for a smaller working set); at least 64; then
+    evened out over the chunks it needs.  (A micro-batch of a few thousand tokens is cut
     into 13 chunks of a few hundred by the first bound alone, and a chunk's
     launches take about 150 us however few its tokens are: at width 512, 8192
     tokens, 2.40 ms in chunks of 640 against 2.0 ms in chunks of about 1000.)
@@ -195,7 +196,9 @@ def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool,
     if whole:
         return tokens
     per64 = _lib.query("gptrig_flce_keep_bytes", 64, vocab)
-    budget = max(tokens * vocab_tile_size * 4, vocab * width * 4)
+    budget = tokens * vocab_tile_size * 4
+    if vocab_tile_size >= lce.DEFAULT_VOCAB_TILE_SIZE:
+        budget = max(budget, vocab * width * 4)
     cap = max(1, budget // per64) * 64
     if cap >= tokens:
         return tokens
@@ -547,8 +550,8 @@ class GPTTrainer:
         # Kept softmax: the forward keeps its probabilities (fp16 [vocab,
         # chunk]) and the backward rescales them into the logit gradient
         # instead of recomputing the logits GEMM; each token chunk runs its
-        # forward and backward back to back (bounded by vocab_tile_size unless
-        # flce_whole_vocab).  The head gradient accumulates over chunks.
+        # forward and backward back to back (bounded as flce_token_chunk says
+        # unless flce_whole_vocab).  The head gradient accumulates over chunks.
         chunk = flce_token_chunk(N, c.vocab_size, c.vocab_tile_size, c.flce_whole_vocab, d) \
             if d % 128 == 0 and N % 8 == 0 else 0
         if chunk:

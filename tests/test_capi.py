@@ -153,6 +153,25 @@ def test_blocked_logit_gradients_stay_addressable():
     assert flce_token_chunk(64, most - 3, 2048, True) == 64 and flce_token_chunk(64, most - 2, 2048, True) == 0
 
 
+def test_trainer_chunk_follows_a_tile_below_the_default():
+    """The trainer's kept buffer may take the size of the head's float32 gradient
+    only from the default tile up: below it, the tile alone bounds it."""
+    from gptrig.train import flce_token_chunk
+
+    vocab, width = 50304, 768
+    for tokens in (8192, 16384):
+        last = None
+        for tile in (256, 512, 1024, 2047):
+            chunk = flce_token_chunk(tokens, vocab, tile, False, width)
+            assert chunk == flce_token_chunk(tokens, vocab, tile, False), (tokens, tile)
+            assert _lib.query("gptrig_flce_keep_bytes", chunk, vocab) <= tokens * tile * 4
+            assert last is None or chunk > last
+            last = chunk
+        chunk = flce_token_chunk(tokens, vocab, 2048, False, width)
+        assert chunk > last
+        assert _lib.query("gptrig_flce_keep_bytes", chunk, vocab) <= max(4 * tokens * 2048, 4 * vocab * width)
+
+
 def test_trainer_whole_vocabulary_chunk_opt_in():
     # The trainer's explicit opt-in: one chunk covering the whole vocabulary
     # while its bf16 G^T fits 8 GiB, else the fewest equal 256-row-tile chunks.

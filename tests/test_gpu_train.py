@@ -81,7 +81,7 @@ def test_train_step_flce_paths_match_oracle(label, model, trainer_only):
     opt = dict(learning_rate=2.0 ** -8, steps=steps, warmup_steps=1)
     ocfg = om.Config(**common, attention_backend="flash", optimizer=oopt.OptimizerConfig(**opt))
     gcfg = GPTConfig(**common, **trainer_only, micro_batch_size=2, optimizer=OptimizerConfig(**opt))
-    chunk = flce_token_chunk(256, 1000, gcfg.vocab_tile_size, gcfg.flce_whole_vocab)
+    chunk = flce_token_chunk(256, 1000, gcfg.vocab_tile_size, gcfg.flce_whole_vocab, gcfg.d_model)
     print(f"train case {label}: token chunk {chunk}", flush=True)
     if "token chunks" in label:
         assert chunk == 128
