@@ -186,6 +186,58 @@ __device__ __forceinline__ void mma_stage32(f32x16 (&acc)[2][2], const lds_t* st
       for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(a[i][kTerm[t][0]], b[j][kTerm[t][1]], acc[i][j]);
 }
 
+// The elements of tile32's product that came out infinite or NaN, again as
+// plain float32 multiply-adds: an infinite operand has no finite remainders to
+// split off (inf - inf), and the pieces of an overflowing product may differ in
+// sign.  The others keep their bits.  Both operands' stages are staged as
+// [k][row] floats, rows padded to 132; one column block at a time, for the
+// registers.
+template <bool AK, bool BKM>
+__device__ __forceinline__ void tile32_plain(f32x16 (&acc)[2][2], Mat A, Mat B, int m_end, int n_end, int k0,
+                                             int k_end, int m0, int n0) {
+  typedef __attribute__((address_space(3))) float lds_f;
+  typedef __attribute__((address_space(3))) f32x4 lds_f4;
+  constexpr int kRow = kT + 4;
+  static_assert(kK * kRow * sizeof(float) <= kStage * sizeof(bf16), "one operand per stage array");
+  lds_f* const as = (lds_f*)gemm::lds_cast(s32_stage0);
+  lds_f* const bs = (lds_f*)gemm::lds_cast(s32_stage1);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm0 = 64 * (wave & 1), wn0 = 64 * (wave >> 1);
+  auto fill = [&](lds_f* dst, Mat m, bool kmajor, int mn0, int mn_end, int kb) {
+    for (int idx = tid; idx < kT * kK; idx += kThreads) {
+      const int r = kmajor ? idx / kK : idx % kT, kk = kmajor ? idx % kK : idx / kT;
+      const int mn = mn0 + r, k = kb + kk;
+      dst[kk * kRow + r] = mn < mn_end && k < k_end ? m.p[kmajor ? mn * m.ld + k : k * m.ld + mn] : 0.f;
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    f32x16 sum[2] = {};
+    for (int kb = k0; kb < k_end; kb += kK) {
+      __syncthreads();
+      fill(as, A, AK, m0, m_end, kb);
+      fill(bs, B, BKM, n0, n_end, kb);
+      __syncthreads();
+      for (int kk = 0; kk < kK; ++kk) {
+        const float b = bs[kk * kRow + wn0 + 32 * j + (lane & 31)];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 a = *(const lds_f4*)(as + kk * kRow + wm0 + 32 * i + 8 * q + 4 * (lane >> 5));
+#pragma unroll
+            for (int u = 0; u < 4; ++u) sum[i][4 * q + u] = fmaf(a[u], b, sum[i][4 * q + u]);
+          }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = fabsf(acc[i][j][r]) < INFINITY ? acc[i][j][r] : sum[i][r];
+  }
+  __syncthreads();
+}
+
 // acc[i][j][r] = C[m0 + wm0 + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4][n0 + wn0 + 32 j + lane % 32],
 // wm0 = 64 (wave % 2), wn0 = 64 (wave / 2), over k in [k0, k_end).  Ends on a barrier:
 // the stage arrays may be reused.
@@ -200,6 +252,8 @@ __device__ __forceinline__ void tile32(f32x16 (&acc)[2][2], Mat A, Mat B, int m_
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
   lds_t* const st0 = gemm::lds_cast(s32_stage0);
   lds_t* const st1 = gemm::lds_cast(s32_stage1);
+  __shared__ int plain_s;
+  if (tid == 0) plain_s = 0;
   Loader<AK, kVec> la;
   Loader<BKM, kVec> lb;
   la.init(A, m0, k0, m_end, k_end, tid);
@@ -227,6 +281,16 @@ __device__ __forceinline__ void tile32(f32x16 (&acc)[2][2], Mat A, Mat B, int m_
     step(st0, st1, kt);
     if (kt + 1 < nk) step(st1, st0, kt + 1);
   }
+  // A sum of zeros unless an element is an infinity or NaN.
+  float zero[4] = {};
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) zero[q] = fmaf(acc[q >> 1][q & 1][r], 0.f, zero[q]);
+  const float z = (zero[0] + zero[1]) + (zero[2] + zero[3]);
+  if (__any(z != z) && lane == 0) plain_s = 1;
+  __syncthreads();
+  if (plain_s) tile32_plain<AK, BKM>(acc, A, B, m_end, n_end, k0, k_end, m0, n0);  // uniform
 }
 
 // Bytes of the rows of a tile that exist (at most kT of `ld` floats), and a

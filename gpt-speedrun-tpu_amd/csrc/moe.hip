@@ -249,7 +249,16 @@ __global__ void __launch_bounds__(64 * kRouterWaves)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int t = t0 + 4 * q + i;  // lane: expert l16, tokens 4 q .. 4 q + 3
-      if (t < T) logits[(size_t)t * E + l16] = acc[2][i] + acc[1][i] + acc[0][i];
+      if (t >= T) continue;
+      float s = acc[2][i] + acc[1][i] + acc[0][i];
+      // An infinity or NaN: again as plain multiply-adds (the pieces of an
+      // infinite weight are not its parts, inf - inf, and an infinite x makes a
+      // NaN of a weight's zero pieces).
+      if (!(fabsf(s) < INFINITY)) {
+        s = 0.f;
+        for (int d = 0; d < D; ++d) s = fmaf((float)x[(size_t)t * D + d], w[(size_t)d * E + l16], s);
+      }
+      logits[(size_t)t * E + l16] = s;
     }
   }
 }

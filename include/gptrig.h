@@ -153,8 +153,9 @@ int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t
  * below 2^31, the backward's d at most 2^22; both directions walk more than
  * 2^22 tokens in blocks (n is then a block in the bounds above).  Results do
  * not depend on the order of the workgroups (no atomics).  The products run on
- * the bf16 matrix cores from exact three-way splits of the float32 operands,
- * so an infinite operand gives NaN where a float32 product may give an infinity. */
+ * the bf16 matrix cores from exact three-way splits of the float32 operands;
+ * results that are infinite or NaN are computed again with float32
+ * multiply-adds, so infinities propagate as in a float32 product. */
 size_t gptrig_flce32_fwd_workspace_bytes(int n, int d, int vocab);
 int gptrig_flce32_fwd(const float* hidden, const float* weight, const int32_t* targets, float* losses, float* lse,
                       void* workspace, size_t workspace_bytes, int n, int d, int vocab, int semantic_vocab,

@@ -597,6 +597,50 @@ def test_public_backward_route_and_memory():
         assert float((a - b).norm()) <= 2.0 ** -9 * float(b.norm())
 
 
+@pytest.mark.parametrize("n,d,V,tile", [(200, 48, 300, 128), (130, 37, 257, 2048)])
+def test_float32_infinite_operands(n, d, V, tile):
+    """Infinite weights and activations give what float32 products give: a
+    class of -inf weights drops out of the sum over positive activations, an
+    infinite activation makes its own token's results infinite or NaN, and the
+    products past the largest float32 are infinities.  Finite values as in the
+    other float32 tests (1e-5)."""
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    g = torch.Generator().manual_seed(n)
+    h = (torch.rand((n, d), generator=g) + 0.1).to(DEV)
+    w = (torch.randn((V, d), generator=g) * 0.3).to(DEV)
+    w[10] = w[130] = -torch.inf
+    w[11, 3] = -torch.inf
+    h[7, 5] = torch.inf
+    h[9] = 1e30
+    w[12] = -1e30  # (-inf as a product of finite operands, for token 9)
+    t = torch.randint(20, 120, (n,), generator=g, dtype=torch.int32).to(DEV)
+    ct = torch.rand(n, generator=g).to(DEV)
+    print(f"flce float32 infinities n={n} d={d} V={V}", flush=True)
+    losses, lse = lce.flce32_forward(h, w, t, V)
+    dh, dw = lce.flce32_backward(h, w, t, lse, ct, 0.0, V, tile)
+    logits = (h.double()[:, None, :] * w.double()[None]).sum(-1)
+    fine = torch.ones(n, dtype=torch.bool, device=DEV)
+    fine[7] = False
+    want_lse = torch.logsumexp(logits, -1)
+    want = want_lse - logits.gather(1, t.long()[:, None])[:, 0]
+    assert torch.isfinite(want[fine]).all()
+    assert float(((losses.double() - want).abs() / (want.abs() + 1))[fine].max()) <= 1e-5
+    assert not torch.isfinite(losses[7])
+    # dw of the classes from the other tokens (without 9, whose 1e30 hides them).
+    fine[9] = False
+    keep = fine.nonzero()[:, 0]
+    _, dw2 = lce.flce32_backward(h[keep].contiguous(), w, t[keep].contiguous(), lse[keep].contiguous(),
+                                 ct[keep].contiguous(), 0.0, V, tile)
+    grad = torch.exp(logits[keep] - want_lse[keep, None])
+    grad[torch.arange(len(keep), device=DEV), t[keep].long()] -= 1
+    want_dw = (grad * ct[keep, None].double()).T @ h[keep].double()
+    assert torch.isfinite(want_dw).all() and (want_dw[10] == 0).all() and (dw2[10] == 0).all()
+    assert float((dw2.double() - want_dw).abs().max()) <= 1e-5 * float(want_dw.abs().max())
+    # dh is 0 x -inf where a class of -inf weights has probability 0, as in a float32 product.
+    assert torch.isnan(dh[fine]).any(1).all() and torch.isnan(dw[20:120]).any()
+
+
 def test_float32_chunk_rows_follow_the_tile_and_the_weight_gradient():
     """The float32 backward's chunk: the tile itself below the default,
     otherwise at least the tile, and the logit gradient within the tile's or half

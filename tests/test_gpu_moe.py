@@ -214,6 +214,36 @@ def test_router_logits_against_float64(tokens, width, experts):
     assert excess <= 1
 
 
+@pytest.mark.parametrize("tokens,width,experts", [(70, 64, 8), (17, 36, 3)])
+def test_router_logits_of_infinite_operands(tokens, width, experts):
+    """Infinite weights, activations and products give the infinities and NaN
+    of a float32 sum of products, in their own tokens and experts alone."""
+    from gptrig import _lib
+
+    g = torch.Generator().manual_seed(tokens)
+    x = torch.rand((tokens, width), generator=g).add(0.1).bfloat16().to(DEV)
+    w = (torch.randn((width, experts), generator=g) * 0.3).to(DEV)
+    logits = torch.empty((tokens, experts), device=DEV)
+    run = lambda: _lib.call("gptrig_moe_router_logits", x.data_ptr(), w.data_ptr(), logits.data_ptr(), tokens,  # noqa: E731
+                            width, experts, _lib.stream())
+    print(f"router infinities tokens={tokens} width={width} experts={experts}", flush=True)
+    run()
+    before = logits.clone()
+    w[3, 0] = -torch.inf
+    w[5, 1] = torch.inf
+    x[4, 7] = torch.inf
+    x[6, 2] = torch.nan
+    run()
+    sign = torch.sign(w[7].double())
+    want = before.clone()
+    want[:, 0], want[:, 1] = -torch.inf, torch.inf
+    for e in range(experts):
+        inf = float(sign[e]) * torch.inf
+        want[4, e] = inf if e > 1 or want[4, e] == inf else torch.nan
+    want[6] = torch.nan
+    assert torch.equal(torch.nan_to_num(logits, 7e37, 8e37, -9e37), torch.nan_to_num(want, 7e37, 8e37, -9e37))
+
+
 @pytest.mark.parametrize("tokens,width,experts,top_k", [
     (1, 8, 2, 1), (255, 64, 4, 2), (257, 72, 8, 2), (300, 136, 16, 3), (130, 264, 5, 1),
 ])
