@@ -12,14 +12,18 @@
 // Float32 products on the bf16 matrix cores: every float32 operand element is
 // split exactly into three bf16 pieces (x = hi + mid + lo, 8 significant bits
 // each, by truncation), and a product keeps the six terms of weight 2^-16 and
-// above (lo*hi, hi*lo, mid*mid, mid*hi, hi*mid, hi*hi, added smallest first in
-// the MFMA's float32 accumulator).  What is dropped is below 2^-22 of a
-// product, less than the rounding of a float32 sum of a few products.
-// Relative error of dh and dW against 64 bits at 2048 tokens, d 512, V 50304:
-// 2.8e-7 (5.1e-7 with the longer sums of 6288-row chunks), against 8.1e-7 for
-// one float32 multiply-add chain per output on the
-// vector ALU (fewer roundings of the running sum); at every size tried (1..2048
-// tokens, d 1..768, V 1..50304) no larger than that chain's.
+// above (lo*hi, hi*lo, mid*mid, mid*hi, hi*mid, hi*hi).  What is dropped is
+// below 2^-21 of a product (mid*lo + lo*mid, each below 2^-7 2^-15).  hi*hi has
+// an accumulator of its own and the five smaller terms, smallest first, another,
+// added at the end: with one for all, six roundings of the whole sum per 16
+// products cost up to twice the error over products of one sign.
+// Short sums take more: up to 64 products also the two dropped terms, up to 16
+// plain float32 multiply-adds (there a dropped term, or one rounding more, shows
+// against the few roundings of a chain).
+// Error against 64 bits, relative to one float32 multiply-add chain per output
+// on the vector ALU, operands of random signs, 1..200 tokens, d 1..512, V 1000:
+// dW 0.35 to 1.0, dh 0.2 to 0.4; of one sign: dW 0.35 to 1.1, dh 0.5 to 0.9 (the
+// six terms alone: dW up to 2.2 at one token).
 // A bf16 MFMA has 16 times the float32 MFMA's rate, so six of them are 2.7
 // times cheaper than one float32 MFMA and 5 times cheaper than the vector
 // ALU's multiply-adds.
@@ -30,12 +34,12 @@
 // written as three bf16 planes per operand into a double-buffered LDS stage
 // (24 KB): splitting on the way costs 5.5 vector operations per element, far
 // below the 24 MFMAs per wave and stage, and needs neither a pre-pass over the
-// weight nor a buffer for its planes.  ~50 KB of LDS and under 170 registers
-// let three workgroups share a CU, so one's loads, splits and epilogue run
-// under another's MFMAs.
+// weight nor a buffer for its planes.  The two accumulators leave registers for
+// two workgroups per CU, so one's loads, splits and epilogue run under another's
+// MFMAs (one accumulator and three workgroups: 2% faster).
 // Measured at 2048 tokens, d 512, V 50304, against 64 x 64 vector-ALU tiles:
-// logits 592 us (178 TFLOP/s, 1.07 PFLOP/s of MFMA) against 1430, forward +
-// backward 2.83 ms in chunks of 2048 rows (2.51 in the 6288 the front end takes)
+// logits 606 us (174 TFLOP/s, 1.04 PFLOP/s of MFMA) against 1430, forward +
+// backward 2.57 ms in the 6288-row chunks the front end takes (3.8 of 1024 rows)
 // against 23.0.  What bounds it now: a chunk of 2048 rows (37 us logit gradient,
 // 55 us the two products) holds one or two workgroups per CU at this size, so a
 // stage's serial parts (fragment reads, 24 MFMAs, split, barrier) overlap only
@@ -51,6 +55,8 @@ constexpr int kK = 16;       // k per LDS stage
 constexpr int kThreads = 256;
 constexpr int kPlane = kT * kK;          // bf16 elements of one plane of one operand
 constexpr int kStage = 6 * kPlane;       // A's three planes, then B's
+constexpr int kFewTerms = kK;            // sums of so many products run as multiply-adds
+constexpr int kFewStages = 4;            // sums of so many stages take eight terms of a product
 constexpr int kChunkRows = 64;           // granularity of the vocabulary chunk
 
 using gemm::lds_t;
@@ -165,8 +171,11 @@ __device__ __forceinline__ bf16x8 frag32(const lds_t* plane, int r0, int lane) {
   return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
+// One stage: hi*hi into acc, the smaller terms into small.  all (uniform): also
+// the two terms of weight 2^-21 and below (lo*mid, mid*lo).
 template <bool AK, bool BKM>
-__device__ __forceinline__ void mma_stage32(f32x16 (&acc)[2][2], const lds_t* st, int wm0, int wn0, int lane) {
+__device__ __forceinline__ void mma_stage32(f32x16 (&acc)[2][2], f32x16 (&small)[2][2], const lds_t* st, int wm0,
+                                            int wn0, int lane, bool all) {
   bf16x8 a[2][3], b[2][3];
 #pragma unroll
   for (int q = 0; q < 3; ++q)
@@ -175,26 +184,35 @@ __device__ __forceinline__ void mma_stage32(f32x16 (&acc)[2][2], const lds_t* st
       a[i][q] = frag32<AK>(st + q * kPlane, wm0 + 32 * i, lane);
       b[i][q] = frag32<BKM>(st + (3 + q) * kPlane, wn0 + 32 * i, lane);
     }
-  // Smallest terms first; the four accumulators alternate, so no MFMA waits
-  // for the one before it.
-  constexpr int kTerm[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
-#pragma unroll
-  for (int t = 0; t < 6; ++t)
+  // Smallest terms first; the accumulators alternate, so no MFMA waits for the
+  // one before it.
+  constexpr int kTerm[8][2] = {{2, 1}, {1, 2}, {2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+  auto term = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(a[i][kTerm[t][0]], b[j][kTerm[t][1]], acc[i][j]);
+      for (int j = 0; j < 2; ++j) {
+        f32x16& c = t == 7 ? acc[i][j] : small[i][j];
+        c = mfma32(a[i][kTerm[t][0]], b[j][kTerm[t][1]], c);
+      }
+  };
+  if (all) {
+    term(0);
+    term(1);
+  }
+#pragma unroll
+  for (int t = 2; t < 8; ++t) term(t);
 }
 
-// The elements of tile32's product that came out infinite or NaN, again as
-// plain float32 multiply-adds: an infinite operand has no finite remainders to
-// split off (inf - inf), and the pieces of an overflowing product may differ in
-// sign.  The others keep their bits.  Both operands' stages are staged as
-// [k][row] floats, rows padded to 132; one column block at a time, for the
-// registers.
+// tile32's product as plain float32 multiply-adds, one chain per output: all of
+// it (`all`, the shortest sums), or the elements that came out infinite or NaN,
+// while the others keep their bits (an infinite operand has no finite remainders
+// to split off, inf - inf, and the pieces of an overflowing product may differ
+// in sign).  Both operands' stages are staged as [k][row] floats, rows padded to
+// 132; one column block at a time, for the registers.
 template <bool AK, bool BKM>
 __device__ __forceinline__ void tile32_plain(f32x16 (&acc)[2][2], Mat A, Mat B, int m_end, int n_end, int k0,
-                                             int k_end, int m0, int n0) {
+                                             int k_end, int m0, int n0, bool all) {
   typedef __attribute__((address_space(3))) float lds_f;
   typedef __attribute__((address_space(3))) f32x4 lds_f4;
   constexpr int kRow = kT + 4;
@@ -214,11 +232,13 @@ __device__ __forceinline__ void tile32_plain(f32x16 (&acc)[2][2], Mat A, Mat B, 
   for (int j = 0; j < 2; ++j) {
     f32x16 sum[2] = {};
     for (int kb = k0; kb < k_end; kb += kK) {
-      __syncthreads();
-      fill(as, A, AK, m0, m_end, kb);
-      fill(bs, B, BKM, n0, n_end, kb);
-      __syncthreads();
-      for (int kk = 0; kk < kK; ++kk) {
+      if (j == 0 || k_end - k0 > kK) {  // (one stage stays for the second column block)
+        __syncthreads();
+        fill(as, A, AK, m0, m_end, kb);
+        fill(bs, B, BKM, n0, n_end, kb);
+        __syncthreads();
+      }
+      for (int kk = 0; kk < min(kK, k_end - kb); ++kk) {
         const float b = bs[kk * kRow + wn0 + 32 * j + (lane & 31)];
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -233,7 +253,8 @@ __device__ __forceinline__ void tile32_plain(f32x16 (&acc)[2][2], Mat A, Mat B, 
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = fabsf(acc[i][j][r]) < INFINITY ? acc[i][j][r] : sum[i][r];
+      for (int r = 0; r < 16; ++r)
+        acc[i][j][r] = !all && fabsf(acc[i][j][r]) < INFINITY ? acc[i][j][r] : sum[i][r];
   }
   __syncthreads();
 }
@@ -241,7 +262,9 @@ __device__ __forceinline__ void tile32_plain(f32x16 (&acc)[2][2], Mat A, Mat B, 
 // acc[i][j][r] = C[m0 + wm0 + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4][n0 + wn0 + 32 j + lane % 32],
 // wm0 = 64 (wave % 2), wn0 = 64 (wave / 2), over k in [k0, k_end).  Ends on a barrier:
 // the stage arrays may be reused.
-template <bool AK, bool BKM, bool kVec>
+// kShort: the sum may be short enough for more terms or plain multiply-adds
+// (a template parameter: the test of every stage costs a long sum 1.6%).
+template <bool AK, bool BKM, bool kVec, bool kShort>
 __device__ __forceinline__ void tile32(f32x16 (&acc)[2][2], Mat A, Mat B, int m_end, int n_end, int k0, int k_end,
                                        int m0, int n0) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -250,47 +273,55 @@ __device__ __forceinline__ void tile32(f32x16 (&acc)[2][2], Mat A, Mat B, int m_
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-  lds_t* const st0 = gemm::lds_cast(s32_stage0);
-  lds_t* const st1 = gemm::lds_cast(s32_stage1);
+  f32x16 small[2][2] = {};
+  const bool few = kShort && k_end - k0 <= kFewTerms;  // uniform
   __shared__ int plain_s;
-  if (tid == 0) plain_s = 0;
-  Loader<AK, kVec> la;
-  Loader<BKM, kVec> lb;
-  la.init(A, m0, k0, m_end, k_end, tid);
-  lb.init(B, n0, k0, n_end, k_end, tid);
-  const int nk = (k_end - k0 + kK - 1) / kK;
-  la.load(0);
-  lb.load(0);
-  la.store(st0, 0, tid);
-  lb.store(st0 + 3 * kPlane, 0, tid);
-  la.load(1);
-  lb.load(1);
-  __syncthreads();
-  // Stage kt + 1 (already in registers) is written into the other buffer, whose
-  // readers passed the last barrier, while stage kt is multiplied.
-  auto step = [&](const lds_t* cur, lds_t* nxt, int kt) __attribute__((always_inline)) {
-    mma_stage32<AK, BKM>(acc, cur, wm0, wn0, lane);
-    la.store(nxt, kt + 1, tid);
-    lb.store(nxt + 3 * kPlane, kt + 1, tid);
-    la.load(kt + 2);
-    lb.load(kt + 2);
-    GPTRIG_WAIT_LGKM0();  // this wave's LDS writes (the global loads stay in flight)
-    wg_barrier();
-  };
-  for (int kt = 0; kt < nk; kt += 2) {
-    step(st0, st1, kt);
-    if (kt + 1 < nk) step(st1, st0, kt + 1);
+  if (!few) {
+    lds_t* const st0 = gemm::lds_cast(s32_stage0);
+    lds_t* const st1 = gemm::lds_cast(s32_stage1);
+    if (tid == 0) plain_s = 0;
+    Loader<AK, kVec> la;
+    Loader<BKM, kVec> lb;
+    la.init(A, m0, k0, m_end, k_end, tid);
+    lb.init(B, n0, k0, n_end, k_end, tid);
+    const int nk = (k_end - k0 + kK - 1) / kK;
+    la.load(0);
+    lb.load(0);
+    la.store(st0, 0, tid);
+    lb.store(st0 + 3 * kPlane, 0, tid);
+    la.load(1);
+    lb.load(1);
+    __syncthreads();
+    // Stage kt + 1 (already in registers) is written into the other buffer, whose
+    // readers passed the last barrier, while stage kt is multiplied.
+    auto step = [&](const lds_t* cur, lds_t* nxt, int kt) __attribute__((always_inline)) {
+      mma_stage32<AK, BKM>(acc, small, cur, wm0, wn0, lane, kShort && nk <= kFewStages);
+      la.store(nxt, kt + 1, tid);
+      lb.store(nxt + 3 * kPlane, kt + 1, tid);
+      la.load(kt + 2);
+      lb.load(kt + 2);
+      GPTRIG_WAIT_LGKM0();  // this wave's LDS writes (the global loads stay in flight)
+      wg_barrier();
+    };
+    for (int kt = 0; kt < nk; kt += 2) {
+      step(st0, st1, kt);
+      if (kt + 1 < nk) step(st1, st0, kt + 1);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] += small[i][j];
+    // A sum of zeros unless an element is an infinity or NaN.
+    float zero[4] = {};
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) zero[q] = fmaf(acc[q >> 1][q & 1][r], 0.f, zero[q]);
+    const float z = (zero[0] + zero[1]) + (zero[2] + zero[3]);
+    if (__any(z != z) && lane == 0) plain_s = 1;
+    __syncthreads();
   }
-  // A sum of zeros unless an element is an infinity or NaN.
-  float zero[4] = {};
-#pragma unroll
-  for (int r = 0; r < 16; ++r)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) zero[q] = fmaf(acc[q >> 1][q & 1][r], 0.f, zero[q]);
-  const float z = (zero[0] + zero[1]) + (zero[2] + zero[3]);
-  if (__any(z != z) && lane == 0) plain_s = 1;
-  __syncthreads();
-  if (plain_s) tile32_plain<AK, BKM>(acc, A, B, m_end, n_end, k0, k_end, m0, n0);  // uniform
+  if (few || plain_s) tile32_plain<AK, BKM>(acc, A, B, m_end, n_end, k0, k_end, m0, n0, few);  // uniform
 }
 
 // Bytes of the rows of a tile that exist (at most kT of `ld` floats), and a
@@ -316,8 +347,8 @@ __device__ __forceinline__ void tile_of(int pid, int total, int col_tiles, int& 
 
 // Logits of 128 vocabulary rows x 128 tokens (rows = vocabulary) and their
 // per-token (max, sum exp(logit - max)) over the tile's classes.
-template <bool kVec>
-__global__ void __launch_bounds__(kThreads, 3)
+template <bool kVec, bool kShort>
+__global__ void __launch_bounds__(kThreads, 2)
     stats32_kernel(const float* __restrict__ w, const float* __restrict__ h, int V, int N, int D, int sem_v,
                    float2* __restrict__ partial) {
   __shared__ float2 half_s[kT];
@@ -325,7 +356,7 @@ __global__ void __launch_bounds__(kThreads, 3)
   int tv, tn;
   tile_of(blockIdx.x, gridDim.x, tok_tiles, tv, tn);
   f32x16 acc[2][2];
-  tile32<true, true, kVec>(acc, Mat{w, D}, Mat{h, D}, V, N, 0, D, tv * kT, tn * kT);
+  tile32<true, true, kVec, kShort>(acc, Mat{w, D}, Mat{h, D}, V, N, 0, D, tv * kT, tn * kT);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
   const int wm0 = 64 * (wave & 1), wn0 = 64 * (wave >> 1);
   const int left = sem_v - (tv * kT + wm0 + 4 * hl);  // classes from this lane's first row on
@@ -372,8 +403,8 @@ __global__ void __launch_bounds__(kThreads, 3)
 // G^T of one vocabulary chunk: gt[v][n] = (exp(logit - lse) - [v == target]) ct,
 // zero for rows that are no classes (linear_cross_entropy.py:255-266) and for
 // the padding columns N .. ld - 1.
-template <bool kVec>
-__global__ void __launch_bounds__(kThreads, 3)
+template <bool kVec, bool kShort>
+__global__ void __launch_bounds__(kThreads, 2)
     grad32_kernel(const float* __restrict__ w, const float* __restrict__ h, int C, int N, int D, int v0, int sem_v,
                   const int32_t* __restrict__ targets, const float* __restrict__ lse, const float* __restrict__ cot,
                   float cot_scale, float* __restrict__ gt, int ld) {
@@ -381,7 +412,7 @@ __global__ void __launch_bounds__(kThreads, 3)
   int tv, tn;
   tile_of(blockIdx.x, gridDim.x, tok_tiles, tv, tn);
   f32x16 acc[2][2];
-  tile32<true, true, kVec>(acc, Mat{w, D}, Mat{h, D}, C, N, 0, D, tv * kT, tn * kT);
+  tile32<true, true, kVec, kShort>(acc, Mat{w, D}, Mat{h, D}, C, N, 0, D, tv * kT, tn * kT);
   // Branch-free, through a buffer resource over the tile's rows: stores past
   // the chunk or the row are dropped.  (With a branch per element the 64
   // elements of a lane ran one after the other: 44 against 37 us per chunk of
@@ -426,8 +457,8 @@ struct Out32 {
   bool add;        // += (the slice holds earlier sums) instead of =
 };
 
-template <bool kVec>
-__global__ void __launch_bounds__(kThreads, 3)
+template <bool kVec, bool kShort>
+__global__ void __launch_bounds__(kThreads, 2)
     grads32_kernel(const float* __restrict__ gt, int ld, const float* __restrict__ w, const float* __restrict__ h, int C,
                    int N, int D, Out32 dw, Out32 dh, int n_dw) {
   const int col_tiles = (D + kT - 1) / kT;
@@ -442,9 +473,9 @@ __global__ void __launch_bounds__(kThreads, 3)
   const int per = ((depth + o.slices - 1) / o.slices + kK - 1) / kK * kK;
   const int k0 = slice * per, k1 = min(depth, k0 + per);  // (an empty slice writes zeros)
   if (is_dw)
-    tile32<true, false, kVec>(acc, Mat{gt, ld}, Mat{h, D}, C, D, k0, k1, tr * kT, tc * kT);
+    tile32<true, false, kVec, kShort>(acc, Mat{gt, ld}, Mat{h, D}, C, D, k0, k1, tr * kT, tc * kT);
   else
-    tile32<false, false, kVec>(acc, Mat{gt, ld}, Mat{w, D}, ld, D, k0, k1, tr * kT, tc * kT);
+    tile32<false, false, kVec, kShort>(acc, Mat{gt, ld}, Mat{w, D}, ld, D, k0, k1, tr * kT, tc * kT);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
   const int wm0 = 64 * (wave & 1), wn0 = 64 * (wave >> 1);
   const __amdgpu_buffer_rsrc_t rs =
@@ -596,6 +627,13 @@ Plan32 plan32(int n, int d, int vocab, int vocab_chunk) {
   return p;
 }
 
+// A kernel's form for 16-byte loads or not, for short sums or not.
+constexpr int kShort32 = kFewStages * kK;
+template <class Kernel>
+Kernel* pick32(bool vec, bool is_short, Kernel* v, Kernel* e, Kernel* v_short, Kernel* e_short) {
+  return is_short ? (vec ? v_short : e_short) : (vec ? v : e);
+}
+
 // 16-byte loads of rows of d floats.
 bool vec32(const float* a, const float* b, int d) {
   return d % 4 == 0 && (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
@@ -630,7 +668,8 @@ int gptrig_flce32_fwd(const float* hidden, const float* weight, const int32_t* t
     const float* hb = hidden + t0 * d;
     // logits[v][token] = sum_d W[v][d] h[token][d]
     const unsigned grid = (unsigned)tiles32(vocab, nb);
-    (vec32(hb, weight, d) ? stats32_kernel<true> : stats32_kernel<false>)<<<grid, kThreads, 0, s>>>(
+    pick32(vec32(hb, weight, d), d <= kShort32, stats32_kernel<true, false>, stats32_kernel<false, false>,
+           stats32_kernel<true, true>, stats32_kernel<false, true>)<<<grid, kThreads, 0, s>>>(
         weight, hb, vocab, nb, d, semantic_vocab, partial);
     GPTRIG_CHECK_LAUNCH();
     target32_kernel<<<(unsigned)((nb + 3) / 4), 256, 0, s>>>(hb, weight, targets + t0, nb, d, semantic_vocab, tlogit);
@@ -677,7 +716,8 @@ int gptrig_flce32_bwd(const float* hidden, const float* weight, const int32_t* t
       const float* Wc = weight + (int64_t)v0 * d;
       float* dWc = dweight + (int64_t)v0 * d;
       const int64_t cd = (int64_t)c * d;
-      (vec ? grad32_kernel<true> : grad32_kernel<false>)<<<(unsigned)tiles32(c, nb), kThreads, 0, s>>>(
+      pick32(vec, d <= kShort32, grad32_kernel<true, false>, grad32_kernel<false, false>, grad32_kernel<true, true>,
+             grad32_kernel<false, true>)<<<(unsigned)tiles32(c, nb), kThreads, 0, s>>>(
           Wc, hb, c, nb, d, v0, semantic_vocab, targets + t0, lse + t0, cot, cotangent_scale, G, ld);
       GPTRIG_CHECK_LAUNCH();
       // dW[chunk] (+)= G^T h (the dynamic_update_slice of :279-283) and
@@ -685,7 +725,8 @@ int gptrig_flce32_bwd(const float* hidden, const float* weight, const int32_t* t
       const Out32 dw{p.dw_bytes ? dw_parts : dWc, p.dw_slices, cd, !p.dw_bytes && add};
       const Out32 dh{p.dh_bytes ? dh_parts : dhb, p.dh_slices, nd, v0 > 0};
       const int64_t n_dw = tiles32(c, d) * p.dw_slices, n_dh = tiles32(nb, d) * p.dh_slices;
-      (vec ? grads32_kernel<true> : grads32_kernel<false>)<<<(unsigned)(n_dw + n_dh), kThreads, 0, s>>>(
+      pick32(vec, nb <= kShort32 || c <= kShort32, grads32_kernel<true, false>, grads32_kernel<false, false>,
+             grads32_kernel<true, true>, grads32_kernel<false, true>)<<<(unsigned)(n_dw + n_dh), kThreads, 0, s>>>(
           G, ld, Wc, hb, c, nb, d, dw, dh, (int)n_dw);
       GPTRIG_CHECK_LAUNCH();
       if (p.dw_bytes) {

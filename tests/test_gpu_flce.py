@@ -348,22 +348,29 @@ def test_float32_compute_matches_float64_dense(n, d, V, sv, tile):
     (129, 37, 385, 300, 200, 0),   # odd width (element loads), ragged chunks
     (514, 64, 1100, 1100, 2048, 1),  # 16-byte loads ruled out by the base address; sliced partial sums
     (1280, 128, 2048, 2000, 1024, 0),  # several slices of both products, two chunks
+    (16, 17, 60, 60, 64, 0),       # sums of 16 (multiply-adds), 17 and 60 (eight terms)
+    (65, 200, 300, 300, 64, 0),    # sums of 65 and 200 (six terms) beside 64 and 44
+    (150, 144, 200, 190, 256, "worst"),  # operands whose dropped terms are the largest
 ])
 def test_float32_split_products_at_tile_edges(n, d, V, sv, tile, offset):
     """The split-operand float32 tiles against float64 where they can go
     wrong: tile, stage, slice and chunk edges, widths and bases without
     16-byte loads, accumulation into dweight, and the same bits twice.
 
-    Bound: a product drops less than 2^-22 of itself and the operands are
-    split exactly; a sum over k is rounded once per MFMA (16 products), so an
-    output is within (2^-22 + ceil(k/16) 6 2^-24) of the sum of its products'
-    magnitudes, k the contraction's length; G adds the error of its logits."""
+    Bound: a product drops less than 2^-21 of itself (two terms of pieces below
+    2^-7 and 2^-15 of their operands) and the operands are split exactly; a sum
+    over k is rounded at most six times per 16 products, so an output is within
+    (2^-21 + ceil(k/16) 6 2^-24) of the sum of its products' magnitudes, k the
+    contraction's length; G adds the error of its logits."""
     from gptrig.kernels import linear_cross_entropy as lce
 
     g = torch.Generator().manual_seed(n)
     flat = torch.randn(n * d + V * d + 1, generator=g).to(DEV)
+    worst = offset == "worst"
+    if worst:
+        offset, flat = 0, torch.sign(flat) * (1 + 0xFFFF * 2.0 ** -23)
     h = flat[offset:offset + n * d].view(n, d)
-    w = flat[offset + n * d:offset + n * d + V * d].mul_(0.3).view(V, d)
+    w = flat[offset + n * d:offset + n * d + V * d].mul_(0.25 if worst else 0.3).view(V, d)
     t = torch.randint(0, sv, (n,), generator=g, dtype=torch.int32).to(DEV)
     if n > 5:
         t[3] = -1
@@ -386,7 +393,7 @@ def test_float32_split_products_at_tile_edges(n, d, V, sv, tile, offset):
     grad = torch.zeros((n, V), dtype=torch.float64)
     grad[:, :sv] = torch.exp(logits - lse64[:, None]) * c64
     grad.scatter_add_(1, safe, -c64)
-    eps = lambda k: 2.0 ** -22 + -(-k // 16) * 6 * 2.0 ** -24  # noqa: E731
+    eps = lambda k: 2.0 ** -21 + -(-k // 16) * 6 * 2.0 ** -24  # noqa: E731
     # A logit's absolute error; the probabilities (and lse) carry it relatively.
     mags = (h64.abs() @ w64.abs().t()).max()
     dl = float(mags) * eps(d) + 4 * 2.0 ** -24 * float(lse64.abs().max() + 1)
@@ -639,6 +646,56 @@ def test_float32_infinite_operands(n, d, V, tile):
     assert float((dw2.double() - want_dw).abs().max()) <= 1e-5 * float(want_dw.abs().max())
     # dh is 0 x -inf where a class of -inf weights has probability 0, as in a float32 product.
     assert torch.isnan(dh[fine]).any(1).all() and torch.isnan(dw[20:120]).any()
+
+
+@pytest.mark.parametrize("n,d,positive", [
+    (1, 4, False), (2, 8, False), (4, 16, False), (9, 32, False), (17, 200, False), (129, 64, False),
+    (65, 70, False), (4, 16, True), (64, 24, True), (65, 66, True), (140, 140, True),
+])
+def test_float32_products_are_no_less_precise_than_a_chain(n, d, positive):
+    """Both gradients' errors against float64 next to those of one float32
+    multiply-add chain per output (from the same log-sum-exp), over short and
+    long sums, operands of random signs and of one sign.  Errors are random: over
+    these draws the ratio of their root mean squares spreads by about a tenth, so
+    1.15 for random signs; 1.35 for one sign, where the matrix cores' roundings
+    share theirs (without the two further terms, the short sums' multiply-adds and
+    the small terms' accumulator: 1.9 to 2.3)."""
+    from gptrig.kernels import linear_cross_entropy as lce
+
+    V, draws = 400, 48 if n <= 4 else 12
+
+    def chain(a, b):
+        acc = torch.zeros((a.shape[0], b.shape[1]), dtype=torch.float64, device=DEV)
+        for k in range(a.shape[1]):  # a float64 product of two float32 is exact
+            acc = (acc + a[:, k, None].double() * b[k].double()).float().double()
+        return acc
+
+    def grad(logits, lse, t, ct):
+        g = torch.exp(logits - lse[:, None])
+        g[torch.arange(n, device=DEV), t.long()] -= 1
+        return g * ct[:, None]
+
+    print(f"flce float32 precision n={n} d={d} positive={positive}", flush=True)
+    err = torch.zeros(4, dtype=torch.float64)
+    for seed in range(draws):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        h = torch.randn((n, d), generator=g, device=DEV)
+        w = torch.randn((V, d), generator=g, device=DEV) * 0.3
+        if positive:
+            h.abs_(), w.abs_()
+        t = torch.randint(0, V, (n,), generator=g, device=DEV, dtype=torch.int32)
+        ct = torch.rand(n, generator=g, device=DEV)
+        l64 = h.double() @ w.double().T
+        g64 = grad(l64, torch.logsumexp(l64, -1), t, ct.double())
+        _, lse = lce.flce32_forward(h, w, t, V)
+        gc = grad(chain(h, w.T.contiguous()).float(), lse, t, ct)
+        dh, dw = lce.flce32_backward(h, w, t, lse, ct, 0.0, V, 2048)
+        for i, (got, want) in enumerate(((dw, g64.T @ h.double()), (chain(gc.T.contiguous(), h), g64.T @ h.double()),
+                                         (dh, g64 @ w.double()), (chain(gc, w), g64 @ w.double()))):
+            err[i] += float(((got.double() - want).norm() / want.norm()) ** 2)
+    dw_ratio, dh_ratio = float((err[0] / err[1]).sqrt()), float((err[2] / err[3]).sqrt())
+    print(f"  error over the chain's: dw {dw_ratio:.2f}, dh {dh_ratio:.2f}", flush=True)
+    assert max(dw_ratio, dh_ratio) <= (1.35 if positive else 1.15)
 
 
 def test_float32_chunk_rows_follow_the_tile_and_the_weight_gradient():
