@@ -6,8 +6,8 @@
 // einsums with compute_dtype float32 (`_tile_logits`, :92-112; the backward,
 // :220-302).  The [n, vocab] logits never exist; the backward's working set is
 // one float32 [n, chunk] logit gradient, the reference's own [n,
-// vocab_tile_size] bound, plus partial sums of at most the same size each for
-// the two gradient products (below).
+// vocab_tile_size] bound, plus, from the default tile up, partial sums of at
+// most the same size each for the two gradient products (below).
 //
 // Float32 products on the bf16 matrix cores: every float32 operand element is
 // split exactly into three bf16 pieces (x = hi + mid + lo, 8 significant bits
@@ -39,8 +39,7 @@
 // MFMAs (one accumulator and three workgroups: 2% faster).
 // Measured at 2048 tokens, d 512, V 50304, against 64 x 64 vector-ALU tiles:
 // logits 606 us (174 TFLOP/s, 1.04 PFLOP/s of MFMA) against 1430, forward +
-// backward 2.57 ms in the 6288-row chunks the front end takes (3.8 of 1024 rows)
-// against 23.0.  What bounds it now: a chunk of 2048 rows (37 us logit gradient,
+// backward 2.57 ms in the 6288-row chunks the front end takes, against 23.0.  What bounds it now: a chunk of 2048 rows (37 us logit gradient,
 // 55 us the two products) holds one or two workgroups per CU at this size, so a
 // stage's serial parts (fragment reads, 24 MFMAs, split, barrier) overlap only
 // partly; larger ones run at the logits' rate.
@@ -58,6 +57,7 @@ constexpr int kStage = 6 * kPlane;       // A's three planes, then B's
 constexpr int kFewTerms = kK;            // sums of so many products run as multiply-adds
 constexpr int kFewStages = 4;            // sums of so many stages take eight terms of a product
 constexpr int kChunkRows = 64;           // granularity of the vocabulary chunk
+constexpr int kDefaultChunk = 2048;      // the reference's default vocab_tile_size
 
 using gemm::lds_t;
 using gemm::lds_x8;
@@ -575,7 +575,7 @@ __global__ void __launch_bounds__(64 * kCombineWaves)
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 int chunk32(int vocab, int vocab_chunk) {
-  const int64_t c = vocab_chunk <= 0 ? 2048 : ((int64_t)vocab_chunk + kChunkRows - 1) / kChunkRows * kChunkRows;
+  const int64_t c = vocab_chunk <= 0 ? kDefaultChunk : ((int64_t)vocab_chunk + kChunkRows - 1) / kChunkRows * kChunkRows;
   return (int)(c < vocab ? c : ((int64_t)vocab + kChunkRows - 1) / kChunkRows * kChunkRows);
 }
 
@@ -597,7 +597,10 @@ int block32(int n, int64_t rows) {
 // Slices of a gradient product of rows x d outputs over `depth`: enough
 // workgroups for one per CU (256 are assumed; a fixed number keeps the
 // workspace query independent of the device), slices at least 8 stages deep,
-// and all partial sums together no larger than the [n, chunk] gradient.
+// and all partial sums together no larger than `budget` values: the [n, chunk]
+// gradient, or none for a chunk below the default, which asks for a small working
+// set (the backward at 2048 tokens, d 512, V 50304 in chunks of 1024: 3.3 ms with
+// partial sums, 6.0 without, 32.5 on the vector ALU in the same bytes).
 int slices32(int64_t rows, int d, int depth, int64_t budget) {
   const int64_t tiles = tiles32(rows, d);
   int64_t s = (256 + tiles / 2) / tiles;
@@ -619,8 +622,9 @@ Plan32 plan32(int n, int d, int vocab, int vocab_chunk) {
   p.block = n = block32(n, p.chunk);
   p.ld = gt_ld(n);
   const int64_t gt = (int64_t)p.chunk * p.ld;
-  p.dh_slices = slices32(n, d, p.chunk, gt);
-  p.dw_slices = slices32(p.chunk, d, n, gt);
+  const int64_t budget = vocab_chunk > 0 && vocab_chunk < kDefaultChunk ? 0 : gt;
+  p.dh_slices = slices32(n, d, p.chunk, budget);
+  p.dw_slices = slices32(p.chunk, d, n, budget);
   p.gt_bytes = align256((size_t)gt * sizeof(float));
   p.dh_bytes = p.dh_slices > 1 ? align256((size_t)p.dh_slices * n * d * sizeof(float)) : 0;
   p.dw_bytes = p.dw_slices > 1 ? align256((size_t)p.dw_slices * p.chunk * d * sizeof(float)) : 0;

@@ -17,7 +17,8 @@ accepted: widths that are not a multiple of 64 are zero-padded, which leaves
 every logit unchanged.  With ``compute_dtype=torch.float32`` every product and
 sum is float32 (``gptrig_flce32_*``: the same tiled algorithm on float32
 operands, a float32 ``[tokens, chunk]`` logit-gradient workspace, ``vocab_rows32``
-rows a chunk, and the products' partial sums, each at most as large); gradients
+rows a chunk, and from the default tile up the products' partial sums, each at
+most as large); gradients
 come back in the inputs' dtypes, as the reference casts them (``:297-302``).
 """
 

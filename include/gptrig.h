@@ -146,9 +146,10 @@ int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t
  * _tile_logits :92-112): hidden f32 [n, d], weight f32 [vocab, d], every
  * product and sum in float32 (lse and losses as gptrig_flce_fwd); the
  * backward recomputes the logits per chunk of vocab_chunk rows (0: 2048,
- * rounded up to 64) with a float32 [n, chunk] logit-gradient workspace, the
- * reference's [n, vocab_tile_size] bound, plus partial sums of the two gradient
- * products, each at most as large, and writes dhidden f32 [n, d] and
+ * rounded up to 64) with a float32 [n, chunk] logit-gradient workspace (n
+ * rounded up to 4), the reference's [n, vocab_tile_size] bound, plus, for chunks
+ * of 2048 and more, partial sums of the two gradient products, each at most as
+ * large, and writes dhidden f32 [n, d] and
  * dweight f32 [vocab, d] (+= with accumulate_dweight).  n * d and vocab * d
  * below 2^31, the backward's d at most 2^22; both directions walk more than
  * 2^22 tokens in blocks (n is then a block in the bounds above).  Results do

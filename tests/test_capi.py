@@ -128,6 +128,20 @@ def test_float32_loss_walks_many_tokens_in_blocks():
                                  ctypes.c_size_t(1 << 62), 2, limit + 1, 3, 3, 64, None) == -2
 
 
+def test_float32_workspace_below_the_default_tile_is_the_logit_gradient():
+    """A tile below the default asks for a smaller working set: the float32
+    backward's workspace is then the [tokens, chunk] logit gradient alone (chunk
+    the tile rounded up to 64, tokens to 4); from the default up, partial sums may
+    add twice as much."""
+    query = lambda *a: _lib.query("gptrig_flce32_bwd_workspace_bytes", *a)  # noqa: E731
+    for n, d in ((2048, 512), (512, 256), (128, 768), (1, 5), (1001, 64)):
+        for tile in (1, 64, 256, 1000, 1024, 2047):
+            rows = -(-tile // 64) * 64
+            assert query(n, d, 50304, tile) == -(-4 * rows * (-(-n // 4) * 4) // 256) * 256, (n, d, tile)
+        gradient = 4 * 2048 * (-(-n // 4) * 4)
+        assert gradient <= query(n, d, 50304, 0) == query(n, d, 50304, 2048) <= 3 * gradient + 768
+
+
 def test_blocked_logit_gradients_stay_addressable():
     """A 256-token tile of the blocked logit gradient spans 448 bytes times its
     rows, addressed by 32-bit offsets into a range of 2^31 - 1: larger
