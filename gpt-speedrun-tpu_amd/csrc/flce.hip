@@ -39,9 +39,6 @@
 #include <math.h>
 
 #include <algorithm>
-#include <functional>
-#include <mutex>
-#include <vector>
 
 namespace {
 
@@ -1069,19 +1066,25 @@ int gptrig_flce_fwd_keep(const void* hidden, const void* weight, const int32_t* 
 
 namespace {
 
-// Work split of flce_keep_gemms_kernel, chosen by simulating the
+// Work split of flce_keep_gemms_kernel, chosen by the makespan under the
 // dispatcher: the items (dh tiles x dh_split, dW tiles x dw_split) are handed
 // out in launch order to whichever CU frees up first, each costing its
 // 32-deep stages (rounded up to the main loop's groups of four) plus its
 // epilogue, in units of one stage: about 60 for an fp32 atomic add of a 256 KB
 // tile into a large array, 20 for a read-modify-write and 10 for a plain store
 // (measured at 5120 and 65536 tokens per call).  The plan with the shortest
-// estimated makespan wins; plans are cached per shape.
+// makespan wins.
 struct KeepPlan {
   int dh_split, dw_split, dh_mode, dw_mode;
   bool dh_first;
 };
 
+// The makespan of the dispatch in closed form (walking the items through a heap
+// took 0.1 to 2.5 ms a shape; a plan of 64 candidates now takes 2 us).  k1
+// items of length l1 leave nb CUs free at b and the other na at a = b - l1; the
+// items of length l2 <= l1 that follow end at a + i l2 (na times each) and
+// b + j l2 (nb times each), i and j from 1, and the k2-th smallest of these is
+// the last.
 double keep_makespan(int cus, unsigned dh_tiles, int dh_k, int dh_split, double dh_epi, unsigned dw_tiles, int dw_k,
                      int dw_split, double dw_epi, bool& dh_first) {
   auto len = [](int k_iters, int split) {
@@ -1093,33 +1096,21 @@ double keep_makespan(int cus, unsigned dh_tiles, int dh_k, int dh_split, double 
   const double l1 = dh_first ? l_dh : l_dw, l2 = dh_first ? l_dw : l_dh;
   const int64_t k1 = (int64_t)(dh_first ? dh_tiles * dh_split : dw_tiles * dw_split);
   const int64_t k2 = (int64_t)(dh_first ? dw_tiles * dw_split : dh_tiles * dh_split);
-  // Min-heap of CU free times (all items of a group have one length).
-  std::vector<double> heap((size_t)cus, 0.0);
-  auto take = [&](double l) {
-    std::pop_heap(heap.begin(), heap.end(), std::greater<double>());
-    heap.back() += l;
-    std::push_heap(heap.begin(), heap.end(), std::greater<double>());
-  };
-  for (int64_t i = 0; i < k1; ++i) take(l1);
-  for (int64_t i = 0; i < k2; ++i) take(l2);
-  return *std::max_element(heap.begin(), heap.end());
+  const int64_t nb = k1 % cus, na = cus - nb;
+  const double a = (double)(k1 / cus) * l1, b = nb ? a + l1 : a;
+  const int64_t first = (int64_t)ceil(l1 / l2), whole = (int64_t)floor(l1 / l2);
+  // The a-CUs alone until round `first`, which the b-CUs' first items do not end before.
+  int64_t i = (k2 + na - 1) / na;
+  if (nb && i > first) i = (k2 + nb * first + cus - 1) / cus;
+  double end = a + (double)i * l2;
+  if (nb) {
+    const int64_t left = k2 - na * whole, j = left > 0 ? (left + cus - 1) / cus : 0;
+    end = std::min(end, b + (double)j * l2);
+  }
+  return std::max(end, b);
 }
 
 KeepPlan keep_plan(int n, int d, int vocab, bool accumulate) {
-  struct Entry {
-    int dev, n, d, vocab;
-    bool acc;
-    KeepPlan plan;
-  };
-  static std::mutex mu;
-  static std::vector<Entry> cache;
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  {
-    std::lock_guard<std::mutex> lock(mu);
-    for (const Entry& e : cache)
-      if (e.dev == dev && e.n == n && e.d == d && e.vocab == vocab && e.acc == accumulate) return e.plan;
-  }
   const int cus = gemm::device_cus();
   const unsigned dh_tiles = tiles_of(n, d), dw_tiles = tiles_of(vocab, d);
   const int dh_k = ceil_div(vocab, gemm::BK), dw_k = ceil_div(n, gemm::BK);
@@ -1139,8 +1130,6 @@ KeepPlan keep_plan(int n, int d, int vocab, bool accumulate) {
       }
     }
   }
-  std::lock_guard<std::mutex> lock(mu);
-  cache.push_back(Entry{dev, n, d, vocab, accumulate, best});
   return best;
 }
 
