@@ -317,16 +317,21 @@ class GPTTrainer:
         # marks the point; the step's optimizer update waits for the stream.
         self.wgrad_stream = torch.cuda.Stream(device=self.device)
         self._layer_ready = [torch.cuda.Event() for _ in range(config.layers)]
-        # Layers per weight-gradient launch: enough that each of the 256 CUs has
-        # about 512 stages (32 tokens of a 256 x 256 tile) to run, several times
-        # the epilogue of a split launch: all eight layers of the 60M-class model
-        # at its 8192 tokens per step (8.0 -> 6.7 ms a step).  Where one layer has
-        # that much (the 125M model at 131072 tokens) its linears are launched one
-        # by one: grouped they are 8% faster alone (1638 against 1789 us a layer)
-        # but the step, whose clock the matrix cores' power sets, is 0.3% slower
-        # with their longer workgroups beside the backward of the layers below.
+        # Layers per weight-gradient launch: enough that each CU has about 512
+        # stages (32 tokens of a 256 x 256 tile) to run, several times the epilogue
+        # of a split launch.  Step in ms with 1 / 2 / 4 / all 8 layers a launch:
+        # width 512, 8192 tokens (11 by the rule) 7.21 / 6.17 / 6.10 / 6.20, 32768
+        # (3) 17.73 / 16.59 / 16.53 / 16.61, 65536 (2) 31.64 / 30.93 / 30.95 /
+        # 31.05; width 768, 8192 (5) 10.15 / 8.86 / 8.91 / 8.96, 32768 (2) 26.55 /
+        # 26.01 / 26.13 / 26.00, 65536 (1) 48.14 / 48.31 / 48.18 / 48.34.  From one
+        # layer with that much work on (the 125M model at 131072 tokens too) its
+        # linears are launched one by one: grouped they are 8% faster alone (1638
+        # against 1789 us a layer) but the step, whose clock the matrix cores' power
+        # sets, is 0.3% slower with their longer workgroups beside the backward of
+        # the layers below.
         tiles = sum(-(-a // 256) * -(-b // 256) for a, b in widths.values())
-        self.wgrad_layers = max(1, -(-512 * 256 // (tiles * -(-T // 32))))
+        cus = torch.cuda.get_device_properties(self.device).multi_processor_count
+        self.wgrad_layers = max(1, -(-512 * cus // (tiles * -(-T // 32))))
 
     # -- helpers -----------------------------------------------------------------
     def _workspace(self, name: str, nbytes: int) -> torch.Tensor:

@@ -147,6 +147,32 @@ def test_train_step_head_dim_128_matches_oracle(masking):
     assert np.all(np.abs(got[:, 2] - want[:, 2]) <= 2e-2 * want[:, 2])
 
 
+def test_weight_gradient_groups_cover_every_layer():
+    """Five layers' weight gradients in launches of one, two (the last of one
+    layer), three (of two) and all layers: the same gradients after one step but
+    for the order of their float32 sums (n 2^-24 of the magnitudes at most, here
+    bounded by the norm)."""
+    from gptrig.optim import OptimizerConfig
+    from gptrig.train import GPTConfig, GPTTrainer
+
+    cfg = GPTConfig(layers=5, heads=2, d_model=128, vocab_size=1000, semantic_vocab_size=997, seq_len=128, batch_size=4,
+                    micro_batch_size=2, base_width=128, base_depth=5, optimizer=OptimizerConfig(steps=3, warmup_steps=1))
+    w = torch.from_numpy(om.synthetic_windows(5, 1, 4, 128, 997)[0]).cuda()
+    grads = {}
+    for group in (1, 2, 3, 5):
+        trainer = GPTTrainer(cfg, seed=0)
+        assert trainer.wgrad_layers >= 5  # (so few tokens take one launch by themselves)
+        trainer.wgrad_layers = group
+        trainer.train_step(w[:, :-1], w[:, 1:])
+        grads[group] = {k: trainer.arena.grad(k).double() for k in trainer.arena.paths if k.startswith("blocks/")}
+        torch.cuda.synchronize()
+    print(f"trainer weight gradient groups, {len(grads[1])} tensors", flush=True)
+    for group in (2, 3, 5):
+        for k, want in grads[1].items():
+            assert float(want.norm()) > 0, k
+            assert float((grads[group][k] - want).norm()) <= 256 * 2.0 ** -24 * float(want.norm()), (group, k)
+
+
 def test_train_step_completep_clip_and_residual_scale_match_oracle():
     """The official parameterization (completep_fixed_tpp_v1, recipes/reference/
     config.yaml:22-30) at width multiplier 2 and depth multiplier 2 with
