@@ -137,9 +137,11 @@ __global__ void attn_dq_convert_kernel(const float* __restrict__ dq_acc, MutView
 // 1513 -> 595 us (backward kernel 994 -> 396, forward 554 -> 232); what is left
 // above the visible share of the work (about a quarter) is the uneven lengths
 // of the workgroups.  Where nothing can be skipped (one document) the test costs
-// about 2 us per workgroup and saves the compares: B16 H12 S1024 D64 forward
-// 93 -> 60, backward 192 -> 184 us; B8 H6 S1024 D128 forward 75 -> 39, backward
-// 122 -> 128 us.
+// 1 to 2 us per workgroup and saves the compares: B16 H12 S1024 D64 forward 87 ->
+// 56, backward 188 -> 172 us; B64 H12 S256 D64 44 -> 31, 111 -> 115; B8 H6 S1024
+// D128 75 -> 39, 121 -> 124; B64 H6 S256 D128 44 -> 31, 121 -> 123.  The backward
+// has the test's ids loaded with its first operands (waited for on their own: 127
+// at B8 H6 S1024 D128, 121 at B64 H12 S256 D64).
 template <int kWaves>
 struct SegScan {
   static constexpr int kPer = 64 / kWaves;  // blocks a wave tests
@@ -148,47 +150,76 @@ struct SegScan {
   uint64_t* sh;        // LDS: the need and the same bits of 64 blocks (kept here: registers are short)
   int S, lo, hi;       // the owned block's id range
   int group;           // the 64 blocks that the bits describe
+  bool on = true;      // off: every block is walked with the compare
 
   // Id range of the owned positions p0 .. p0 + 64 kOwn - 1 (those below S).
   template <int kOwn>
   __device__ __forceinline__ void init(const int32_t* seq_ids, uint64_t* lds, int seq, int p0, int lane) {
+    int own[kOwn];
+    fetch_own<kOwn>(own, seq_ids, lds, seq, p0, lane);
+    range<kOwn>(own);
+  }
+  template <int kOwn>
+  __device__ __forceinline__ void fetch_own(int (&own)[kOwn], const int32_t* seq_ids, uint64_t* lds, int seq, int p0,
+                                            int lane) {
     ids = seq_ids;
     sh = lds;
     S = seq;
     group = -1;
-    int a = ids[min(p0 + lane, S - 1)], z = a;
+#pragma unroll
+    for (int j = 0; j < kOwn; ++j) own[j] = ids[min(p0 + 64 * j + lane, S - 1)];
+  }
+  template <int kOwn>
+  __device__ __forceinline__ void range(const int (&own)[kOwn]) {
+    int a = own[0], z = a;
 #pragma unroll
     for (int j = 1; j < kOwn; ++j) {
-      const int x = ids[min(p0 + 64 * j + lane, S - 1)];
-      a = min(a, x);
-      z = max(z, x);
+      a = min(a, own[j]);
+      z = max(z, own[j]);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      a = min(a, __shfl_xor(a, o));
-      z = max(z, __shfl_xor(z, o));
-    }
-    lo = __builtin_amdgcn_readfirstlane(a);
-    hi = __builtin_amdgcn_readfirstlane(z);
+    // Over the wave without LDS: quads, half rows, rows, then row 15 / 31 on to
+    // the rows above; lane 63 ends with the whole.
+#define SEG_FOLD(ctrl)                                                              \
+  a = min(a, __builtin_amdgcn_update_dpp(a, a, ctrl, 0xF, 0xF, false));             \
+  z = max(z, __builtin_amdgcn_update_dpp(z, z, ctrl, 0xF, 0xF, false));
+    SEG_FOLD(0xB1)   // quad_perm [1, 0, 3, 2]
+    SEG_FOLD(0x4E)   // quad_perm [2, 3, 0, 1]
+    SEG_FOLD(0x141)  // row_half_mirror
+    SEG_FOLD(0x140)  // row_mirror
+    SEG_FOLD(0x142)  // row_bcast15
+    SEG_FOLD(0x143)  // row_bcast31
+#undef SEG_FOLD
+    lo = __builtin_amdgcn_readlane(a, 63);
+    hi = __builtin_amdgcn_readlane(z, 63);
   }
 
-  // (Every wave calls this the same number of times: it holds two barriers.)
-  __device__ __forceinline__ void load(int g, int wave, int lane) {
+  // This wave's share of the ids of group g, and its bits of them into LDS.
+  __device__ __forceinline__ void fetch(int (&id)[kPer], int g, int wave, int lane) const {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) id[j] = ids[min((64 * g + kPer * wave + j) * 64 + lane, S - 1)];
+  }
+  __device__ __forceinline__ void publish(const int (&id)[kPer], int g, int wave, int lane) {
     group = g;
     uint32_t n = 0, f = 0;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       const int p = (64 * g + kPer * wave + j) * 64 + lane;
-      const int id = ids[min(p, S - 1)];
-      const bool in = id >= lo && id <= hi;
+      const bool in = id[j] >= lo && id[j] <= hi;
       n |= __ballot(in && p < S) != 0 ? 1u << j : 0u;
       f |= __ballot(in || p >= S) == ~0ull ? 1u << j : 0u;
     }
-    __syncthreads();
     if (lane == 0) {
       reinterpret_cast<Piece*>(sh)[wave] = (Piece)n;
       reinterpret_cast<Piece*>(sh + 1)[wave] = (Piece)(lo == hi ? f : 0u);
     }
+  }
+
+  // (Every wave calls this the same number of times: it holds two barriers.)
+  __device__ __forceinline__ void load(int g, int wave, int lane) {
+    int id[kPer];
+    fetch(id, g, wave, lane);
+    __syncthreads();
+    publish(id, g, wave, lane);
     __syncthreads();
   }
 
@@ -202,6 +233,7 @@ struct SegScan {
   // same: its ids need no compare.
   __device__ __forceinline__ int next(int t, int nblk, int wave, int lane, bool& same) {
     same = false;
+    if (!on) return min(t, nblk);
     while (t < nblk) {
       if ((t >> 6) != group) load(t >> 6, wave, lane);
       const uint64_t m = bits(0) >> (t & 63);
@@ -485,8 +517,17 @@ __global__ void __launch_bounds__(kBwd64Threads, 2)
 
   const int seg_k = (kSeg && k_ok) ? seg[(size_t)b * S + my_k] : 0;
   __shared__ uint64_t scan_s[2];
+  // (The ids of the document test are loaded ahead of everything that is waited
+  // for.  A workgroup whose only query blocks are those of its own keys, which
+  // always hold visible pairs, goes without the test.)
   SegScan<8> scan;
-  if constexpr (kSeg) scan.template init<NK / 64>(seg + (size_t)b * S, scan_s, S, k0, lane);
+  int own_id[NK / 64], block_id[SegScan<8>::kPer];
+  const int qb_first = k0 / kBwdM, nqb = (S + kBwdM - 1) / kBwdM;
+  scan.on = nqb - qb_first > NK / kBwdM;
+  if (kSeg && scan.on) {
+    scan.template fetch_own<NK / 64>(own_id, seg + (size_t)b * S, scan_s, S, k0, lane);
+    scan.fetch(block_id, qb_first >> 6, wave, lane);
+  }
 
   {
     // (Branch-free, so these loads issue together with the K / V loads below.)
@@ -569,10 +610,16 @@ __global__ void __launch_bounds__(kBwd64Threads, 2)
     }
   };
 
-  const int qb_first = k0 / kBwdM;
-  const int nqb = (S + kBwdM - 1) / kBwdM;
   load_q(qb_first * kBwdM);
+  if (kSeg && scan.on) {
+    scan.template range<NK / 64>(own_id);
+    scan.publish(block_id, qb_first >> 6, wave, lane);
+  }
   store_q();
+  if (kSeg && scan.on) {
+    GPTRIG_WAIT_LGKM0();  // the bits are published
+    wg_barrier();
+  }
 
   // (The first block is the diagonal one: always visible.)
   bool same = false, same_n = false;
@@ -798,12 +845,17 @@ __global__ void __launch_bounds__(kBwd128Threads, 1)
   }
   const int seg_k = (kSeg && my_k < S) ? seg[(size_t)b * S + my_k] : 0;
   __shared__ uint64_t scan_s[2];
+  // (One wave per SIMD: nothing else hides the latency of the document test, so
+  // its ids and the first query block are loaded before anything is waited for.
+  // A workgroup whose only query blocks are those of its own keys, which always
+  // hold visible pairs, goes without the test.)
   SegScan<4> scan;
-  if constexpr (kSeg) scan.template init<NK / 64>(seg + (size_t)b * S, scan_s, S, k0, lane);
-#pragma unroll
-  for (int r = 0; r < KR; ++r) {
-    const int idx = tid + NT * r;
-    *(at64::lds_x8*)(Ks + at128(NK, idx >> 4, idx & 15)) = kst[r];
+  int own_id[NK / 64], block_id[SegScan<4>::kPer];
+  const int qb_first = k0 / M, nqb = (S + M - 1) / M;
+  scan.on = nqb - qb_first > NK / M;
+  if (kSeg && scan.on) {
+    scan.template fetch_own<NK / 64>(own_id, seg + (size_t)b * S, scan_s, S, k0, lane);
+    scan.fetch(block_id, qb_first >> 6, wave, lane);
   }
 
   f32x16 dv_acc[DB], dk_acc[DB];
@@ -903,10 +955,21 @@ __global__ void __launch_bounds__(kBwd128Threads, 1)
       *(at64::lds_x8*)(dSt + 32 * M * wave + 8 * (lane + 64 * r)) = bf16x8{};
   };
 
-  const int qb_first = k0 / M;
-  const int nqb = (S + M - 1) / M;
   load_q(qb_first * M);
+#pragma unroll
+  for (int r = 0; r < KR; ++r) {
+    const int idx = tid + NT * r;
+    *(at64::lds_x8*)(Ks + at128(NK, idx >> 4, idx & 15)) = kst[r];
+  }
+  if (kSeg && scan.on) {
+    scan.template range<NK / 64>(own_id);
+    scan.publish(block_id, qb_first >> 6, wave, lane);
+  }
   store_q(0);
+  if (kSeg && scan.on) {
+    GPTRIG_WAIT_LGKM0();  // the bits are published
+    wg_barrier();
+  }
 
   // The query block after qb that is computed.
   auto after = [&](int qb) {
