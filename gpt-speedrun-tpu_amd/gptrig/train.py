@@ -185,10 +185,14 @@ def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool,
     the default tile up and with ``width``, the size of the head's float32
     gradient ``[vocab, width]`` that the step holds anyway, whichever is larger
     (a tile below the default asks for a smaller working set); at least 64; then
-    evened out over the chunks it needs.  (A micro-batch of a few thousand tokens is cut
-    into 13 chunks of a few hundred by the first bound alone, and a chunk's
+    evened out over the chunks it needs.  (A micro-batch of a few thousand tokens
+    is cut into 13 chunks of a few hundred by the first bound alone, and a chunk's
     launches take about 150 us however few its tokens are: at width 512, 8192
-    tokens, 2.40 ms in chunks of 640 against 2.0 ms in chunks of about 1000.)
+    tokens, 2.51 ms in chunks of 640 against 2.17 in chunks of 960.)  Within the
+    second bound, whole token tiles of 256 instead where they come to 2% fewer
+    tiles, a chunk costing about 1.7 tiles of width 768 besides: 16384 tokens, width
+    768, 13 chunks of 1280 5.07 ms, 12 of 1408 5.49; 8192 tokens 7 of 1280 2.58, 6
+    of 1408 2.66; but width 512, 4096 tokens, 6 of 768 1.142, 5 of 832 1.135.
     """
 
     if vocab > KEEP_MAX_VOCAB:
@@ -197,13 +201,22 @@ def flce_token_chunk(tokens: int, vocab: int, vocab_tile_size: int, whole: bool,
         return tokens
     per64 = _lib.query("gptrig_flce_keep_bytes", 64, vocab)
     budget = tokens * vocab_tile_size * 4
-    if vocab_tile_size >= lce.DEFAULT_VOCAB_TILE_SIZE:
-        budget = max(budget, vocab * width * 4)
-    cap = max(1, budget // per64) * 64
+    head = vocab * width * 4 if vocab_tile_size >= lce.DEFAULT_VOCAB_TILE_SIZE else 0
+    cap = max(1, max(budget, head) // per64) * 64
     if cap >= tokens:
         return tokens
     share = -(-tokens // -(-tokens // cap))  # an even share of the chunks needed, <= cap
-    return -(-share // 64) * 64  # still <= cap, a multiple of 64
+    even = -(-share // 64) * 64  # still <= cap, a multiple of 64
+    tiles = cap // 256 * 256
+    if head <= budget or not tiles:
+        return even
+
+    def cost(chunk: int) -> float:
+        chunks, last = divmod(tokens, chunk)
+        each = 1.7 * 768 / width
+        return chunks * (-(-chunk // 256) + each) + (-(-last // 256) + each if last else 0.0)
+
+    return tiles if cost(tiles) < 0.98 * cost(even) else even
 
 
 class ParamArena:

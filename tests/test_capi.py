@@ -182,8 +182,15 @@ def test_trainer_chunk_follows_a_tile_below_the_default():
             assert last is None or chunk > last
             last = chunk
         chunk = flce_token_chunk(tokens, vocab, 2048, False, width)
-        assert chunk > last
+        assert chunk >= last
         assert _lib.query("gptrig_flce_keep_bytes", chunk, vocab) <= max(4 * tokens * 2048, 4 * vocab * width)
+    # Whole token tiles where an even share would leave each chunk a part of one
+    # (16384 tokens: 5.07 ms against 5.49 in chunks of 1408); not where the tile's
+    # own bound is the larger.
+    assert flce_token_chunk(16384, vocab, 2048, False, width) == flce_token_chunk(8192, vocab, 2048, False, width) == 1280
+    assert flce_token_chunk(8192, vocab, 2048, False, 512) == 960 and flce_token_chunk(4096, vocab, 2048, False, 512) == 832
+    for tokens in (20480, 65536):
+        assert flce_token_chunk(tokens, vocab, 2048, False, width) == flce_token_chunk(tokens, vocab, 2048, False)
 
 
 def test_trainer_whole_vocabulary_chunk_opt_in():
