@@ -85,7 +85,7 @@ def traffic_pass(micro_batch: int) -> None:
     from gptrig.train import flce_token_chunk
 
     dw = torch.empty(vocab, d, device=dev)
-    for chunk in (flce_token_chunk(n, vocab, 2048, False), n):
+    for chunk in (flce_token_chunk(n, vocab, 2048, False, d), n):
         keep = None
         for c0 in range(0, n, chunk):
             c1 = min(n, c0 + chunk)
@@ -196,9 +196,9 @@ def isolated_configs(reps: int = 20) -> dict:
 
     # The trainer's path (kept softmax over token chunks bounded by the default
     # vocab_tile_size), the same over one chunk of all tokens, the whole
-    # vocabulary with the logits recomputed, and the public API's default
-    # vocab_tile_size (2048: the reference's bounded [tokens, tile] working set).
-    chunk = flce_token_chunk(n, vocab, lce.DEFAULT_VOCAB_TILE_SIZE, False)
+    # vocabulary with the logits recomputed, and the public API's call with its
+    # default vocab_tile_size (2048): the token chunks it takes.
+    chunk = flce_token_chunk(n, vocab, lce.DEFAULT_VOCAB_TILE_SIZE, False, d)
     flce_ms = timed(flce_keep(chunk))
     flce_tf = flce_flops(n, d, vocab) / (flce_ms / 1e3) / 1e12
     keep_bytes = keep_buf[0].numel()
@@ -209,7 +209,14 @@ def isolated_configs(reps: int = 20) -> dict:
     del dw
     whole_ms = timed(flce_with(lce.grad_chunk(n, vocab)))
     whole_tf = flce_flops(n, d, vocab) / (whole_ms / 1e3) / 1e12
-    tile_ms = timed(flce_with(lce.chunk_for(lce.DEFAULT_VOCAB_TILE_SIZE)))
+    public = lce.token_chunk(n, d, vocab, lce.chunk_for(lce.DEFAULT_VOCAB_TILE_SIZE))
+    cot = torch.full((n,), 1.0 / n, device=dev)
+
+    def flce_public():
+        _, lse_c = lce.flce_forward(h, w, t, vocab)
+        lce.flce_backward_tokens(h, w, t, lse_c, cot, 0.0, vocab, public)
+
+    tile_ms = timed(flce_public)
     tile_tf = flce_flops(n, d, vocab) / (tile_ms / 1e3) / 1e12
     peak = MFMA_BF16_PEAK_TFLOPS
     return {
@@ -224,7 +231,8 @@ def isolated_configs(reps: int = 20) -> dict:
         "flce_N16384_d768_V50304": {"ms": round(flce_ms, 4), "tflops": round(flce_tf, 1),
                                     "frac": round(flce_tf / peak, 4), "algorithmic_flops": flce_flops(n, d, vocab),
                                     "path": f"kept softmax over token chunks of {chunk} (the trainer's default: "
-                                            f"{keep_bytes} kept bytes <= tokens x 2048 x 4)",
+                                            f"{keep_bytes} kept bytes, at most the larger of tokens x 2048 x 4 "
+                                            "and the weight gradient's)",
                                     "one_chunk_kept": {"ms": round(one_ms, 4), "tflops": round(one_tf, 1),
                                                        "frac": round(one_tf / peak, 4)},
                                     "whole_vocabulary_recompute": {"ms": round(whole_ms, 4),
@@ -232,7 +240,10 @@ def isolated_configs(reps: int = 20) -> dict:
                                                                    "frac": round(whole_tf / peak, 4)},
                                     "default_tile_2048": {"ms": round(tile_ms, 4), "tflops": round(tile_tf, 1),
                                                           "frac": round(tile_tf / peak, 4),
-                                                          "workspace_bytes": lce.workspace_bytes(n, d, vocab)}},
+                                                          "token_chunk": public,
+                                                          "workspace_bytes": _lib.query(
+                                                              "gptrig_flce_bwd_tokens_workspace_bytes", n, d, vocab,
+                                                              public)}},
     }
 
 
@@ -488,7 +499,7 @@ def main():
 
     n_micro = cfg.batch_size // cfg.micro_batch_size
     mb_tokens = cfg.micro_batch_size * cfg.seq_len
-    chunk = flce_token_chunk(mb_tokens, cfg.vocab_size, cfg.vocab_tile_size, cfg.flce_whole_vocab)
+    chunk = flce_token_chunk(mb_tokens, cfg.vocab_size, cfg.vocab_tile_size, cfg.flce_whole_vocab, cfg.d_model)
     traffic = FLCE_TRAFFIC_BYTES.get((mb_tokens, chunk))  # measured per shape; None for an unmeasured one
     # FLCE: every timed launch sequence of the step, per micro-batch (fwd + bwd of all its token chunks).
     flce_ms_launch, flce_n = avg_ms("flce")
