@@ -20,7 +20,10 @@ BF16 = torch.bfloat16
 F32 = torch.float32
 
 
-def _route(flat: torch.Tensor, router_w: torch.Tensor, experts: int, top_k: int):
+def _route(flat: torch.Tensor, router_w: torch.Tensor, experts: int, top_k: int, ws: torch.Tensor | None = None):
+    """Router logits and bucket routing of the bf16 rows ``flat`` alone (the
+    trainer's routed block); ``ws``: a workspace to reuse."""
+
     tokens, width = flat.shape
     dev = flat.device
     s = _lib.stream()
@@ -34,7 +37,8 @@ def _route(flat: torch.Tensor, router_w: torch.Tensor, experts: int, top_k: int)
     order = torch.empty(tokens * top_k, dtype=torch.int32, device=dev)
     rows = torch.empty(tokens * top_k, dtype=torch.int32, device=dev)
     position = torch.empty(tokens * top_k, dtype=torch.int32, device=dev)
-    ws = _lib.workspace(_lib.query("gptrig_moe_route_workspace_bytes", tokens, experts, top_k), dev)
+    if ws is None:
+        ws = _lib.workspace(_lib.query("gptrig_moe_route_workspace_bytes", tokens, experts, top_k), dev)
     _lib.call("gptrig_moe_route", logits.data_ptr(), probs.data_ptr(), chosen.data_ptr(), gate.data_ptr(),
               counts.data_ptr(), order.data_ptr(), rows.data_ptr(), position.data_ptr(), ws.data_ptr(), ws.numel(),
               tokens, experts, top_k, s)

@@ -35,6 +35,7 @@ import torch
 from . import _lib
 from .attention import attention_softmax_scale, document_segments
 from .kernels import linear_cross_entropy as lce
+from .moe import _route
 from .nn import add_rmsnorm_forward, normal, rmsnorm_backward, rmsnorm_forward, rope_tables
 from .optim import OptimizerConfig, effective_adam_betas, learning_rate, tensor_hparams
 
@@ -384,20 +385,8 @@ class GPTTrainer:
         E, k, eh = c.experts, c.expert_top_k, c.expert_mult * c.d_model
         R = N * k
         dev, s = self.device, _lib.stream()
-        logits = torch.empty((N, E), dtype=F32, device=dev)
-        _lib.call("gptrig_moe_router_logits", xn2.data_ptr(), A.param(p + "router_w").data_ptr(), logits.data_ptr(),
-                  N, d, E, s)
-        probs = torch.empty((N, E), dtype=F32, device=dev)
-        chosen = torch.empty((N, k), dtype=torch.int32, device=dev)
-        gate = torch.empty((N, k), dtype=F32, device=dev)
-        counts = torch.empty(E, dtype=torch.int32, device=dev)
-        order = torch.empty(R, dtype=torch.int32, device=dev)
-        rows = torch.empty(R, dtype=torch.int32, device=dev)
-        position = torch.empty(R, dtype=torch.int32, device=dev)
         ws = self._workspace("moe_route", _lib.query("gptrig_moe_route_workspace_bytes", N, E, k))
-        _lib.call("gptrig_moe_route", logits.data_ptr(), probs.data_ptr(), chosen.data_ptr(), gate.data_ptr(),
-                  counts.data_ptr(), order.data_ptr(), rows.data_ptr(), position.data_ptr(), ws.data_ptr(), ws.numel(),
-                  N, E, k, s)
+        logits, probs, chosen, gate, counts, rows, position = _route(xn2, A.param(p + "router_w"), E, k, ws)
         grouped = torch.empty((R, d), dtype=BF16, device=dev)
         _lib.call("gptrig_moe_gather_rows", xn2.data_ptr(), rows.data_ptr(), grouped.data_ptr(), R, d, s)
         pre = torch.empty((R, eh), dtype=BF16, device=dev)
