@@ -680,14 +680,13 @@ __global__ void stats_finalize_kernel(const int32_t* __restrict__ counts, int T,
 // chunk's dw partial f32 [8][EP] grows in registers.  After the last tile the
 // 32 token lanes' partials are summed with xor exchanges and through LDS, and
 // the workgroup adds one value per (column, expert) to dw with an atomic.  The
-// grid is about one workgroup per CU: every workgroup of a column tile adds to
-// the same few cache lines, and those adds run one after the other (128
-// workgroups per column tile: 99 us, 21: 67 us at 32768 tokens x 768; about 0.7
-// us per workgroup of a column tile).
+// grid is one or two workgroups per CU: every workgroup of a column tile adds to
+// the same few cache lines, and those adds run one after the other (32768 tokens
+// x 768, inputs past the caches: 84 workgroups per column tile 84 us, 42 72, 21 81).
 // kGather >= 0: the row the router's part is added to is not read from dx but
 // is the VJP of grouped = flat[rows], the bf16 sum of the token's rows of
 // dgrouped in bucket order (moe_gather_bwd_kernel's), so dx is written once and
-// never read: at 32768 tokens x 768, top 2, 67 us against 36 + 81 us for the
+// never read: at 32768 tokens x 768, top 2, 72 us against 36 + 62 us for the
 // two passes.  kGather is top_k where it is 1 or 2 (0: any), so the loops over
 // a token's slots unroll and their loads go out together; four tokens' loads
 // are in flight per thread.
@@ -884,7 +883,13 @@ int router_bwd(const void* x, const float* router_w, const float* probs, const i
   if (tokens <= 0 || width <= 0 || experts <= 0 || top_k <= 0 || top_k > experts) return GPTRIG_E_SHAPE;
   if (experts > kMaxRouterExperts || (size_t)width * experts * sizeof(float) > 32768) return GPTRIG_E_UNSUPPORTED;
   const int ncol = ceil_div(width, kRouterBwdCols);
-  const int runs = gemm::device_cus() / ncol > 1 ? gemm::device_cus() / ncol : 1;
+  int runs = gemm::device_cus() / ncol > 1 ? gemm::device_cus() / ncol : 1;
+  // Two workgroups fit a CU up to 8 experts; where each still has a whole tile of
+  // tokens they are worth the second round of adds (gathered / two-pass form, one and
+  // two per CU, 32768 tokens, inputs past the caches: 2048 columns 148 -> 138 / 124 ->
+  // 106 us, 1024 99 -> 88 / 86 -> 73, 768 81 -> 72 / 74 -> 62, 512 58 -> 57 / 51 -> 50;
+  // 8192 x 1024 35 -> 35; but 4096 x 512 18 -> 21, and 16 experts of 512 90 -> 111).
+  if (experts <= 8 && tokens / (2 * runs) >= kRouterBwdTokens) runs *= 2;
   // Tokens per workgroup: an even share, in whole sweeps of the 32 token lanes.
   const int run = ceil_div(ceil_div(tokens, runs), 32) * 32;
   const unsigned grid = (unsigned)ncol * (unsigned)ceil_div(tokens, run);

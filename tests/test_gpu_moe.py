@@ -246,6 +246,7 @@ def test_router_logits_of_infinite_operands(tokens, width, experts):
 
 @pytest.mark.parametrize("tokens,width,experts,top_k", [
     (1, 8, 2, 1), (255, 64, 4, 2), (257, 72, 8, 2), (300, 136, 16, 3), (130, 264, 5, 1),
+    (2048, 4096, 2, 2), (2047, 4096, 2, 1),  # two workgroups per CU (of 256) or just not: runs of one and two tiles
 ])
 def test_fused_input_backward_equals_two_passes(tokens, width, experts, top_k):
     """gptrig_moe_input_bwd against gptrig_moe_gather_bwd then
