@@ -582,14 +582,14 @@ __global__ void __launch_bounds__(gemm::THREADS) wgrad_kernel(WgradGroup g) {
 // of a slice's stages (rounded up to the main loop's groups of four) plus its
 // epilogue, in stages: about 60 for the atomic add of a tile, 20 for a read-
 // add-write (measured in the FLCE gradient launches), which one slice per tile
-// takes unless the caller asks for atomics.
-int wgrad_split(unsigned tiles, int k_iters, bool atomic) {
+// takes.
+int wgrad_split(unsigned tiles, int k_iters) {
   const int cus = gemm::device_cus();
   const int most = k_iters / 8 > 1 ? k_iters / 8 : 1;
   int best = 1;
   double best_cost = 1e300;
   for (int s = 1; s <= most && s <= 256; ++s) {
-    const double stages = (double)((ceil_div(k_iters, s) + 3) & ~3) + (s > 1 || atomic ? 60.0 : 20.0);
+    const double stages = (double)((ceil_div(k_iters, s) + 3) & ~3) + (s > 1 ? 60.0 : 20.0);
     const double cost = (double)ceil_div((int64_t)tiles * s, (int64_t)cus) * stages;
     if (cost < best_cost * 0.999) {
       best_cost = cost;
@@ -1455,7 +1455,7 @@ int gptrig_flce_bwd_tokens(const void* hidden, const void* weight, const int32_t
 
 // The weight and bias gradients of several linears over the same n tokens
 // (rig/nn.py:55-56) in grouped split-K launches; see wgrad_kernel.
-static int weight_grads(const gptrig_wgrad* items, int count, int n, bool atomic, void* stream) {
+int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* stream) {
   if (!items) return GPTRIG_E_NULL;
   if (count < 0 || n <= 0) return GPTRIG_E_SHAPE;
   for (int i = 0; i < count; ++i) {
@@ -1470,8 +1470,8 @@ static int weight_grads(const gptrig_wgrad* items, int count, int n, bool atomic
     g.n = n;
     unsigned tiles = 0;
     for (int i = 0; i < g.count; ++i) tiles += tiles_of(items[at + i].rows_in, items[at + i].cols_out);
-    g.split = wgrad_split(tiles, ceil_div(n, gemm::BK), atomic);
-    g.mode = atomic || g.split > 1 ? 2 : 1;
+    g.split = wgrad_split(tiles, ceil_div(n, gemm::BK));
+    g.mode = g.split > 1 ? 2 : 1;
     unsigned first = 0;
     for (int i = 0; i < g.count; ++i) {
       const gptrig_wgrad& w = items[at + i];
@@ -1484,14 +1484,20 @@ static int weight_grads(const gptrig_wgrad* items, int count, int n, bool atomic
   return GPTRIG_OK;
 }
 
-int gptrig_weight_grads(const gptrig_wgrad* items, int count, int n, void* stream) {
-  return weight_grads(items, count, n, false, stream);
-}
-
+// One linear's, added with fp32 atomics whatever the split.
 int gptrig_weight_grad(const void* x, const void* dy, float* dw, float* db, int n, int rows_in, int cols_out,
                        void* stream) {
-  const gptrig_wgrad item{x, dy, dw, db, rows_in, cols_out};
-  return weight_grads(&item, 1, n, true, stream);
+  if (!x || !dy || !dw) return GPTRIG_E_NULL;
+  if (n <= 0 || rows_in <= 0 || cols_out <= 0 || rows_in % 8 || cols_out % 8) return GPTRIG_E_SHAPE;
+  if (((uintptr_t)x | (uintptr_t)dy) & 15) return GPTRIG_E_SHAPE;
+  const unsigned tiles = tiles_of(rows_in, cols_out);
+  const int split = gemm::choose_split(tiles, ceil_div(n, gemm::BK));
+  // A(m = i, k = t) = X[t][i] (MN-major), B(k = t, n = j) = dY[t][j] (MN-major).
+  Operand A{(const bf16*)x, rows_in}, B{(const bf16*)dy, cols_out};
+  gemm_f32_kernel<false, false><<<tiles * split, gemm::THREADS, 0, (hipStream_t)stream>>>(A, B, rows_in, cols_out, n,
+                                                                                         split, dw, cols_out, 2, db);
+  GPTRIG_CHECK_LAUNCH();
+  return GPTRIG_OK;
 }
 
 }  // extern "C"
